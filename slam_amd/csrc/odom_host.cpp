@@ -315,15 +315,11 @@ int enqueue_populate(odom_ctx* c, const odom_frame_view* rgb, float** dstDepth, 
     py.h0 = c->h[0];
     if (dstDepth) {
         PyrSrc& q = py.p[py.count++];
-        q.kind = 0;
-        q.gen = 1;
         q.vz = c->vz;
         q.cutoff = 6.0f;
         for (int l = 0; l < kLevels; ++l) q.dst[l] = dstDepth[l];
     }
     PyrSrc& q = py.p[py.count++];
-    q.kind = 1;
-    q.gen = 2;
     q.rgb = (const uint8_t*)p;
     q.pitch = pitch;
     q.ch = fmt == ODOM_FMT_RGB8 ? 3 : 4;

@@ -55,19 +55,16 @@ struct ModelLevels {
     const float* pose_dev;          // if set: [R|t] (3x4 row-major) read on the device
 };
 void launch_model_maps(const ModelLevels& a, hipStream_t s);
-// Levels 0 (when generated), 1 and 2 of up to two pyramids in one launch.
-// kind: 0 = float Gaussian (a9), 1 = uint8 Gaussian (a11), 2 = uint16
-// bilateral-gated (a2).  gen: 0 = level 0 given (src0); 1 = level-0 depth
-// from the vertex z plane vz (verticesToDepth, cutoff); 2 = level-0
-// intensity from colour (rgb, pitch, ch).  dst[0] is written when gen != 0.
+// The three levels of up to two pyramids in one launch: a depth pyramid (a8,
+// a9) from the vertex z plane `vz` (verticesToDepth, cutoff; float levels), or
+// with vz null an intensity pyramid (a10, a11) from colour (rgb, pitch, ch;
+// uint8 levels).
 struct PyrSrc {
-    int kind, gen;
-    const void* src0;
     const float* vz;
     float cutoff;
     const uint8_t* rgb;
     int pitch, ch;
-    void* dst[3];
+    void* dst[kLevels];
 };
 struct PyrJob {
     PyrSrc p[2];

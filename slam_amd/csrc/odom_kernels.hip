@@ -263,11 +263,12 @@ struct Cam6 {
 // The texels are loaded whole and the NaN rules applied by selects, so every
 // load of an output is issued before the first wait (with branches the
 // compiler splits the loads and waits for each texel's z first).
-__device__ __forceinline__ Cam6 model_l0(const ModelLevels& a, int x, int y)
+__device__ __forceinline__ Cam6 model_l0(const ModelLevels& a, int x, int y, float& z)
 {
     const float4 vv = gp(a.v4)[(size_t)y * a.v_pitch + x];
     const float4 nn = gp(a.n4)[(size_t)y * a.n_pitch + x];
     const bool ok = !(vv.z == 0);
+    z = vv.z;
     Cam6 c;
     c.v[0] = ok ? vv.x : QNAN;
     c.v[1] = ok ? vv.y : QNAN;
@@ -291,22 +292,22 @@ __device__ __forceinline__ void mean4(const float* a, const float* b, const floa
     for (int k = 0; k < 3; ++k) o[k] = bad ? QNAN : m[k];
 }
 
-// 2x2 mean of four texels (x, y), (x+1, y), (x, y+1), (x+1, y+1).
-__device__ __forceinline__ Cam6 mean_cam(const Cam6& c00, const Cam6& c01, const Cam6& c10, const Cam6& c11)
+// 2x2 mean of the texels at i, i + 1, i + ld, i + ld + 1 of planar LDS values.
+template <int N>
+__device__ __forceinline__ Cam6 mean_lds(const float (&p)[6][N], int i, int ld)
 {
-    Cam6 o;
-    mean4(c00.v, c01.v, c10.v, c11.v, false, o.v);
-    mean4(c00.n, c01.n, c10.n, c11.n, true, o.n);
+    Cam6 q[4], o;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            q[k].v[m] = p[m][i + (k & 1) + (k >> 1) * ld];
+            q[k].n[m] = p[3 + m][i + (k & 1) + (k >> 1) * ld];
+        }
+    mean4(q[0].v, q[1].v, q[2].v, q[3].v, false, o.v);
+    mean4(q[0].n, q[1].n, q[2].n, q[3].n, true, o.n);
     return o;
 }
-
-__device__ __forceinline__ Cam6 model_l1(const ModelLevels& a, int x, int y)
-{
-    const Cam6 c00 = model_l0(a, 2 * x, 2 * y), c01 = model_l0(a, 2 * x + 1, 2 * y);
-    const Cam6 c10 = model_l0(a, 2 * x, 2 * y + 1), c11 = model_l0(a, 2 * x + 1, 2 * y + 1);
-    return mean_cam(c00, c01, c10, c11);
-}
-
 
 // Transform (when set) and store output i of level l.
 __device__ __forceinline__ void model_store(const ModelLevels& a, int l, size_t i, Cam6 c, const float* R,
@@ -333,12 +334,18 @@ __device__ __forceinline__ void model_store(const ModelLevels& a, int l, size_t 
     nm[i] = c.n[0]; nm[i + P] = c.n[1]; nm[i + 2 * P] = c.n[2];
 }
 
-// Blocks [0, nb1): a 16x16 tile of level 1 each, whose untransformed values
-// also give, from LDS, the 8x8 level-2 outputs the tile covers (2x2 means of
-// level-1 values, as level 1 is of level 0); then 256 level-0 pixels per block.
-__global__ __launch_bounds__(256) void k_model_maps(ModelLevels a, int nb1, int tiles_x1)
+// A workgroup computes all levels of a 64x16 tile of level 0, one texel per
+// thread: the untransformed values go through LDS to the 32x8 level-1 and
+// 16x4 level-2 outputs (2x2 means, each level of the one below), so each
+// texel is read once: bound by its bytes at 1920x1080 (140 MB, 27 us; 37 us
+// when level-1 workgroups read the texels again), by latency at 640x480
+// (8.3 us either way).
+constexpr int kMMX = 64, kMMY = 16;
+
+__global__ __launch_bounds__(kMMX * kMMY) void k_model_maps(ModelLevels a, int tiles_x)
 {
-    __shared__ float s1[6][16][16];
+    __shared__ float s0[6][kMMX * kMMY];
+    __shared__ float s1[6][kMMX * kMMY / 4];
     float R[9], t[3];
     if (a.transform) {
         if (a.pose_dev) {
@@ -352,49 +359,50 @@ __global__ __launch_bounds__(256) void k_model_maps(ModelLevels a, int nb1, int 
             for (int k = 0; k < 3; ++k) t[k] = a.t[k];
         }
     }
-    if ((int)blockIdx.x < nb1) {
-        const int tx = blockIdx.x % tiles_x1, ty = blockIdx.x / tiles_x1;
-        const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-        const int x = 16 * tx + lx, y = 16 * ty + ly;
-        if (x < a.w[1] && y < a.h[1]) {
-            const Cam6 c = model_l1(a, x, y);
+    const int tx = (int)blockIdx.x % tiles_x, ty = (int)blockIdx.x / tiles_x;
+    const int tid = threadIdx.x;
+    {
+        const int x = kMMX * tx + tid % kMMX, y = kMMY * ty + tid / kMMX;
+        if (x < a.w[0] && y < a.h[0]) {
+            float z;
+            const Cam6 c = model_l0(a, x, y, z);
+            const size_t i = (size_t)y * a.w[0] + x;
+            if (a.vz) gp(a.vz)[i] = z;
+#pragma unroll
             for (int m = 0; m < 3; ++m) {
-                s1[m][ly][lx] = c.v[m];
-                s1[3 + m][ly][lx] = c.n[m];
+                s0[m][tid] = c.v[m];
+                s0[3 + m][tid] = c.n[m];
+            }
+            model_store(a, 0, i, c, R, t);
+        }
+    }
+    __syncthreads();
+    if (tid < kMMX * kMMY / 4) {
+        const int lx = tid % (kMMX / 2), ly = tid / (kMMX / 2);
+        const int x = kMMX / 2 * tx + lx, y = kMMY / 2 * ty + ly;
+        if (x < a.w[1] && y < a.h[1]) {
+            const Cam6 c = mean_lds<kMMX * kMMY>(s0, 2 * ly * kMMX + 2 * lx, kMMX);
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                s1[m][tid] = c.v[m];
+                s1[3 + m][tid] = c.n[m];
             }
             model_store(a, 1, (size_t)y * a.w[1] + x, c, R, t);
         }
-        __syncthreads();
-        if (threadIdx.x < 64) {
-            const int qx = threadIdx.x & 7, qy = threadIdx.x >> 3;
-            const int X = 8 * tx + qx, Y = 8 * ty + qy;
-            if (X < a.w[2] && Y < a.h[2]) {
-                Cam6 q[4];   // (2X, 2Y), (2X+1, 2Y), (2X, 2Y+1), (2X+1, 2Y+1) of level 1
-                for (int k = 0; k < 4; ++k) {
-                    const int sx = 2 * qx + (k & 1), sy = 2 * qy + (k >> 1);
-                    for (int m = 0; m < 3; ++m) {
-                        q[k].v[m] = s1[m][sy][sx];
-                        q[k].n[m] = s1[3 + m][sy][sx];
-                    }
-                }
-                model_store(a, 2, (size_t)Y * a.w[2] + X, mean_cam(q[0], q[1], q[2], q[3]), R, t);
-            }
-        }
-        return;
     }
-    const int i = (blockIdx.x - nb1) * 256 + threadIdx.x;
-    const int w = a.w[0];
-    if (i >= w * a.h[0]) return;
-    const int y = i / w, x = i - y * w;
-    if (a.vz) gp(a.vz)[i] = gp(a.v4)[(size_t)y * a.v_pitch + x].z;
-    model_store(a, 0, (size_t)i, model_l0(a, x, y), R, t);
+    __syncthreads();
+    if (tid < kMMX * kMMY / 16) {
+        const int lx = tid % (kMMX / 4), ly = tid / (kMMX / 4);
+        const int x = kMMX / 4 * tx + lx, y = kMMY / 4 * ty + ly;
+        if (x < a.w[2] && y < a.h[2])
+            model_store(a, 2, (size_t)y * a.w[2] + x, mean_lds<kMMX * kMMY / 4>(s1, ly * kMMX + 2 * lx, kMMX / 2), R, t);
+    }
 }
 
 void launch_model_maps(const ModelLevels& a, hipStream_t s)
 {
-    const int tiles_x1 = cdiv(a.w[1], 16), nb1 = tiles_x1 * cdiv(a.h[1], 16);
-    const int nb0 = cdiv(a.w[0] * a.h[0], 256);
-    hipLaunchKernelGGL(k_model_maps, dim3(nb1 + nb0), dim3(256), 0, s, a, nb1, tiles_x1);
+    const int tiles_x = cdiv(a.w[0], kMMX);
+    hipLaunchKernelGGL(k_model_maps, dim3(tiles_x * cdiv(a.h[0], kMMY)), dim3(kMMX * kMMY), 0, s, a, tiles_x);
 }
 
 // ============================================== a9 + a11 Gaussian pyrDown
@@ -408,360 +416,302 @@ __device__ __forceinline__ int gauss5i(int k)
 }
 
 // ===================================================== pyramid launches
-// One pyramid level of up to two pyramids per launch.  Each output reads its
-// 5x5 window as 25 independent loads (coordinates clamped into the image, so
-// every address is valid) that are all in flight together; taps outside the
-// window of the reference's loops are then skipped in the accumulation, which
-// visits the rest in the loops' row-major order, so every sum is the value
-// the loops produce.
-template <class T, class Get>
-__device__ __forceinline__ void window5(Get get, int sw, int sh, int x, int y, T (&v)[25])
+// A workgroup computes all levels of one tile of one pyramid in LDS: it
+// stages the level-0 texels that its level-2 outputs depend on, then forms
+// the level-1 values they read (a margin beyond the tile's own, which the
+// neighbouring workgroups compute too), then its level-2 outputs, and stores
+// its own part of each level.  The taps and the summation order are those of
+// the reference's loops, so every value has the bits that they produce.
+//
+// The launches are bound by latency, not by bytes: a workgroup waits for one
+// round of loads, then runs two short dependent sums.  Tiles of 16x8 level-2
+// outputs give 150 workgroups per 640x480 pyramid (two pyramids a launch
+// fill the 256 CUs once) at 1.46 staged texels per texel; with separate
+// level-0, level-1 and 8x4 level-2 workgroups the same launch had 4 200
+// workgroups and staged 2.3 texels per texel for level 2 and 1.3 for level 1.
+// Two pyramids: 11.0 -> 7.4 us at 640x480, 54 -> 19 us at 1920x1080 (the
+// bytes alone: 5 us); the depth pyramid with its maps 10.0 -> 8.9 and 40 -> 24.
+constexpr int kTile2X = 16, kTile2Y = 8;       // level-2 outputs of a tile
+// Thread counts: with half as many workgroups a launch (the depth maps: one
+// pyramid) more waves per tile hide more (640x480: 8.9 us at 1024 threads,
+// 10.2 at 512); with two pyramids the counts are level at 640x480 (7.2, 7.4)
+// and 512 is ahead at 1920x1080 (19.2, 21.0).
+constexpr int kPyrThreads = 512, kMapsThreads = 1024;
+
+// The weights of the 5-tap window of output x along one axis of length n
+// (utils.cu:332-363): taps [2x-2, min(2x+3, n-1)) inside the axis, with the
+// index counted down from the last, so the weights shift at the far edge;
+// 0 for a tap outside.
+__device__ __forceinline__ void gauss_weights(int x, int n, int (&g)[5])
 {
+    const int t = min(2 * x + 3, n - 1);
 #pragma unroll
-    for (int dy = 0; dy < 5; ++dy) {
-        const int cy = min(max(2 * y - 2 + dy, 0), sh - 1);
-#pragma unroll
-        for (int dx = 0; dx < 5; ++dx) v[dy * 5 + dx] = get(min(max(2 * x - 2 + dx, 0), sw - 1), cy);
+    for (int d = 0; d < 5; ++d) {
+        const int c = 2 * x - 2 + d;
+        g[d] = (c >= 0 && c < t) ? gauss5i(t - c - 1) : 0;
     }
 }
 
-template <class Get>
-__device__ __forceinline__ float gauss_f32_at(Get get, int sw, int sh, int x, int y)
+// Gaussian means over the valid texels (above 0) of the 5x5 window that
+// starts at p in an LDS tile of row length ld.  An invalid depth is staged as
+// 0: its term is +0, which leaves the sum's bits.
+__device__ __forceinline__ float gauss_f32(const float* p, int ld, const int (&gx)[5], const int (&gy)[5])
 {
-    const int tx = min(2 * x + 3, sw - 1), ty = min(2 * y + 3, sh - 1);
-    float v[25];
-    window5(get, sw, sh, x, y, v);
-    // the reference adds each float weight to an int count, truncating; the
-    // weights are integers, so an integer sum is the same count
-    float sum = 0.0f;
-    int count = 0;
+    float sum = 0.0f, count = 0.0f;   // the weights are integers, so the count is exact
 #pragma unroll
     for (int dy = 0; dy < 5; ++dy)
 #pragma unroll
         for (int dx = 0; dx < 5; ++dx) {
-            const int cy = 2 * y - 2 + dy, cx = 2 * x - 2 + dx;
-            const float val = v[dy * 5 + dx];
-            if (cy >= 0 && cy < ty && cx >= 0 && cx < tx && !isnan(val)) {
-                const int gk = gauss5i(ty - cy - 1) * gauss5i(tx - cx - 1);
-                sum = sum + val * (float)gk;
-                count += gk;
-            }
+            const float v = p[dy * ld + dx];
+            const float g = (float)(gx[dx] * gy[dy]);
+            sum = sum + v * g;
+            count += v > 0.0f ? g : 0.0f;
         }
-    return sum / (float)count;
+    return sum / count;               // 0 / 0: NaN, as the reference
 }
 
-template <class Get>
-__device__ __forceinline__ uint8_t gauss_u8_at(Get get, int sw, int sh, int x, int y)
+// Texels are staged as value | (value > 0) << 16.  The weighted sum of the
+// values stays below 2^16 (255 * 256) and the count is at most 256, so one
+// integer holds both, and both are separable; the reference's float sum of
+// these integers is exact, so the integer sums give its bits.
+__device__ __forceinline__ uint32_t u8_texel(uint32_t v) { return v | (v > 0 ? 0x10000u : 0u); }
+
+__device__ __forceinline__ uint32_t gauss_u8(const uint32_t* p, int ld, const int (&gx)[5], const int (&gy)[5])
 {
-    const int tx = min(2 * x + 3, sw - 1), ty = min(2 * y + 3, sh - 1);
-    uint8_t v[25];
-    window5(get, sw, sh, x, y, v);
-    // every term val * gk is an integer below 2^14 and their sum stays below
-    // 2^24, so the reference's float sum is exact in any order: integer sums
-    // give the same bits
-    int sum = 0, count = 0;
+    uint32_t s = 0;
 #pragma unroll
-    for (int dy = 0; dy < 5; ++dy)
+    for (int dy = 0; dy < 5; ++dy) {
+        uint32_t r = 0;
 #pragma unroll
-        for (int dx = 0; dx < 5; ++dx) {
-            const int cy = 2 * y - 2 + dy, cx = 2 * x - 2 + dx;
-            const int val = v[dy * 5 + dx];
-            if (cy >= 0 && cy < ty && cx >= 0 && cx < tx && val > 0) {
-                const int gk = gauss5i(ty - cy - 1) * gauss5i(tx - cx - 1);
-                sum += val * gk;
-                count += gk;
-            }
-        }
-    const float q = (float)sum / (float)count;
-    return (count == 0) ? (uint8_t)0 : (uint8_t)q;
+        for (int dx = 0; dx < 5; ++dx) r += __umul24(p[dy * ld + dx], (uint32_t)gx[dx]);
+        s += r * (uint32_t)gy[dy];
+    }
+    const uint32_t count = s >> 16;
+    const float q = (float)(s & 0xFFFFu) / (float)count;
+    return count == 0 ? 0u : (uint32_t)(uint8_t)q;
 }
 
 // utils.cu:57-94 (sigma_color 30): taps at offsets -2..2 inside the image,
 // weighted {0.0625, 0.25, 0.375, 0.25, 0.0625} per axis, kept when within
-// 3 sigma of the centre value.
-template <class Get>
-__device__ __forceinline__ uint16_t pyr_u16_at(Get get, int sw, int sh, int x, int y)
+// 3 sigma of the centre value.  In 1/256 units the weights are the integers
+// {1 4 6 4 1} x {1 4 6 4 1} and the sums stay below 2^24 units, so the
+// reference's float sums are exact and equal the integer sums; scaling both
+// by 2^-8 leaves their quotient unchanged.  Texels outside the image are
+// staged as kNoTexel, far from every 16-bit value.
+constexpr int kNoTexel = 1 << 20;
+
+__device__ __forceinline__ int gauss_u16(const int* p, int ld)
 {
-    // In 1/256 units the weights are the integers {1 4 6 4 1} x {1 4 6 4 1}:
-    // each float term val * w * w is exact, and the sums stay below 2^24
-    // units, so the reference's float sums are exact in any order and equal
-    // the integer sums; scaling both by 2^-8 leaves their quotient unchanged.
-    int v[25];
-    window5(get, sw, sh, x, y, v);
-    const int center = v[12];
+    const int center = p[2 * ld + 2];
     int sum = 0, wall = 0;
 #pragma unroll
     for (int dy = 0; dy < 5; ++dy)
 #pragma unroll
         for (int dx = 0; dx < 5; ++dx) {
-            const int cy = 2 * y - 2 + dy, cx = 2 * x - 2 + dx;
-            const int val = v[dy * 5 + dx];
-            if (cy >= 0 && cy < sh && cx >= 0 && cx < sw && abs(val - center) < 90) {
-                const int wk = gauss5i(dx) * gauss5i(dy);
-                sum += val * wk;
-                wall += wk;
-            }
+            const int v = p[dy * ld + dx];
+            const int wk = abs(v - center) < 90 ? gauss5i(dx) * gauss5i(dy) : 0;
+            sum += __mul24(v, wk);
+            wall += wk;
         }
-    return (uint16_t)(int)((float)sum / (float)wall);
+    return (int)(uint16_t)(int)((float)sum / (float)wall);
 }
 
-// Levels 0 (when generated), 1 and 2 of up to two pyramids in one launch,
-// from LDS tiles.  A level-1 block stages the level-0 texels of its 16x16
-// outputs' windows (36x36); a level-2 block stages 43x27 level-0 texels,
-// computes the 20x12 level-1 values its 8x4 outputs read (the same
-// computation the level-1 blocks store; one value per thread, so the block
-// runs two dependent Gaussian sums, not three), then its outputs.  Level 0 is read
-// from memory or generated (verticesToDepth, or the intensity conversion of
-// populateRGBDData, RGBDOdometryef.cpp:212, 225), in which case level-0
-// blocks also store it.  The taps, their clamped coordinates and the
-// summation order are those of the per-level functions above.
-constexpr int kPT = 16;                 // level-1 output tile edge
-constexpr int kT1 = 2 * kPT + 4;        // its level-0 texels
-constexpr int kPT2X = 8, kPT2Y = 4;     // level-2 output tile (its level-1 values, below, fit
-                                        // one pass of the 256 threads)
-constexpr int kT21X = 2 * kPT2X + 4, kT21Y = 2 * kPT2Y + 4;   // its level-1 values
-constexpr int kT20X = 2 * kT21X + 3, kT20Y = 2 * kT21Y + 3;   // its level-0 texels
-static_assert(kT21X * kT21Y <= 256, "one level-1 value per thread");
+// A staged tile's geometry: level-2 outputs (with `margin` more beyond the
+// right and lower edges), the level-1 values and level-0 texels they need.
+template <int MARGIN, int NT>
+struct TileDims {
+    static constexpr int R2X = kTile2X + MARGIN, R2Y = kTile2Y + MARGIN;
+    static constexpr int X1 = 2 * R2X + 3, Y1 = 2 * R2Y + 3, N1 = X1 * Y1;
+    static constexpr int X0 = 2 * X1 + 3, Y0 = 2 * Y1 + 3, N0 = X0 * Y0;
+    static constexpr int R0 = (N0 + NT - 1) / NT;   // texels per thread
+};
 
 struct PyrGrid {
     PyrJob j;
-    int nseg;
-    int b0[7];
-    int seg_q[6], seg_t[6];             // pyramid, and level (0 generation, 1, 2) of a segment
-    int tiles_x[3];                     // tiles per row at levels 1, 2 (index by level)
+    int tiles_x, tiles;               // tiles per row, per pyramid
 };
 
-template <class T>
-__device__ __forceinline__ T pyr_l0(const PyrSrc& q, int w0, int x, int y)
-{
-    const size_t i = (size_t)y * w0 + x;
-    if constexpr (sizeof(T) == 4) {
-        if (q.gen == 1) {
-            const float z = gp(q.vz)[i];
-            return (z > q.cutoff || z <= 0) ? QNAN : z;
-        }
-    } else if constexpr (sizeof(T) == 1) {
-        if (q.gen == 2) {
-            const GLOBAL_AS uint8_t* px = gp(q.rgb) + (size_t)y * q.pitch + (size_t)x * q.ch;
-            return (uint8_t)(int)((float)px[0] * 0.114f + (float)px[1] * 0.299f + (float)px[2] * 0.587f);
-        }
-    }
-    return gp((const T*)q.src0)[i];
-}
+// Level 0 of the depth pyramid (a8 verticesToDepth): NaN outside (0, cutoff].
+// Level 0 of the intensity pyramid (populateRGBDData, RGBDOdometryef.cpp:212,
+// 225) from the texel's first three bytes, read as one 4-byte word; the
+// image's last texel is read one byte early, so that no byte past it is read.
+typedef uint32_t __attribute__((aligned(1))) word_at_any_byte;
 
-// Level-0 texels of a tile in LDS (texels outside the image hold their
-// clamped neighbour; the windows clamp their coordinates, so never read them).
-// The source kind is uniform, so each kind stages with its own straight-line
-// loads.
-template <int N, class T>
-__device__ __forceinline__ void pyr_stage(const PyrSrc& q, T* tile, int ld, int ox, int oy, int w0, int h0)
+template <bool DEPTH>
+__device__ void pyr_tile(const PyrSrc& P, int w0, int h0, int tx, int ty, unsigned char* smem)
 {
-    if constexpr (sizeof(T) == 4) {
-        if (q.gen == 1) {
-            stage_tile<N, 256, false>(tile, ld, ox, oy, w0, h0, [&](int x, int y) {
-                const float z = gp(q.vz)[(size_t)y * w0 + x];
-                return (T)((z > q.cutoff || z <= 0) ? QNAN : z);
-            });
-            return;
-        }
-    } else if constexpr (sizeof(T) == 1) {
-        if (q.gen == 2) {
-            stage_tile<N, 256, false>(tile, ld, ox, oy, w0, h0, [&](int x, int y) {
-                const GLOBAL_AS uint8_t* px = gp(q.rgb) + (size_t)y * q.pitch + (size_t)x * q.ch;
-                return (T)(uint8_t)(int)((float)px[0] * 0.114f + (float)px[1] * 0.299f + (float)px[2] * 0.587f);
-            });
-            return;
-        }
-    }
-    stage_tile<N, 256, false>(tile, ld, ox, oy, w0, h0,
-                              [&](int x, int y) { return gp((const T*)q.src0)[(size_t)y * w0 + x]; });
-}
-
-// One output of level `lvl` from its source level `src` (sw x sh texels)
-// held in an LDS tile with origin (ox, oy) and row length `ld`.
-template <int KIND, class T>
-__device__ __forceinline__ T pyr_at(const T* tile, int ld, int ox, int oy, int sw, int sh, int x, int y)
-{
-    auto get = [&](int cx, int cy) { return tile[(cy - oy) * ld + (cx - ox)]; };
-    if constexpr (KIND == 0) {
-        return gauss_f32_at(get, sw, sh, x, y);
-    } else if constexpr (KIND == 1) {
-        return gauss_u8_at(get, sw, sh, x, y);
-    } else {
-        auto geti = [&](int cx, int cy) { return (int)get(cx, cy); };
-        return pyr_u16_at(geti, sw, sh, x, y);
-    }
-}
-
-template <int KIND, class T>
-__device__ void pyr_block(const PyrGrid& g, int q, int t, int lb, unsigned char* smem)
-{
-    const PyrSrc& P = g.j.p[q];
-    const int w0 = g.j.w0, h0 = g.j.h0, w1 = w0 / 2, h1 = h0 / 2, w2 = w1 / 2, h2 = h1 / 2;
+    using D = TileDims<0, kPyrThreads>;
+    using T = std::conditional_t<DEPTH, float, uint32_t>;
+    T* s0 = (T*)smem;
+    T* s1 = s0 + D::N0;
+    const int w1 = w0 / 2, h1 = h0 / 2, w2 = w1 / 2, h2 = h1 / 2;
+    const int c2x = tx * kTile2X, c2y = ty * kTile2Y;             // the tile's first output of each level
+    const int c1x = 2 * c2x, c1y = 2 * c2y, c0x = 2 * c1x, c0y = 2 * c1y;
     const int tid = threadIdx.x;
-    if (t == 0) {
-        const int i = lb * 256 + tid;
-        if (i < w0 * h0) {
-            const int y = i / w0, x = i - y * w0;
-            gp((T*)P.dst[0])[i] = pyr_l0<T>(P, w0, x, y);
+    uint32_t raw[D::R0];
+#pragma unroll
+    for (int r = 0; r < D::R0; ++r) {
+        const int i = min(tid + r * kPyrThreads, D::N0 - 1);
+        const int x = min(max(c0x - 6 + i % D::X0, 0), w0 - 1), y = min(max(c0y - 6 + i / D::X0, 0), h0 - 1);
+        if constexpr (DEPTH) {
+            raw[r] = gp((const uint32_t*)P.vz)[(size_t)y * w0 + x];
+        } else {
+            const int early = (x == w0 - 1 && y == h0 - 1 && P.ch == 3) ? 1 : 0;
+            const GLOBAL_AS uint8_t* px = gp(P.rgb) + ((size_t)y * P.pitch + (size_t)x * P.ch - early);
+            raw[r] = *(const GLOBAL_AS word_at_any_byte*)px >> (8 * early);
         }
-        return;
     }
-    const int tx = lb % g.tiles_x[t], ty = lb / g.tiles_x[t];
-    T* t1 = (T*)smem;                            // texels one level below the outputs
-    if (t == 1) {
-        const int X0 = tx * kPT, Y0 = ty * kPT;
-        const int x = X0 + (tid & (kPT - 1)), y = Y0 + tid / kPT;
-        const int ox = 2 * X0 - 2, oy = 2 * Y0 - 2;
-        pyr_stage<kT1 * kT1, T>(P, t1, kT1, ox, oy, w0, h0);
-        __syncthreads();
-        if (x < w1 && y < h1) gp((T*)P.dst[1])[(size_t)y * w1 + x] = pyr_at<KIND>(t1, kT1, ox, oy, w0, h0, x, y);
-        return;
-    }
-    const int X0 = tx * kPT2X, Y0 = ty * kPT2Y;
-    T* t0 = t1 + kT21X * kT21Y;                  // level-0 texels
-    const int o1x = 2 * X0 - 2, o1y = 2 * Y0 - 2;
-    const int o0x = 2 * o1x - 2, o0y = 2 * o1y - 2;
-    pyr_stage<kT20X * kT20Y, T>(P, t0, kT20X, o0x, o0y, w0, h0);
-    __syncthreads();
-    if (tid < kT21X * kT21Y) {
-        const int x1 = o1x + tid % kT21X, y1 = o1y + tid / kT21X;
-        if (x1 >= 0 && x1 < w1 && y1 >= 0 && y1 < h1) t1[tid] = pyr_at<KIND>(t0, kT20X, o0x, o0y, w0, h0, x1, y1);
+#pragma unroll
+    for (int r = 0; r < D::R0; ++r) {
+        const int i = tid + r * kPyrThreads;
+        if (i >= D::N0) break;
+        const int x = c0x - 6 + i % D::X0, y = c0y - 6 + i / D::X0;
+        const bool own = x >= c0x && x < min(c0x + 4 * kTile2X, w0) && y >= c0y && y < min(c0y + 4 * kTile2Y, h0);
+        if constexpr (DEPTH) {
+            const float z = __uint_as_float(raw[r]);
+            const bool bad = z > P.cutoff || z <= 0 || isnan(z);
+            s0[i] = bad ? 0.0f : z;
+            if (own) gp((float*)P.dst[0])[(size_t)y * w0 + x] = (z > P.cutoff || z <= 0) ? QNAN : z;
+        } else {
+            const uint32_t v = (uint8_t)(int)((float)(raw[r] & 0xFFu) * 0.114f + (float)((raw[r] >> 8) & 0xFFu) * 0.299f +
+                                              (float)((raw[r] >> 16) & 0xFFu) * 0.587f);
+            s0[i] = u8_texel(v);
+            if (own) gp((uint8_t*)P.dst[0])[(size_t)y * w0 + x] = (uint8_t)v;
+        }
     }
     __syncthreads();
-    const int x = X0 + (tid & (kPT2X - 1)), y = Y0 + tid / kPT2X;
-    if (tid < kPT2X * kPT2Y && x < w2 && y < h2)
-        gp((T*)P.dst[2])[(size_t)y * w2 + x] = pyr_at<KIND>(t1, kT21X, o1x, o1y, w1, h1, x, y);
+    for (int e = tid; e < D::N1; e += kPyrThreads) {
+        const int ex = e % D::X1, ey = e / D::X1;
+        const int x = c1x - 2 + ex, y = c1y - 2 + ey;
+        T v = T(0);                  // outside the level: no weight, but read
+        if (x >= 0 && x < w1 && y >= 0 && y < h1) {
+            int gx[5], gy[5];
+            gauss_weights(x, w0, gx);
+            gauss_weights(y, h0, gy);
+            const bool own = x >= c1x && x < c1x + 2 * kTile2X && y >= c1y && y < c1y + 2 * kTile2Y;
+            const T* p = s0 + 2 * ey * D::X0 + 2 * ex;
+            if constexpr (DEPTH) {
+                const float z = gauss_f32(p, D::X0, gx, gy);
+                v = isnan(z) ? 0.0f : z;
+                if (own) gp((float*)P.dst[1])[(size_t)y * w1 + x] = z;
+            } else {
+                const uint32_t u = gauss_u8(p, D::X0, gx, gy);
+                v = u8_texel(u);
+                if (own) gp((uint8_t*)P.dst[1])[(size_t)y * w1 + x] = (uint8_t)u;
+            }
+        }
+        s1[e] = v;
+    }
+    __syncthreads();
+    if (tid < kTile2X * kTile2Y) {
+        const int ex = tid % kTile2X, ey = tid / kTile2X;
+        const int x = c2x + ex, y = c2y + ey;
+        if (x < w2 && y < h2) {
+            int gx[5], gy[5];
+            gauss_weights(x, w1, gx);
+            gauss_weights(y, h1, gy);
+            const T* p = s1 + 2 * ey * D::X1 + 2 * ex;
+            if constexpr (DEPTH) gp((float*)P.dst[2])[(size_t)y * w2 + x] = gauss_f32(p, D::X1, gx, gy);
+            else gp((uint8_t*)P.dst[2])[(size_t)y * w2 + x] = (uint8_t)gauss_u8(p, D::X1, gx, gy);
+        }
+    }
 }
 
-__global__ __launch_bounds__(256) void k_pyramid(PyrGrid g)
+__global__ __launch_bounds__(kPyrThreads) void k_pyramid(PyrGrid g)
 {
-    constexpr int kL2 = kT21X * kT21Y + kT20X * kT20Y;
-    __shared__ __align__(16) unsigned char smem[(kT1 * kT1 > kL2 ? kT1 * kT1 : kL2) * 4];
-    int sgi = 0;
-    while (sgi + 1 < g.nseg && (int)blockIdx.x >= g.b0[sgi + 1]) ++sgi;
-    const int q = g.seg_q[sgi], t = g.seg_t[sgi], lb = blockIdx.x - g.b0[sgi];
-    const int kind = g.j.p[q].kind;
-    if (kind == 0) pyr_block<0, float>(g, q, t, lb, smem);
-    else if (kind == 1) pyr_block<1, uint8_t>(g, q, t, lb, smem);
-    else pyr_block<2, uint16_t>(g, q, t, lb, smem);
+    __shared__ __align__(16) unsigned char smem[(TileDims<0, kPyrThreads>::N0 + TileDims<0, kPyrThreads>::N1) * 4];
+    const int q = (int)blockIdx.x / g.tiles, t = (int)blockIdx.x - q * g.tiles;
+    const int ty = t / g.tiles_x, tx = t - ty * g.tiles_x;
+    const PyrSrc& P = g.j.p[q];
+    if (P.vz) pyr_tile<true>(P, g.j.w0, g.j.h0, tx, ty, smem);
+    else pyr_tile<false>(P, g.j.w0, g.j.h0, tx, ty, smem);
 }
 
 void launch_pyramid(const PyrJob& j, hipStream_t s)
 {
     PyrGrid g{};
     g.j = j;
-    const int w1 = j.w0 / 2, h1 = j.h0 / 2, w2 = w1 / 2, h2 = h1 / 2;
-    g.tiles_x[1] = cdiv(w1, kPT);
-    g.tiles_x[2] = cdiv(w2, kPT2X);
-    const int n2 = g.tiles_x[2] * cdiv(h2, kPT2Y), n1 = g.tiles_x[1] * cdiv(h1, kPT);
-    int nb = 0;
-    // level-2 tiles first (the longest blocks), then level 1, then level-0 generation
-    for (int t = 2; t >= 0; --t)
-        for (int q = 0; q < j.count; ++q) {
-            const int n = t == 2 ? n2 : (t == 1 ? n1 : (j.p[q].gen ? cdiv(j.w0 * j.h0, 256) : 0));
-            if (!n) continue;
-            g.b0[g.nseg] = nb;
-            g.seg_q[g.nseg] = q;
-            g.seg_t[g.nseg] = t;
-            g.nseg++;
-            nb += n;
-        }
-    g.b0[g.nseg] = nb;
-    hipLaunchKernelGGL(k_pyramid, dim3(nb), dim3(256), 0, s, g);
+    // the tiles cover level 0; the coarser levels' outputs lie inside
+    g.tiles_x = cdiv(j.w0, 4 * kTile2X);
+    g.tiles = g.tiles_x * cdiv(j.h0, 4 * kTile2Y);
+    hipLaunchKernelGGL(k_pyramid, dim3(j.count * g.tiles), dim3(kPyrThreads), 0, s, g);
 }
 
 // initICP's depth pyramid (a2) and the vertex and normal maps of its three
-// levels (a3, a4) in one launch.  Level-2 tiles come first, then level-1
-// tiles, then the level-0 maps one pixel per thread from the input.  A tile
-// computes its level's depth one output beyond its right and lower edges
-// too, in LDS only (the neighbouring tile stores those), so the normals of
-// its edge pixels, which read their right and lower neighbours, come from
-// the tile itself.  The depths are those of k_pyramid (the same windows and
-// sums) and every level's maps come from vn_pixel, the same expressions
-// whichever block computes them.
-constexpr int kDM1 = 16;                                      // level-1 tile edge
-constexpr int kDM1R = kDM1 + 1;                               // with the one-output margin
-constexpr int kDM1T = 2 * kDM1R + 3;                          // its level-0 texels (37)
-constexpr int kDM2X = 8, kDM2Y = 4;                           // level-2 tile
-constexpr int kDM2RX = kDM2X + 1, kDM2RY = kDM2Y + 1;         // with the margin
-constexpr int kDM21X = 2 * kDM2RX + 3, kDM21Y = 2 * kDM2RY + 3;   // its level-1 values (21 x 13)
-constexpr int kDM20X = 2 * kDM21X + 3, kDM20Y = 2 * kDM21Y + 3;   // their level-0 texels (45 x 29)
-static_assert(kDM1R * kDM1R <= 2 * 256 && kDM21X * kDM21Y <= 2 * 256 && kDM2RX * kDM2RY <= 256, "passes");
-
+// levels (a3, a4) in one launch, a tile per workgroup as above.  The normals
+// read the right and lower neighbours, so a tile's level-2 depths have a
+// margin of one output (in LDS only; the neighbouring tile stores those), and
+// the staged level-0 texels and level-1 values hold the others' margins.
 struct DepthMapsGrid {
     VNLevels a;                   // a.depth[0] is the input; a.depth[1], a.depth[2] are written
-    int n2, n1;                   // level-2 and level-1 tiles
-    int tx2, tx1;                 // tiles per row
+    int tiles_x;
 };
 
-__global__ __launch_bounds__(256) void k_depth_pyramid_maps(DepthMapsGrid g)
+__global__ __launch_bounds__(kMapsThreads) void k_depth_pyramid_maps(DepthMapsGrid g)
 {
-    constexpr int kS0 = kDM20X * kDM20Y > kDM1T * kDM1T ? kDM20X * kDM20Y : kDM1T * kDM1T;
-    constexpr int kS1 = kDM21X * kDM21Y > kDM1R * kDM1R ? kDM21X * kDM21Y : kDM1R * kDM1R;
-    __shared__ uint16_t s0[kS0];
-    __shared__ uint16_t s1[kS1];
-    __shared__ uint16_t s2[kDM2RX * kDM2RY];
+    using D = TileDims<1, kMapsThreads>;
+    __shared__ int s0[D::N0], s1[D::N1], s2[D::R2X * D::R2Y];
     const VNLevels& a = g.a;
-    const int tid = threadIdx.x;
     const int w0 = a.w[0], h0 = a.h[0], w1 = a.w[1], h1 = a.h[1], w2 = a.w[2], h2 = a.h[2];
-    const uint16_t* d0 = a.depth[0];
-    auto load0 = [&](int x, int y) { return d0[(size_t)y * w0 + x]; };
-    int b = blockIdx.x;
-    if (b < g.n2) {
-        const int X0 = (b % g.tx2) * kDM2X, Y0 = (b / g.tx2) * kDM2Y;
-        const int o1x = 2 * X0 - 2, o1y = 2 * Y0 - 2;
-        const int o0x = 2 * o1x - 2, o0y = 2 * o1y - 2;
-        stage_tile<kDM20X * kDM20Y, 256, false>(s0, kDM20X, o0x, o0y, w0, h0, load0);
-        __syncthreads();
-        for (int e = tid; e < kDM21X * kDM21Y; e += 256) {
-            const int x1 = o1x + e % kDM21X, y1 = o1y + e / kDM21X;
-            if (x1 >= 0 && x1 < w1 && y1 >= 0 && y1 < h1)
-                s1[e] = pyr_at<2>((const uint16_t*)s0, kDM20X, o0x, o0y, w0, h0, x1, y1);
-        }
-        __syncthreads();
-        if (tid < kDM2RX * kDM2RY) {
-            const int cx = tid % kDM2RX, cy = tid / kDM2RX;
-            const int x = X0 + cx, y = Y0 + cy;
-            if (x < w2 && y < h2) {
-                const uint16_t v = pyr_at<2>((const uint16_t*)s1, kDM21X, o1x, o1y, w1, h1, x, y);
-                s2[tid] = v;
-                if (cx < kDM2X && cy < kDM2Y) a.depth[2][(size_t)y * w2 + x] = v;
-            }
-        }
-        __syncthreads();
-        if (tid < kDM2X * kDM2Y) {
-            const int x = X0 + tid % kDM2X, y = Y0 + tid / kDM2X;
-            if (x < w2 && y < h2)
-                vn_pixel(a, 2, x, y, [&](int u, int v) { return s2[(v - Y0) * kDM2RX + (u - X0)]; });
-        }
-        return;
+    const int ty = (int)blockIdx.x / g.tiles_x, tx = (int)blockIdx.x - ty * g.tiles_x;
+    const int c2x = tx * kTile2X, c2y = ty * kTile2Y;
+    const int c1x = 2 * c2x, c1y = 2 * c2y, c0x = 2 * c1x, c0y = 2 * c1y;
+    const int tid = threadIdx.x;
+    uint16_t raw[D::R0];
+#pragma unroll
+    for (int r = 0; r < D::R0; ++r) {
+        const int i = min(tid + r * kMapsThreads, D::N0 - 1);
+        const int x = min(max(c0x - 6 + i % D::X0, 0), w0 - 1), y = min(max(c0y - 6 + i / D::X0, 0), h0 - 1);
+        raw[r] = gp((const uint16_t*)a.depth[0])[(size_t)y * w0 + x];
     }
-    b -= g.n2;
-    if (b < g.n1) {
-        const int X0 = (b % g.tx1) * kDM1, Y0 = (b / g.tx1) * kDM1;
-        const int ox = 2 * X0 - 2, oy = 2 * Y0 - 2;
-        stage_tile<kDM1T * kDM1T, 256, false>(s0, kDM1T, ox, oy, w0, h0, load0);
-        __syncthreads();
-        for (int e = tid; e < kDM1R * kDM1R; e += 256) {
-            const int cx = e % kDM1R, cy = e / kDM1R;
-            const int x = X0 + cx, y = Y0 + cy;
-            if (x < w1 && y < h1) {
-                const uint16_t v = pyr_at<2>((const uint16_t*)s0, kDM1T, ox, oy, w0, h0, x, y);
-                s1[e] = v;
-                if (cx < kDM1 && cy < kDM1) a.depth[1][(size_t)y * w1 + x] = v;
-            }
-        }
-        __syncthreads();
-        const int x = X0 + (tid & (kDM1 - 1)), y = Y0 + tid / kDM1;
-        if (x < w1 && y < h1) vn_pixel(a, 1, x, y, [&](int u, int v) { return s1[(v - Y0) * kDM1R + (u - X0)]; });
-        return;
+#pragma unroll
+    for (int r = 0; r < D::R0; ++r) {
+        const int i = tid + r * kMapsThreads;
+        if (i >= D::N0) break;
+        const int x = c0x - 6 + i % D::X0, y = c0y - 6 + i / D::X0;
+        s0[i] = (x >= 0 && x < w0 && y >= 0 && y < h0) ? (int)raw[r] : kNoTexel;
     }
-    b -= g.n1;
-    const int i = b * 256 + tid;
-    if (i < w0 * h0) {
-        const int y = i / w0, x = i - y * w0;
-        vn_pixel(a, 0, x, y, load0);
+    __syncthreads();
+    for (int e = tid; e < D::N1; e += kMapsThreads) {
+        const int ex = e % D::X1, ey = e / D::X1;
+        const int x = c1x - 2 + ex, y = c1y - 2 + ey;
+        int v = kNoTexel;
+        if (x >= 0 && x < w1 && y >= 0 && y < h1) {
+            v = gauss_u16(s0 + 2 * ey * D::X0 + 2 * ex, D::X0);
+            if (x >= c1x && x < c1x + 2 * kTile2X && y >= c1y && y < c1y + 2 * kTile2Y)
+                gp(a.depth[1])[(size_t)y * w1 + x] = (uint16_t)v;
+        }
+        s1[e] = v;
+    }
+    // level 0's maps while level 1 settles: four pixels a thread
+#pragma unroll
+    for (int r = 0; r < 16 * kTile2X * kTile2Y / kMapsThreads; ++r) {
+        const int i = tid + r * kMapsThreads;
+        const int x = c0x + i % (4 * kTile2X), y = c0y + i / (4 * kTile2X);
+        if (x < w0 && y < h0)
+            vn_pixel(a, 0, x, y, [&](int u, int v) { return (uint16_t)s0[(v - c0y + 6) * D::X0 + (u - c0x + 6)]; });
+    }
+    __syncthreads();
+    if (tid < D::R2X * D::R2Y) {
+        const int ex = tid % D::R2X, ey = tid / D::R2X;
+        const int x = c2x + ex, y = c2y + ey;
+        if (x < w2 && y < h2) {
+            const int v = gauss_u16(s1 + 2 * ey * D::X1 + 2 * ex, D::X1);
+            s2[tid] = v;
+            if (ex < kTile2X && ey < kTile2Y) gp(a.depth[2])[(size_t)y * w2 + x] = (uint16_t)v;
+        }
+    }
+    static_assert(4 * kTile2X * kTile2Y <= kMapsThreads && D::R2X * D::R2Y <= kMapsThreads, "a pixel a thread");
+    if (tid < 4 * kTile2X * kTile2Y) {
+        const int x = c1x + tid % (2 * kTile2X), y = c1y + tid / (2 * kTile2X);
+        if (x < w1 && y < h1)
+            vn_pixel(a, 1, x, y, [&](int u, int v) { return (uint16_t)s1[(v - c1y + 2) * D::X1 + (u - c1x + 2)]; });
+    }
+    __syncthreads();
+    if (tid < kTile2X * kTile2Y) {
+        const int x = c2x + tid % kTile2X, y = c2y + tid / kTile2X;
+        if (x < w2 && y < h2)
+            vn_pixel(a, 2, x, y, [&](int u, int v) { return (uint16_t)s2[(v - c2y) * D::R2X + (u - c2x)]; });
     }
 }
 
@@ -769,12 +719,8 @@ void launch_depth_pyramid_maps(const VNLevels& a, hipStream_t s)
 {
     DepthMapsGrid g;
     g.a = a;
-    g.tx2 = cdiv(a.w[2], kDM2X);
-    g.tx1 = cdiv(a.w[1], kDM1);
-    g.n2 = g.tx2 * cdiv(a.h[2], kDM2Y);
-    g.n1 = g.tx1 * cdiv(a.h[1], kDM1);
-    const int n0 = cdiv(a.w[0] * a.h[0], 256);
-    hipLaunchKernelGGL(k_depth_pyramid_maps, dim3(g.n2 + g.n1 + n0), dim3(256), 0, s, g);
+    g.tiles_x = cdiv(a.w[0], 4 * kTile2X);
+    hipLaunchKernelGGL(k_depth_pyramid_maps, dim3(g.tiles_x * cdiv(a.h[0], 4 * kTile2Y)), dim3(kMapsThreads), 0, s, g);
 }
 
 // ================================ a12 derivatives + photometric source mask
