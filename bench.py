@@ -380,9 +380,9 @@ def c1_gpu(args) -> dict:
 
 def network_timing(reps: int = 50) -> dict:
     """Microseconds per call of the warm-start network: the fused one-launch
-    inference (cnn_infer) and the training forward (cnn_forward, one GEMM
-    launch per layer plus im2col / split-K passes), at batch 1 and 8, timed
-    with HIP events over `reps` back-to-back calls."""
+    inference (cnn_infer) and the training forward (cnn_forward, one launch
+    per layer), at batch 1 and 8, timed with HIP events over `reps`
+    back-to-back calls."""
     import torch
     from slam_amd import warmstart as ws
     net = ws.WarmStartNet(max_batch=8)

@@ -9,11 +9,12 @@
 // unrelated YOLACT segmenter); the tracker uses the prediction as the initial
 // increment of a Gauss-Newton solve.
 //
-// Every convolution and linear layer runs as one GEMM on MFMA
-// (v_mfma_f32_16x16x16_bf16: bf16 operands, fp32 accumulation): forward
-// Y = im2col(X) W, weight gradient dW = im2col(X)^T dY (split over the
-// reduction and summed in a fixed order), input gradient dX = col2im(dY W^T).
-// Master weights and Adam moments are fp32; the GEMMs read bf16 copies.
+// Every convolution and linear layer is a matrix product on MFMA (bf16
+// operands, fp32 accumulation) that gathers its im2col operand as it runs:
+// forward Y = im2col(X) W, weight gradient dW = im2col(X)^T dY (split over
+// the reduction and summed in a fixed order), input gradient dX =
+// col2im(dY W^T).  Master weights and Adam moments are fp32; the products
+// read bf16 copies.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -21,6 +22,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "slam_cnn.h"
@@ -43,263 +45,593 @@ __host__ __device__ inline float bf2f(bf16 h) { return __builtin_bit_cast(float,
 
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
-// ============================================================= GEMM
-// Eight consecutive bf16 from p[i..i+7] when `row_ok`, of which the first
-// `avail` exist (zero-filled beyond); one 16-byte load when all eight do.
-// Every operand's leading dimension and base offset are multiples of 8
-// elements, so full segments are 16-byte aligned.
-__device__ __forceinline__ void load8(const bf16* __restrict__ p, size_t i, bool row_ok, int avail, bf16 (&v)[8])
+// ============================================================= training
+// Layers as matrix products on MFMA (bf16 operands, fp32 sums), without
+// im2col or col2im in memory: a lane's fragment is 4 consecutive channels of
+// one tap, loaded from the activations (or gradients) themselves, which the
+// caches hold.  The first operand of a product is the weights, so a lane's
+// four results are four consecutive channels of one position: an 8-byte bf16
+// store.  The passes up to the activations' gradients run 16-deep products in
+// ascending order of the reduction: a rounding that moves a bf16 activation
+// moves a ReLU's mask and, through Adam, whole weights, so the order of their
+// sums is part of what a training run reproduces.
+//
+// Bound by latency and launches: a training step of 256 samples is 23 GFLOP
+// (10 us at the card's dense rate) and about 150 MB.  With im2col and col2im
+// buffers, 64x64 LDS-staged products, one-thread-per-column sums and 75
+// launches it took 2.1 ms, 0.9 ms of it in the sums over partial results.
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ v4f mma16(uint2 a, uint2 b, v4f c)
 {
-    if (row_ok && avail >= 8) {
-        *(uint4*)v = *(const uint4*)(p + i);
-        return;
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = (row_ok && q < avail) ? p[i + q] : (bf16)0;
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(v4s, a), __builtin_bit_cast(v4s, b), c, 0, 0,
+                                                     0);
 }
 
-// C[m][n] = sum_k A(m, k) B(k, n); A(m, k) = TA ? A[k][m] : A[m][k],
-// B(k, n) = TB ? B[n][k] : B[k][n].  64x64 block tile, 32-deep k tiles, four
-// waves each owning a 32x32 quarter as 2x2 MFMA 16x16 tiles.  Both operands
-// are staged in LDS k-contiguous ([m][k] and [n][k]) so each lane's MFMA
-// fragment (4 consecutive k) is one 8-byte read.
-//   splits == 1: C = acc (+ bias[n]) (ReLU) stored as fp32 (Cf) or bf16 (Cb);
-//   splits  > 1: the k range is cut into gridDim.z chunks of kchunk and chunk z
-//                stores its partial sum to Cf + z * M * ldc (no bias).
-constexpr int BM = 64, BN = 64, BK = 32, LDK = BK + 8;
-
-template <bool TA, bool TB>
-__global__ __launch_bounds__(256) void k_gemm(const bf16* __restrict__ A, int lda, const bf16* __restrict__ B, int ldb,
-                                              float* __restrict__ Cf, bf16* __restrict__ Cb, int ldc, int M, int N,
-                                              int K, int kchunk, const float* __restrict__ bias, int relu)
+__device__ __forceinline__ v4f mma32(uint4 a, uint4 b, v4f c)
 {
-    __shared__ __align__(16) bf16 As[BM][LDK];
-    __shared__ __align__(16) bf16 Bs[BN][LDK];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wm = w >> 1, wn = w & 1;
-    const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-    const int kbeg = blockIdx.z * kchunk;
-    const int kend = min(K, kbeg + kchunk);
-    v4f acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8b, a), __builtin_bit_cast(v8b, b), c, 0, 0, 0);
+}
 
-    for (int k0 = kbeg; k0 < kend; k0 += BK) {
-        // ---- A tile: rows m0..m0+63, k0..k0+31
-        if (!TA) {
-            const int r = t >> 2, ks = (t & 3) * 8;
-            const int m = m0 + r;
-            bf16 v[8];
-            load8(A, (size_t)m * lda + k0 + ks, m < M, kend - (k0 + ks), v);
-            *(uint4*)&As[r][ks] = *(const uint4*)v;
-        } else {
-            const int kr = t >> 3, ms = (t & 7) * 8;
-            const int k = k0 + kr;
-            bf16 v[8];
-            load8(A, (size_t)k * lda + m0 + ms, k < kend, M - (m0 + ms), v);
+__device__ __forceinline__ uint2 pack4(const float (&v)[4])
+{
+    return make_uint2((uint32_t)f2bf(v[0]) | (uint32_t)f2bf(v[1]) << 16,
+                      (uint32_t)f2bf(v[2]) | (uint32_t)f2bf(v[3]) << 16);
+}
+
+__device__ __forceinline__ float bf_at(uint2 p, int r)
+{
+    const uint32_t w = r < 2 ? p.x : p.y;
+    return bf2f((bf16)((r & 1) ? w >> 16 : w & 0xffffu));
+}
+
+// One layer: a 3x3 / stride 2 / pad 1 convolution (TAPS 9) or a linear layer
+// (TAPS 1, sizes 1).  Reduction index k = tap * CIN + channel, padded with
+// zeros to KP, a multiple of 32.
+template <int TAPS_, int CIN_, int COUT_, int HI_ = 1, int WI_ = 1, int HO_ = 1, int WO_ = 1>
+struct Layer {
+    static constexpr int TAPS = TAPS_, CIN = CIN_, COUT = COUT_, HI = HI_, WI = WI_, HO = HO_, WO = WO_;
+    static constexpr int K = TAPS * CIN, KP = (K + 31) / 32 * 32;
+};
+
+// Where row m of a layer's im2col matrix starts: sample n, upper left tap (h, w).
+struct RowPos {
+    int n, h, w;
+};
+
+template <class L>
+__device__ __forceinline__ RowPos row_pos(int m)
+{
+    const int n = m / (L::HO * L::WO), p = m - n * (L::HO * L::WO);
+    return {n, 2 * (p / L::WO) - 1, 2 * (p % L::WO) - 1};
+}
+
+// Elements k..k+7 (k a multiple of 8) of a row of im2col(X), 0 outside the
+// image and the reduction.  Loads go to a valid address and are selected
+// after, so that several are in flight.
+template <class L>
+__device__ __forceinline__ uint4 patch8(const bf16* __restrict__ X, const RowPos& r, int k, bool live)
+{
+    if constexpr (L::TAPS == 1) {
+        const uint4 v = *(const uint4*)(X + (size_t)r.n * L::CIN + k);
+        return live ? v : make_uint4(0, 0, 0, 0);
+    } else if constexpr (L::CIN % 8 == 0) {
+        const int tap = k / L::CIN, c = k - tap * L::CIN;
+        const int h = r.h + tap / 3, w = r.w + tap % 3;
+        const bool ok = live && k < L::K && h >= 0 && h < L::HI && w >= 0 && w < L::WI;
+        const uint4 v = *(const uint4*)(X + (ok ? ((size_t)(r.n * L::HI + h) * L::WI + w) * L::CIN + c : 0));
+        return ok ? v : make_uint4(0, 0, 0, 0);
+    } else {
+        static_assert(L::CIN == 4, "channels come in groups of 4 or 8");
+        uint32_t o[4];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) As[ms + q][kr] = v[q];
+        for (int q = 0; q < 2; ++q) {
+            const int tap = k / 4 + q;
+            const int h = r.h + tap / 3, w = r.w + tap % 3;
+            const bool ok = live && tap < L::TAPS && h >= 0 && h < L::HI && w >= 0 && w < L::WI;
+            const uint2 v = *(const uint2*)(X + (ok ? ((size_t)(r.n * L::HI + h) * L::WI + w) * 4 : 0));
+            o[2 * q] = ok ? v.x : 0u;
+            o[2 * q + 1] = ok ? v.y : 0u;
         }
-        // ---- B tile: k0..k0+31, cols n0..n0+63
-        if (!TB) {
-            const int kr = t >> 3, ns = (t & 7) * 8;
-            const int k = k0 + kr;
-            bf16 v[8];
-            load8(B, (size_t)k * ldb + n0 + ns, k < kend, N - (n0 + ns), v);
-#pragma unroll
-            for (int q = 0; q < 8; ++q) Bs[ns + q][kr] = v[q];
-        } else {
-            const int r = t >> 2, ks = (t & 3) * 8;
-            const int n = n0 + r;
-            bf16 v[8];
-            load8(B, (size_t)n * ldb + k0 + ks, n < N, kend - (k0 + ks), v);
-            *(uint4*)&Bs[r][ks] = *(const uint4*)v;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 16) {
-            v4s a[2], b[2];
-            const int kq = kk + 4 * (lane >> 4);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) a[i] = *(const v4s*)&As[wm * 32 + i * 16 + (lane & 15)][kq];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) b[j] = *(const v4s*)&Bs[wn * 32 + j * 16 + (lane & 15)][kq];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
+        return make_uint4(o[0], o[1], o[2], o[3]);
     }
-    // ---- epilogue: lane holds rows 4*(lane/16)+r, column lane%16 of each 16x16 tile
-    const bool split = gridDim.z > 1;
+}
+
+// The same for k..k+3 (k a multiple of 4).
+template <class L>
+__device__ __forceinline__ uint2 patch4(const bf16* __restrict__ X, const RowPos& r, int k)
+{
+    if constexpr (L::TAPS == 1) return *(const uint2*)(X + (size_t)r.n * L::CIN + k);
+    const int tap = k / L::CIN, c = k - tap * L::CIN;
+    const int h = r.h + tap / 3, w = r.w + tap % 3;
+    const bool ok = k < L::K && h >= 0 && h < L::HI && w >= 0 && w < L::WI;
+    const uint2 v = *(const uint2*)(X + (ok ? ((size_t)(r.n * L::HI + h) * L::WI + w) * L::CIN + c : 0));
+    return ok ? v : make_uint2(0, 0);
+}
+
+// Forward: Y = relu(im2col(X) W + b) as bf16, and for the last convolution the
+// mean over its two positions (GAP); or fp32 sums without ReLU, eight columns
+// per row and the first kHeadOut of them to `user` (HEAD).
+//   Wf: the weights in fragment order (k_pack): k step s, column tile j, lane
+//   L hold W[16 s + 4 (L >> 4) + q][16 j + (L & 15)], q = 0..3.
+// A wave forms RT row tiles x CT column tiles, in chunks of `chunk` (an even
+// number of) k steps whose sums are added in order.  KS = 1: a workgroup is
+// four waves of different rows; KS > 1, for the layers with few rows, long
+// reductions and several chunks: the KS waves share the chunks, of which there
+// are at most PARTS.  A row's sums do not depend on the rows beside it.
+enum Out { kRelu, kReluGap, kHead };
+constexpr int kHeadOut = 6, kHeadPad = 8;
+
+template <class L, int RT, int CT, int KS, Out OUT, int PARTS>
+__global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_fwd(const bf16* __restrict__ X,
+                                                                 const bf16* __restrict__ Wf,
+                                                                 const float* __restrict__ bias, int M, int chunk,
+                                                                 bf16* __restrict__ Y, bf16* __restrict__ gap,
+                                                                 float* __restrict__ out, float* __restrict__ user)
+{
+    constexpr int NT = (L::COUT + 15) / 16, STEPS = L::KP / 16, UNROLL = STEPS % 6 == 0 ? 6 : (STEPS % 4 == 0 ? 4 : 2);
+    static_assert(NT % CT == 0 && STEPS % 2 == 0, "whole column groups and pairs of steps");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row0 = (KS == 1 ? (int)blockIdx.x * 4 + wave : (int)blockIdx.x) * RT * 16, col0 = blockIdx.y * CT;
+    RowPos pos[RT];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < RT; ++i) pos[i] = row_pos<L>(min(row0 + 16 * i + (lane & 15), M - 1));
+    v4f acc[RT][CT];
+    const auto clear = [&] {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < CT; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    };
+    // U steps from s: all their loads are issued before the first product
+    const auto steps = [&](int s, auto U) {
+        uint2 w[U.value][CT], x[U.value][RT];
+#pragma unroll
+        for (int q = 0; q < U.value; ++q) {
+#pragma unroll
+            for (int j = 0; j < CT; ++j)
+                w[q][j] = *(const uint2*)(Wf + ((size_t)((s + q) * NT + col0 + j) * 64 + lane) * 4);
+#pragma unroll
+            for (int i = 0; i < RT; ++i) x[q][i] = patch4<L>(X, pos[i], 16 * (s + q) + 4 * (lane >> 4));
+        }
+#pragma unroll
+        for (int q = 0; q < U.value; ++q)
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int j = 0; j < CT; ++j) acc[i][j] = mma16(w[q][j], x[q][i], acc[i][j]);
+    };
+    const auto run = [&](int s, int end) {
+        for (; s + UNROLL <= end; s += UNROLL) steps(s, std::integral_constant<int, UNROLL>{});
+        for (; s < end; s += 2) steps(s, std::integral_constant<int, 2>{});
+    };
+    const auto store = [&](int i, int j, v4f a) {
+        const int m = row0 + 16 * i + (lane & 15), n = (col0 + j) * 16 + 4 * (lane >> 4);
+        if constexpr (OUT == kHead) {
+            if (m >= M) return;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int m = m0 + wm * 32 + i * 16 + 4 * (lane >> 4) + r;
-                const int n = n0 + wn * 32 + j * 16 + (lane & 15);
-                if (m >= M || n >= N) continue;
-                float v = acc[i][j][r];
-                if (split) {
-                    Cf[((size_t)blockIdx.z * M + m) * ldc + n] = v;
-                    continue;
-                }
-                if (bias) v += bias[n];
-                if (relu) v = fmaxf(v, 0.0f);
-                if (Cb) Cb[(size_t)m * ldc + n] = f2bf(v);
-                else Cf[(size_t)m * ldc + n] = v;
+                if (n + r >= kHeadPad) break;
+                const float v = a[r] + bias[n + r];
+                out[(size_t)m * kHeadPad + n + r] = v;
+                if (user && n + r < kHeadOut) user[(size_t)m * kHeadOut + n + r] = v;
             }
-}
-
-// Sum of split partials in split order: out[i] = sum_z part[z * n + i].
-__global__ __launch_bounds__(256) void k_split_sum(const float* __restrict__ part, int splits, size_t n,
-                                                   float* __restrict__ out)
-{
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.0f;
-    for (int z = 0; z < splits; ++z) s += part[(size_t)z * n + i];
-    out[i] = s;
-}
-
-// The same with the GEMM epilogue: + bias[col], ReLU, stored as fp32 or bf16.
-__global__ __launch_bounds__(256) void k_split_sum_epi(const float* __restrict__ part, int splits, int M, int N,
-                                                       int ldc, const float* __restrict__ bias, int relu,
-                                                       float* __restrict__ Cf, bf16* __restrict__ Cb)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= M * N) return;
-    const int m = i / N, n = i - m * N;
-    const size_t o = (size_t)m * ldc + n;
-    float s = 0.0f;
-    for (int z = 0; z < splits; ++z) s += part[(size_t)z * M * ldc + o];
-    if (bias) s += bias[n];
-    if (relu) s = fmaxf(s, 0.0f);
-    if (Cb) Cb[o] = f2bf(s);
-    else Cf[o] = s;
-}
-
-// ============================================================= conv helpers
-// im2col of a 3x3 / stride 2 / pad 1 convolution on NHWC bf16:
-// Xcol[m][k], m = (n, ho, wo), k = (kh * 3 + kw) * C + c, zero outside the
-// image and for k >= 9 C (padding of the reduction to Kp).
-__global__ __launch_bounds__(256) void k_im2col(const bf16* __restrict__ X, int Nb, int H, int W, int C, int Ho,
-                                                int Wo, int Kp, bf16* __restrict__ Xcol)
-{
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t total = (size_t)Nb * Ho * Wo * Kp;
-    if (idx >= total) return;
-    const int k = (int)(idx % Kp);
-    const size_t m = idx / Kp;
-    const int wo = (int)(m % Wo);
-    const int ho = (int)((m / Wo) % Ho);
-    const int n = (int)(m / ((size_t)Wo * Ho));
-    bf16 v = 0;
-    if (k < 9 * C) {
-        const int c = k % C, kw = (k / C) % 3, kh = k / (3 * C);
-        const int hi = 2 * ho - 1 + kh, wi = 2 * wo - 1 + kw;
-        if (hi >= 0 && hi < H && wi >= 0 && wi < W) v = X[(((size_t)n * H + hi) * W + wi) * C + c];
-    }
-    Xcol[idx] = v;
-}
-
-// col2im (the input gradient), as a gather: dX[n][h][w][c] = sum over the
-// taps (kh, kw) with h = 2 ho - 1 + kh, w = 2 wo - 1 + kw in range of
-// dXcol[(n, ho, wo)][(kh * 3 + kw) * C + c], in tap order.
-__global__ __launch_bounds__(256) void k_col2im(const float* __restrict__ dXcol, int Nb, int H, int W, int C, int Ho,
-                                                int Wo, int Kp, float* __restrict__ dX)
-{
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t total = (size_t)Nb * H * W * C;
-    if (idx >= total) return;
-    const int c = (int)(idx % C);
-    const int w = (int)((idx / C) % W);
-    const int h = (int)((idx / ((size_t)C * W)) % H);
-    const int n = (int)(idx / ((size_t)C * W * H));
-    float s = 0.0f;
-    for (int kh = 0; kh < 3; ++kh) {
-        const int hh = h + 1 - kh;
-        if (hh < 0 || (hh & 1) || (hh >> 1) >= Ho) continue;
-        for (int kw = 0; kw < 3; ++kw) {
-            const int ww = w + 1 - kw;
-            if (ww < 0 || (ww & 1) || (ww >> 1) >= Wo) continue;
-            const size_t m = ((size_t)n * Ho + (hh >> 1)) * Wo + (ww >> 1);
-            s += dXcol[m * Kp + (kh * 3 + kw) * C + c];
+        } else {
+            const float4 b = *(const float4*)(bias + n);
+            const float v[4] = {fmaxf(a[0] + b.x, 0.0f), fmaxf(a[1] + b.y, 0.0f), fmaxf(a[2] + b.z, 0.0f),
+                                fmaxf(a[3] + b.w, 0.0f)};
+            const uint2 y = pack4(v);
+            if (m < M) *(uint2*)(Y + (size_t)m * L::COUT + n) = y;
+            if constexpr (OUT == kReluGap) {
+                static_assert(L::HO * L::WO == 2, "a sample's positions are two neighbouring lanes");
+                float g[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float f = bf_at(y, r);
+                    g[r] = (f + __shfl_xor(f, 1, 64)) / 2.0f;
+                }
+                if (m < M && (lane & 1) == 0) *(uint2*)(gap + (size_t)(m >> 1) * L::COUT + n) = pack4(g);
+            }
+        }
+    };
+    if constexpr (KS == 1) {
+        v4f sum[RT][CT];
+        for (int s = 0; s < STEPS; s += chunk) {
+            clear();
+            run(s, min(STEPS, s + chunk));
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int j = 0; j < CT; ++j) sum[i][j] = s ? sum[i][j] + acc[i][j] : acc[i][j];
+        }
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < CT; ++j) store(i, j, sum[i][j]);
+    } else {
+        __shared__ v4f part[PARTS][RT * CT][64];
+        const int parts = (STEPS + chunk - 1) / chunk;
+        for (int p = wave; p < parts; p += KS) {
+            clear();
+            run(p * chunk, min(STEPS, (p + 1) * chunk));
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int j = 0; j < CT; ++j) part[p][i * CT + j][lane] = acc[i][j];
+        }
+        __syncthreads();
+        for (int t = wave; t < RT * CT; t += KS) {
+            v4f a = part[0][t][lane];
+            for (int p = 1; p < parts; ++p) a += part[p][t][lane];
+            store(t / CT, t % CT, a);
         }
     }
-    dX[idx] = s;
 }
 
-// dZ = dY where the layer's output was positive (ReLU), else 0; bf16.
-__global__ __launch_bounds__(256) void k_relu_grad(const float* __restrict__ dY, const bf16* __restrict__ Y, size_t n,
-                                                   bf16* __restrict__ dZ, float* __restrict__ dZf)
-{
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float g = (bf2f(Y[i]) > 0.0f) ? dY[i] : 0.0f;
-    dZ[i] = f2bf(g);
-    if (dZf) dZf[i] = g;
-}
+// The weights [K][ld] of every layer in k_fwd's fragment order, columns from
+// ld to the tile's end as 0, and those of the layers with an input gradient in
+// k_dgrad's (the same for the transposed weights: row tile r, k step s, lane L
+// hold W[16 r + (L & 15)][16 s + 4 (L >> 4) + q]) (blockIdx.y = job); and a copy of the input,
+// which backward needs and which gives it the loads' alignment (the last
+// blockIdx.y).
+constexpr int kLayers = 8, kPackJobs = kLayers + 6;
+struct PackJobs {
+    const bf16* src[kPackJobs];
+    bf16* dst[kPackJobs];
+    int n[kPackJobs], nt[kPackJobs], ld[kPackJobs];   // n: fragments of 4 (KP / 16 * nt * 64)
+    const bf16* x;
+    bf16* xcopy;
+    int nx, jobs;                               // fragments of 8; kPackJobs, or 0 when packed already
+};
 
-// Column sums of a [M][N] fp32 matrix (bias gradients) in two fixed-order
-// stages: chunk partials, then their sum.
-__global__ __launch_bounds__(256) void k_colsum_part(const float* __restrict__ G, int M, int N, int rows_per,
-                                                     float* __restrict__ part)
+__global__ __launch_bounds__(256) void k_pack(PackJobs P)
 {
-    const int n = blockIdx.y * 256 + threadIdx.x;
-    if (n >= N) return;
-    const int r0 = blockIdx.x * rows_per, r1 = min(M, r0 + rows_per);
-    float s = 0.0f;
-    for (int r = r0; r < r1; ++r) s += G[(size_t)r * N + n];
-    part[(size_t)blockIdx.x * N + n] = s;
-}
-
-// Global average pooling over P positions: G[n][c] = mean_p Y[n][p][c].
-__global__ __launch_bounds__(256) void k_gap_fwd(const bf16* __restrict__ Y, int Nb, int P, int C, bf16* __restrict__ G)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= Nb * C) return;
-    const int n = i / C, c = i - n * C;
-    float s = 0.0f;
-    for (int p = 0; p < P; ++p) s += bf2f(Y[((size_t)n * P + p) * C + c]);
-    G[i] = f2bf(s / (float)P);
-}
-
-__global__ __launch_bounds__(256) void k_gap_bwd(const float* __restrict__ dG, int Nb, int P, int C,
-                                                 float* __restrict__ dY)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= Nb * P * C) return;
-    const int c = i % C, n = i / (P * C);
-    dY[i] = dG[n * C + c] / (float)P;
-}
-
-// Weighted squared error over the first D of each row of O (stride ldo):
-// loss_n = sum_j w_j (O - T)^2; dO = 2 w_j (O - T) / N as bf16 (and fp32).
-__global__ __launch_bounds__(256) void k_loss(const float* __restrict__ O, int ldo, const float* __restrict__ T,
-                                              const float* __restrict__ wts, int Nb, int D, float* __restrict__ loss_n,
-                                              bf16* __restrict__ dO, float* __restrict__ dOf)
-{
-    const int n = blockIdx.x * 256 + threadIdx.x;
-    if (n >= Nb) return;
-    float l = 0.0f;
-    for (int j = 0; j < ldo; ++j) {
-        float g = 0.0f;
-        if (j < D) {
-            const float e = O[n * ldo + j] - T[n * D + j];
-            l += wts[j] * e * e;
-            g = 2.0f * wts[j] * e / (float)Nb;
+    const int l = blockIdx.y;
+    if (l == P.jobs) {
+        const bool wide = ((uintptr_t)P.x & 15) == 0;
+        for (int e = blockIdx.x * 256 + threadIdx.x; e < P.nx; e += gridDim.x * 256) {
+            const bf16* p = P.x + (size_t)e * 8;
+            uint4 v;
+            if (wide) v = *(const uint4*)p;
+            else v = make_uint4(p[0] | (uint32_t)p[1] << 16, p[2] | (uint32_t)p[3] << 16,
+                                p[4] | (uint32_t)p[5] << 16, p[6] | (uint32_t)p[7] << 16);
+            *(uint4*)(P.xcopy + (size_t)e * 8) = v;
         }
-        dO[n * ldo + j] = f2bf(g);
-        dOf[n * ldo + j] = g;
+        return;
     }
-    loss_n[n] = l;
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= P.n[l]) return;
+    const int lane = e & 63, tile = e >> 6, nt = P.nt[l], ld = P.ld[l];
+    if (l >= kLayers) {
+        const int row = (tile / nt) * 16 + (lane & 15), c = (tile % nt) * 16 + 4 * (lane >> 4);
+        *(uint2*)(P.dst[l] + (size_t)e * 4) = *(const uint2*)(P.src[l] + (size_t)row * ld + c);
+        return;
+    }
+    const int col = (tile % nt) * 16 + (lane & 15), k = (tile / nt) * 16 + 4 * (lane >> 4);
+    uint32_t o[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const bf16* p = P.src[l] + (size_t)(k + 2 * q) * ld + col;
+        o[q] = col < ld ? p[0] | (uint32_t)p[ld] << 16 : 0u;
+    }
+    *(uint2*)(P.dst[l] + (size_t)e * 4) = make_uint2(o[0], o[1]);
+}
+
+// Input gradient, through the ReLU of the layer below: dZl = (Yl > 0) ? dX : 0
+// with dX[h][w] = sum over the taps (kh, kw) with h = 2 ho - 1 + kh, w = 2 wo
+// - 1 + kw of dZ[ho][wo] W[tap]^T, and the sums of dZl over a workgroup's rows
+// (fp32, for the bias gradient) to part[workgroup][CIN].  Positions of one
+// parity of (h, w) meet the same 1, 2, 2 or 4 taps, so each parity is a
+// product of its own (blockIdx.z, the longest first).  For the linear layer
+// above the average pooling (TAPS 1) both of a sample's two positions take
+// half its gradient; it has few tiles and a long reduction, so its waves are
+// workgroups of their own, on as many CUs.  A wave forms RT row tiles x CT
+// column tiles; each tap's product is summed by itself, then the taps in order.
+//   Wp: the weights in k_dgrad's fragment order (k_pack).
+template <class L, int RT, int CT>
+__global__ __launch_bounds__(L::TAPS == 1 ? 64 : 256) void k_dgrad(const bf16* __restrict__ dZ,
+                                                                   const bf16* __restrict__ Wp,
+                                                                   const bf16* __restrict__ Yl, int N,
+                                                                   bf16* __restrict__ dZl, float* __restrict__ part)
+{
+    constexpr int WAVES = L::TAPS == 1 ? 1 : 4;
+    constexpr int NT = L::CIN / 16, STEPS = L::COUT / 16, U = STEPS > 8 ? 24 : STEPS;
+    static_assert(L::CIN % 16 == 0 && NT % CT == 0 && STEPS % U == 0, "whole tiles");
+    __shared__ float sums[WAVES][CT * 16];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row0 = ((int)blockIdx.x * WAVES + wave) * RT * 16, col0 = blockIdx.y * CT;
+    const int ph = L::TAPS == 1 ? 0 : 1 - (int)(blockIdx.z >> 1), pw = L::TAPS == 1 ? 0 : 1 - (int)(blockIdx.z & 1);
+    const int hc = (L::HI - ph + 1) / 2, wc = (L::WI - pw + 1) / 2;
+    const int M = L::TAPS == 1 ? N : N * hc * wc;
+    int n[RT], hh[RT], ww[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+        const int m = min(row0 + 16 * i + (lane & 15), M - 1);
+        if (L::TAPS == 1) {
+            n[i] = m;
+            hh[i] = ww[i] = 0;
+        } else {
+            n[i] = m / (hc * wc);
+            const int p = m - n[i] * (hc * wc);
+            hh[i] = p / wc;
+            ww[i] = p - hh[i] * wc;
+        }
+    }
+    v4f sum[RT][CT];
+    for (int a = 0; a <= ph; ++a)
+        for (int b = 0; b <= pw; ++b) {
+            // kh = 1 (even rows) or 0, 2; the output row it meets
+            const int kh = ph ? 2 * a : 1, kw = pw ? 2 * b : 1;
+            const int tap = L::TAPS == 1 ? 0 : 3 * kh + kw;
+            const int dh = ph && a == 0, dw = pw && b == 0;
+            size_t at[RT];
+            bool ok[RT];
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                const int ho = hh[i] + dh, wo = ww[i] + dw;
+                ok[i] = ho < L::HO && wo < L::WO;
+                at[i] = ok[i] ? ((size_t)(n[i] * L::HO + ho) * L::WO + wo) * L::COUT : 0;
+            }
+            const bf16* wt = Wp + ((size_t)(tap * NT + col0) * STEPS * 64 + lane) * 4;
+            v4f acc[RT][CT];
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int j = 0; j < CT; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+            for (int s = 0; s < STEPS; s += U) {
+                uint2 w[U][CT], x[U][RT];
+#pragma unroll
+                for (int q = 0; q < U; ++q) {
+                    const int c = 16 * (s + q) + 4 * (lane >> 4);
+#pragma unroll
+                    for (int j = 0; j < CT; ++j) w[q][j] = *(const uint2*)(wt + (size_t)(j * STEPS + s + q) * 256);
+#pragma unroll
+                    for (int i = 0; i < RT; ++i) {
+                        const uint2 v = *(const uint2*)(dZ + at[i] + c);
+                        x[q][i] = ok[i] ? v : make_uint2(0, 0);
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < U; ++q)
+#pragma unroll
+                    for (int i = 0; i < RT; ++i)
+#pragma unroll
+                        for (int j = 0; j < CT; ++j) acc[i][j] = mma16(w[q][j], x[q][i], acc[i][j]);
+            }
+            // a tap beyond the image adds nothing
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int j = 0; j < CT; ++j) sum[i][j] = a + b ? sum[i][j] + acc[i][j] : acc[i][j];
+        }
+    // mask, store and the sum over the tile's rows (lanes 0, 16, 32, 48 hold it)
+    const auto store = [&](int i, int j, v4f a, float (&s)[4]) {
+        const bool live = row0 + 16 * i + (lane & 15) < M;
+        const int ch = (col0 + j) * 16 + 4 * (lane >> 4);
+        constexpr int POS = L::TAPS == 1 ? 2 : 1;
+#pragma unroll
+        for (int p = 0; p < POS; ++p) {
+            const size_t o = L::TAPS == 1
+                                 ? (size_t)(2 * n[i] + p) * L::CIN + ch
+                                 : ((size_t)(n[i] * L::HI + 2 * hh[i] + ph) * L::WI + 2 * ww[i] + pw) * L::CIN + ch;
+            const uint2 y = *(const uint2*)(Yl + o);
+            float g[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                g[r] = live && bf_at(y, r) > 0.0f ? (L::TAPS == 1 ? a[r] / 2.0f : a[r]) : 0.0f;
+                s[r] += g[r];
+            }
+            if (live) *(uint2*)(dZl + o) = pack4(g);
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+        float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < RT; ++i) store(i, j, sum[i][j], s);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+#pragma unroll
+            for (int d = 1; d < 16; d <<= 1) s[r] += __shfl_xor(s[r], d, 64);
+            if ((lane & 15) == 0) sums[wave][j * 16 + 4 * (lane >> 4) + r] = s[r];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < CT * 16) {
+        float s = sums[0][threadIdx.x];
+#pragma unroll
+        for (int q = 1; q < WAVES; ++q) s += sums[q][threadIdx.x];
+        part[(size_t)(blockIdx.z * gridDim.x + blockIdx.x) * L::CIN + col0 * 16 + threadIdx.x] = s;
+    }
+}
+
+// Weight gradient: dW = im2col(X)^T dZ over the rows of split blockIdx.z
+// (rows_per of them), to out[split][KP][COUT].  The reduction runs over rows,
+// so both operands go through LDS transposed: a thread loads 4 rows x 8
+// channels and writes 8 four-row columns of 8 bytes; the next chunk's loads
+// fly behind the products.  A workgroup forms 64 reduction rows x BN columns,
+// each wave 16 rows.
+constexpr int kWgTile = 64, kWgChunk = 64, kWgLd = kWgChunk + 8;
+
+__device__ __forceinline__ void transpose_store(const uint4 (&v)[4], bf16* to)
+{
+    const uint32_t r[4][4] = {{v[0].x, v[0].y, v[0].z, v[0].w},
+                              {v[1].x, v[1].y, v[1].z, v[1].w},
+                              {v[2].x, v[2].y, v[2].z, v[2].w},
+                              {v[3].x, v[3].y, v[3].z, v[3].w}};
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const uint32_t sel = (q & 1) ? 0x07060302u : 0x05040100u;
+        *(uint2*)(to + q * kWgLd) = make_uint2(__builtin_amdgcn_perm(r[1][q >> 1], r[0][q >> 1], sel),
+                                               __builtin_amdgcn_perm(r[3][q >> 1], r[2][q >> 1], sel));
+    }
+}
+
+template <class L, int BN>
+__global__ __launch_bounds__(256) void k_wgrad(const bf16* __restrict__ X, const bf16* __restrict__ dZ, int M,
+                                               int rows_per, float* __restrict__ out)
+{
+    constexpr int NT = BN / 16, XU = kWgChunk / 4 * (kWgTile / 8), ZU = kWgChunk / 4 * (BN / 8);
+    static_assert(L::COUT % BN == 0 && ZU <= 256 && XU <= 256, "a thread stages one unit of each operand");
+    __shared__ __align__(16) bf16 Xs[kWgTile][kWgLd];
+    __shared__ __align__(16) bf16 Zs[BN][kWgLd];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int k0 = blockIdx.x * kWgTile, n0 = blockIdx.y * BN;
+    const int mbeg = blockIdx.z * rows_per, mend = min(M, mbeg + rows_per);
+    const int xk = (t % (kWgTile / 8)) * 8, xm = t / (kWgTile / 8) * 4;
+    const int u = 255 - t;                              // the other end's threads stage dZ
+    const int zn = (u % (BN / 8)) * 8, zm = u / (BN / 8) * 4;
+    uint4 xv[4], zv[4];
+    const auto load = [&](int m0) {
+        if (t < XU) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = m0 + xm + r;
+                xv[r] = patch8<L>(X, row_pos<L>(min(m, M - 1)), k0 + xk, m < mend && k0 + xk < L::KP);
+            }
+        }
+        if (u < ZU) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = m0 + zm + r;
+                const uint4 v = *(const uint4*)(dZ + (size_t)min(m, M - 1) * L::COUT + n0 + zn);
+                zv[r] = m < mend ? v : make_uint4(0, 0, 0, 0);
+            }
+        }
+    };
+    v4f acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
+    load(mbeg);
+    for (int m0 = mbeg; m0 < mend; m0 += kWgChunk) {
+        if (t < XU) transpose_store(xv, &Xs[xk][xm]);
+        if (u < ZU) transpose_store(zv, &Zs[zn][zm]);
+        __syncthreads();
+        if (m0 + kWgChunk < mend) load(m0 + kWgChunk);
+#pragma unroll
+        for (int s = 0; s < kWgChunk; s += 32) {
+            const int q = s + 8 * (lane >> 4);
+            const uint4 x = *(const uint4*)&Xs[wave * 16 + (lane & 15)][q];
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[j] = mma32(*(const uint4*)&Zs[j * 16 + (lane & 15)][q], x, acc[j]);
+        }
+        __syncthreads();
+    }
+    const int k = k0 + wave * 16 + (lane & 15);
+    if (k >= L::KP) return;
+    float* o = out + ((size_t)blockIdx.z * L::KP + k) * L::COUT + n0 + 4 * (lane >> 4);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) *(v4f*)(o + 16 * j) = acc[j];
+}
+
+// The head's gradients: the weighted squared error over the first kHeadOut
+// outputs, loss = sum_j w_j (O - T)^2 and dO = 2 w_j (O - T) / N; then for the
+// linear layers dZ1 = (H1 > 0) ? dO W2^T : 0 (bf16) and, summed over the 16
+// samples of a chunk (blockIdx.y), H1^T dO, dZ1 and dO.  A thread is one
+// hidden unit, except in dO W2^T, which is formed as the other layers' products.
+constexpr int kHeadChunk = 16;
+struct LossWeights {
+    float w[kHeadOut];
+};
+
+__global__ __launch_bounds__(256) void k_head_bwd(const float* __restrict__ O, const float* __restrict__ T,
+                                                  LossWeights lw, int N, int H, const bf16* __restrict__ h1,
+                                                  const bf16* __restrict__ W2, float* __restrict__ loss,
+                                                  bf16* __restrict__ dz1, float* __restrict__ partW2,
+                                                  float* __restrict__ partB1, float* __restrict__ partB2)
+{
+    __shared__ float d16[kHeadChunk][kHeadOut], d32[kHeadChunk][kHeadOut];
+    __shared__ __align__(8) bf16 db[kHeadChunk][kHeadPad];
+    __shared__ v4f gs[256 / 4][kHeadChunk + 1];
+    const int r0 = blockIdx.y * kHeadChunk, rows = min(kHeadChunk, N - r0);
+    const int j = blockIdx.x * 256 + threadIdx.x;
+    if (threadIdx.x < kHeadChunk)
+        for (int q = 0; q < kHeadPad; ++q) db[threadIdx.x][q] = 0;
+    if ((int)threadIdx.x < rows) {
+        const int n = r0 + threadIdx.x;
+        float l = 0.0f;
+        for (int q = 0; q < kHeadOut; ++q) {
+            const float e = O[(size_t)n * kHeadPad + q] - T[(size_t)n * kHeadOut + q];
+            l += lw.w[q] * e * e;
+            const float g = 2.0f * lw.w[q] * e / (float)N;
+            d32[threadIdx.x][q] = g;
+            db[threadIdx.x][q] = f2bf(g);
+            d16[threadIdx.x][q] = bf2f(f2bf(g));
+        }
+        if (loss && blockIdx.x == 0) loss[n] = l;
+    }
+    __syncthreads();
+    if (blockIdx.x == 0 && threadIdx.x < kHeadPad) {
+        float s = 0.0f;
+        if (threadIdx.x < kHeadOut)
+            for (int r = 0; r < rows; ++r) s += d32[r][threadIdx.x];
+        partB2[(size_t)blockIdx.y * kHeadPad + threadIdx.x] = s;
+    }
+    {
+        // dO W2^T of the workgroup's units, four tiles of 16 a wave
+        const int lane = threadIdx.x & 63, g4 = lane >> 4;
+        const uint2 x = g4 < 2 ? *(const uint2*)&db[lane & 15][4 * g4] : make_uint2(0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int tile = (threadIdx.x >> 6) * 4 + q, unit = min((int)blockIdx.x * 256 + tile * 16 + (lane & 15), H - 1);
+            const uint2 v = *(const uint2*)(W2 + (size_t)unit * kHeadPad + 4 * (g4 & 1));
+            gs[tile * 4 + g4][lane & 15] = mma16(g4 < 2 ? v : make_uint2(0, 0), x, v4f{0.f, 0.f, 0.f, 0.f});
+        }
+    }
+    __syncthreads();
+    if (j >= H) return;
+    bf16 hv[kHeadChunk];
+#pragma unroll
+    for (int r = 0; r < kHeadChunk; ++r) hv[r] = h1[(size_t)(r0 + min(r, rows - 1)) * H + j];
+    float sw[kHeadPad] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, sb = 0.0f;
+#pragma unroll
+    for (int r = 0; r < kHeadChunk; ++r) {
+        if (r >= rows) break;
+        const float h = bf2f(hv[r]);
+#pragma unroll
+        for (int q = 0; q < kHeadOut; ++q) sw[q] += h * d16[r][q];
+        const float g = h > 0.0f ? gs[threadIdx.x >> 2][r][threadIdx.x & 3] : 0.0f;
+        sb += g;
+        dz1[(size_t)(r0 + r) * H + j] = f2bf(g);
+    }
+    partB1[(size_t)blockIdx.y * H + j] = sb;
+    float* o = partW2 + ((size_t)blockIdx.y * H + j) * kHeadPad;
+    *(float4*)o = make_float4(sw[0], sw[1], sw[2], sw[3]);
+    *(float4*)(o + 4) = make_float4(sw[4], sw[5], sw[6], sw[7]);
+}
+
+// Every gradient's sum over its partial results, in one launch: 16 threads
+// share a group of four values, each sums every 16th part, and their sums are
+// added in order.
+constexpr int kSumJobs = 2 * kLayers;
+struct SumJobs {
+    const float* part[kSumJobs];
+    float* dst[kSumJobs];
+    int parts[kSumJobs], n[kSumJobs], first[kSumJobs];   // values per part (of 4); first workgroup
+    int count;
+};
+
+__global__ __launch_bounds__(256) void k_sum_parts(SumJobs J)
+{
+    int s = 0;
+    while (s + 1 < J.count && (int)blockIdx.x >= J.first[s + 1]) ++s;
+    const int lane = threadIdx.x & 15, share = threadIdx.x >> 4;
+    const int i = (((int)blockIdx.x - J.first[s]) * 16 + lane) * 4, n = J.n[s];
+    __shared__ v4f sums[16][16];
+    v4f a = v4f{0.f, 0.f, 0.f, 0.f};
+    if (i < n) {
+        const float* p = J.part[s] + i;
+        const int parts = J.parts[s];
+#pragma unroll 4
+        for (int z = share; z < parts; z += 16) a += *(const v4f*)(p + (size_t)z * n);
+    }
+    sums[share][lane] = a;
+    __syncthreads();
+    if (share == 0 && i < n) {
+#pragma unroll
+        for (int q = 1; q < 16; ++q) a += sums[q][lane];
+        *(v4f*)(J.dst[s] + i) = a;
+    }
 }
 
 // Adam with decoupled weight decay on fp32 master weights; writes the bf16
@@ -419,16 +751,19 @@ struct cnn_net_s {
     unsigned int* infer_ticket = nullptr;
     uint8_t* mask = nullptr;
     int step = 0;
-    // activations of the last forward (for backward), sized for max_batch
-    bf16* xcol[kConvs] = {};
+    // the weights in k_fwd's and k_dgrad's fragment orders (k_pack), repacked likewise
+    bf16* pf = nullptr;
+    size_t pf_off[kPackJobs] = {};
+    unsigned long long fver = 0;
+    // a copy of the last forward's input (the caller's may be gone before
+    // cnn_backward) and its activations, sized for max_batch
+    bf16* x = nullptr;
     bf16* y[kConvs] = {};
     bf16 *gap = nullptr, *h1 = nullptr;
     float* out = nullptr;            // [N][8]
-    // backward scratch
-    float *dy = nullptr, *dx = nullptr, *dcol = nullptr, *split = nullptr, *colpart = nullptr;
-    bf16 *dz = nullptr, *dob = nullptr;
-    float *dof = nullptr, *lossn = nullptr, *wts = nullptr;
-    size_t split_elems = 0, colpart_elems = 0;
+    // backward scratch: gradients before the activations, partial sums
+    bf16 *dz[kConvs] = {}, *dz1 = nullptr;
+    float* part = nullptr;
     std::vector<void*> allocs;
 };
 
@@ -466,82 +801,155 @@ int launch_check(const char* what)
 
 inline dim3 g1(size_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
-// C = op(A) op(B) with the conventions of k_gemm; splits > 1 reduces through
-// c->split (fp32 [splits][M][ldc]) into Cf.
-int gemm(cnn_net_s* c, bool ta, const bf16* A, int lda, bool tb, const bf16* B, int ldb, float* Cf, bf16* Cb,
-         int ldc, int M, int N, int K, const float* bias, bool relu, int splits)
+// ---- the layers of the training pass, and their tiles
+using Conv0 = Layer<9, 4, 32, 60, 80, 30, 40>;
+using Conv1 = Layer<9, 32, 64, 30, 40, 15, 20>;
+using Conv2 = Layer<9, 64, 96, 15, 20, 8, 10>;
+using Conv3 = Layer<9, 96, 128, 8, 10, 4, 5>;
+using Conv4 = Layer<9, 128, 128, 4, 5, 2, 3>;
+using Conv5 = Layer<9, 128, 128, 2, 3, 1, 2>;
+using Fc1 = Layer<1, kFc1In, kFc1Out>;
+using Fc2 = Layer<1, kFc1Out, kOutPad>;
+static_assert(kOut == kHeadOut && kOutPad == kHeadPad, "the head's outputs");
+
+// A weight gradient's rows are split until its workgroups give each of the
+// 256 CUs one or two (more splits only write more partial sums); with few
+// rows a single workgroup per tile writes the gradient itself.
+constexpr int kWgBlocks = 384;
+
+template <class L, int BN>
+constexpr int wgrad_max_splits()
 {
-    if (splits < 1) splits = 1;
-    const int kchunk = ((cdiv(K, splits) + BK - 1) / BK) * BK;
-    splits = cdiv(K, kchunk);
-    if (splits > 1 && (size_t)splits * M * ldc > c->split_elems) return CNN_ERR_ARG;
-    dim3 grid(cdiv(M, BM), cdiv(N, BN), splits);
-    float* out = splits > 1 ? c->split : Cf;
-    bf16* outb = splits > 1 ? nullptr : Cb;
-    const float* bb = splits > 1 ? nullptr : bias;
-    const int rl = (splits > 1) ? 0 : (relu ? 1 : 0);
-    if (!ta && !tb)
-        hipLaunchKernelGGL((k_gemm<false, false>), grid, dim3(256), 0, c->stream, A, lda, B, ldb, out, outb, ldc, M, N, K,
-                           kchunk, bb, rl);
-    else if (!ta && tb)
-        hipLaunchKernelGGL((k_gemm<false, true>), grid, dim3(256), 0, c->stream, A, lda, B, ldb, out, outb, ldc, M, N, K,
-                           kchunk, bb, rl);
-    else if (ta && !tb)
-        hipLaunchKernelGGL((k_gemm<true, false>), grid, dim3(256), 0, c->stream, A, lda, B, ldb, out, outb, ldc, M, N, K,
-                           kchunk, bb, rl);
-    else
-        hipLaunchKernelGGL((k_gemm<true, true>), grid, dim3(256), 0, c->stream, A, lda, B, ldb, out, outb, ldc, M, N, K,
-                           kchunk, bb, rl);
-    if (splits > 1) {
-        if (!bias && !relu && Cf) {
-            const size_t n = (size_t)M * ldc;
-            hipLaunchKernelGGL(k_split_sum, g1(n), dim3(256), 0, c->stream, c->split, splits, n, Cf);
-        } else {
-            hipLaunchKernelGGL(k_split_sum_epi, g1((size_t)M * N), dim3(256), 0, c->stream, c->split, splits, M, N,
-                               ldc, bias, relu ? 1 : 0, Cf, Cb);
+    return std::max(1, kWgBlocks / (((L::K + kWgTile - 1) / kWgTile) * (L::COUT / BN)));
+}
+
+template <class L, int BN>
+constexpr size_t wgrad_part_elems()
+{
+    return (size_t)wgrad_max_splits<L, BN>() * L::KP * L::COUT;
+}
+
+// Workgroups along the rows of k_dgrad's largest parity class.
+template <class L, int RT>
+int dgrad_blocks(int N)
+{
+    return L::TAPS == 1 ? cdiv(N, 16 * RT) : cdiv(N * ((L::HI + 1) / 2) * ((L::WI + 1) / 2), 64 * RT);
+}
+
+// The chunks of a forward layer's reduction (k steps of 16 each; an even
+// number): one, unless the layer has few 64x64 output tiles, then at most
+// K / 128, aiming at 64 tiles and chunks.  For inference-sized batches (N <=
+// 64) it is chosen from one sample's rows, so a sample's output, bit for bit,
+// does not depend on the batch the sample runs in; training batches choose
+// from all rows.
+template <class L>
+int fwd_chunk(int N)
+{
+    const int rows = L::HO * L::WO, tiles = cdiv(N <= 64 ? rows : N * rows, 64) * cdiv(L::COUT, 64);
+    const int splits = tiles >= 64 ? 1 : std::max(1, std::min(64 / tiles, L::KP / 128));
+    return cdiv(cdiv(L::KP, splits), 32) * 2;
+}
+
+template <class L, int RT, int CT, int KS, Out OUT, int PARTS = 1>
+void launch_fwd(cnn_net_s* c, int layer, const bf16* X, int N, const float* bias, bf16* Y, bf16* gap = nullptr,
+                float* out = nullptr, float* user = nullptr)
+{
+    static_assert(KS == 1 || L::KP / 128 <= PARTS, "fwd_chunk's chunks fit the kernel's LDS");
+    const int M = N * L::HO * L::WO;
+    const dim3 grid(cdiv(M, (KS == 1 ? 64 : 16) * RT), cdiv(L::COUT, 16) / CT);
+    hipLaunchKernelGGL((k_fwd<L, RT, CT, KS, OUT, PARTS>), grid, dim3(KS == 1 ? 256 : 64 * KS), 0, c->stream, X,
+                       c->pf + c->pf_off[layer], bias, M, fwd_chunk<L>(N), Y, gap, out, user);
+}
+
+// The packed weights, when they have changed since the last pack, and a copy
+// of N samples (none: x null).
+void pack(cnn_net_s* c, const bf16* x, int N)
+{
+    PackJobs J{};
+    J.x = x;
+    J.xcopy = c->x;
+    J.nx = x ? N * (60 * 80 * 4 / 8) : 0;
+    int frags = 0;
+    if (c->fver != c->wver) {
+        J.jobs = kPackJobs;
+        for (int q = 0; q < kPackJobs; ++q) {
+            const int l = q < kLayers ? q : q - kLayers + 1;
+            const Param& w = l < kConvs ? c->convW[l] : (l == kConvs ? c->fc1W : c->fc2W);
+            J.ld[q] = l < kConvs ? kSpec[l].cout : (l == kConvs ? kFc1Out : kOutPad);
+            J.nt[q] = cdiv(J.ld[q], 16);
+            J.n[q] = (int)(w.n / J.ld[q]) / 16 * J.nt[q] * 64;
+            J.src[q] = c->pb + w.off;
+            J.dst[q] = c->pf + c->pf_off[q];
+            frags = std::max(frags, J.n[q]);
         }
+        c->fver = c->wver;
     }
-    return launch_check("gemm");
+    const int blocks = std::max(cdiv(frags, 256), std::min(cdiv(J.nx, 256), 2048));
+    hipLaunchKernelGGL(k_pack, dim3(blocks, J.jobs + 1), dim3(256), 0, c->stream, J);
 }
 
-int colsum(cnn_net_s* c, const float* G, int M, int N, float* out)
+// The partial sums of one backward pass, taken from c->part in order.
+struct Parts {
+    cnn_net_s* c;
+    SumJobs jobs{};
+    size_t used = 0;
+    int blocks = 0;
+
+    float* take(size_t n)
+    {
+        float* p = c->part + used;
+        used += n;
+        return p;
+    }
+    // dst = the sum of `parts` parts of n values (a multiple of 4) at p
+    void sum(const float* p, int parts, int n, float* dst)
+    {
+        const int q = jobs.count++;
+        jobs.part[q] = p;
+        jobs.dst[q] = dst;
+        jobs.parts[q] = parts;
+        jobs.n[q] = n;
+        jobs.first[q] = blocks;
+        blocks += cdiv(n, 64);
+    }
+};
+
+template <class L, int BN>
+void launch_wgrad(Parts& w, const bf16* X, const bf16* dZ, int M, float* dst)
 {
-    const int chunks = std::min(256, std::max(1, M / 64));
-    const int rows_per = cdiv(M, chunks);
-    if ((size_t)chunks * N > c->colpart_elems) return CNN_ERR_ARG;
-    hipLaunchKernelGGL(k_colsum_part, dim3(chunks, cdiv(N, 256)), dim3(256), 0, c->stream, G, M, N, rows_per,
-                       c->colpart);
-    hipLaunchKernelGGL(k_split_sum, g1(N), dim3(256), 0, c->stream, c->colpart, chunks, (size_t)N, out);
-    return launch_check("colsum");
+    const int kt = cdiv(L::K, kWgTile), chunks = cdiv(M, kWgChunk);
+    int splits = std::min(wgrad_max_splits<L, BN>(), chunks);
+    if (chunks <= 8 && kt * (L::COUT / BN) >= 48) splits = 1;
+    const int rows_per = cdiv(chunks, splits) * kWgChunk;
+    splits = cdiv(M, rows_per);
+    float* out = splits == 1 ? dst : w.take((size_t)splits * L::KP * L::COUT);
+    hipLaunchKernelGGL((k_wgrad<L, BN>), dim3(kt, L::COUT / BN, splits), dim3(256), 0, w.c->stream, X, dZ, M,
+                       rows_per, out);
+    if (splits > 1) w.sum(out, splits, L::KP * L::COUT, dst);
 }
 
-// Forward GEMMs with few output tiles (small batches) split the reduction so
-// more than a handful of workgroups share it: at most K / 128 chunks, aiming
-// at 64 workgroups.
-int fwd_splits(int M, int N, int K)
+template <class L, int RT, int CT>
+void launch_dgrad(Parts& w, const bf16* dZ, const bf16* W, const bf16* Yl, int N, bf16* dZl, float* dbias)
 {
-    const int tiles = cdiv(M, BM) * cdiv(N, BN);
-    if (tiles >= 64) return 1;
-    return std::max(1, std::min(64 / tiles, K / 128));
+    const int classes = L::TAPS == 1 ? 1 : 4, blocks = dgrad_blocks<L, RT>(N);
+    float* out = w.take((size_t)classes * blocks * L::CIN);
+    hipLaunchKernelGGL((k_dgrad<L, RT, CT>), dim3(blocks, L::CIN / 16 / CT, classes), dim3(L::TAPS == 1 ? 64 : 256), 0, w.c->stream, dZ, W, Yl, N, dZl, out);
+    w.sum(out, classes * blocks, L::CIN, dbias);
 }
 
-// The split count of a forward GEMM of N samples with `rows` output rows
-// each.  For inference-sized batches (N <= 64) it is chosen from one
-// sample's rows, so the k-chunks and their summation order -- and with them
-// a sample's output, bit for bit -- do not depend on the batch the sample
-// runs in; training batches choose from all rows.
-int fwd_splits_n(int N, int rows, int cols, int K)
+// Room for the partial sums of a batch of N (all of cnn_backward's takes).
+size_t part_elems(int N)
 {
-    return fwd_splits(N <= 64 ? rows : N * rows, cols, K);
-}
-
-int splits_for(int K, int MN)
-{
-    // enough blocks along the reduction when the output tile count is small
-    const int tiles = std::max(1, MN / (BM * BN));
-    int s = std::max(1, 512 / tiles);
-    s = std::min(s, std::max(1, K / 512));
-    return s;
+    const size_t chunks = cdiv(N, kHeadChunk);
+    size_t n = wgrad_part_elems<Conv0, 32>() + wgrad_part_elems<Conv1, 64>() + wgrad_part_elems<Conv2, 96>() +
+               wgrad_part_elems<Conv3, 128>() + wgrad_part_elems<Conv4, 128>() + wgrad_part_elems<Conv5, 128>() +
+               wgrad_part_elems<Fc1, 128>();
+    n += chunks * ((size_t)kFc1Out * (kOutPad + 1) + kOutPad);
+    n += 4 * ((size_t)dgrad_blocks<Conv1, 2>(N) * Conv1::CIN + (size_t)dgrad_blocks<Conv2, 2>(N) * Conv2::CIN +
+              (size_t)dgrad_blocks<Conv3, 1>(N) * Conv3::CIN + (size_t)dgrad_blocks<Conv4, 1>(N) * Conv4::CIN +
+              (size_t)dgrad_blocks<Conv5, 1>(N) * Conv5::CIN) +
+         (size_t)dgrad_blocks<Fc1, 1>(N) * Fc1::CIN;
+    return n;
 }
 
 }  // namespace
@@ -691,7 +1099,7 @@ __device__ __forceinline__ void infer_conv(const bf16* __restrict__ X, bf16* __r
                                            const float* __restrict__ bias)
 {
     constexpr int M = HO * WO, MT = (M + 15) / 16, NT = COUT / 16, CH = MT < 4 ? MT : 4;
-    constexpr int KREAL = 9 * CIN, KP = ((KREAL + BK - 1) / BK) * BK, KS = KP / 16;
+    constexpr int KREAL = 9 * CIN, KP = (KREAL + 31) / 32 * 32, KS = KP / 16;
     static_assert(COUT % 16 == 0 && CIN % 4 == 0 && KP % 16 == 0, "tile shapes");
     const int wave = threadIdx.x >> 6;
     constexpr int WAVES = kInferThreads / 64;
@@ -863,7 +1271,7 @@ int cnn_create(int max_batch, cnn_net* out)
         off += (n + 63) & ~(size_t)63;
     };
     for (int l = 0; l < kConvs; ++l) {
-        c->Kp[l] = ((9 * kSpec[l].cin + BK - 1) / BK) * BK;
+        c->Kp[l] = (9 * kSpec[l].cin + 31) / 32 * 32;
         take(c->convW[l], (size_t)c->Kp[l] * kSpec[l].cout);
         take(c->convB[l], kSpec[l].cout);
     }
@@ -873,7 +1281,6 @@ int cnn_create(int max_batch, cnn_net* out)
     take(c->fc2B, kOutPad);
     c->nparam = off;
     const int N = max_batch;
-    size_t big = 0, split = 0;
     int rc = CNN_OK;
     rc = rc ? rc : dalloc(c, &c->p, off);
     rc = rc ? rc : dalloc(c, &c->g, off);
@@ -891,29 +1298,24 @@ int cnn_create(int max_batch, cnn_net* out)
     rc = rc ? rc : dalloc(c, &c->infer_part, (size_t)N * kHeadGroups * kOutPad);
     rc = rc ? rc : dalloc(c, &c->infer_ticket, (size_t)N);
     for (int l = 0; l < kConvs && !rc; ++l) {
-        const size_t M = (size_t)N * kSpec[l].ho * kSpec[l].wo;
-        rc = dalloc(c, &c->xcol[l], M * c->Kp[l]);
-        rc = rc ? rc : dalloc(c, &c->y[l], M * kSpec[l].cout);
-        big = std::max(big, M * (size_t)c->Kp[l]);
-        big = std::max(big, (size_t)N * kSpec[l].hi * kSpec[l].wi * kSpec[l].cin);
-        split = std::max(split, (size_t)c->Kp[l] * kSpec[l].cout);
+        const size_t n = (size_t)N * kSpec[l].ho * kSpec[l].wo * kSpec[l].cout;
+        rc = dalloc(c, &c->y[l], n);
+        rc = rc ? rc : dalloc(c, &c->dz[l], n);
     }
-    split = std::max(split, (size_t)kFc1In * kFc1Out);
-    c->split_elems = split * 64;
-    c->colpart_elems = (size_t)256 * 256;
+    size_t pf_n = 0;
+    for (int q = 0; q < kPackJobs; ++q) {
+        const int l = q < kLayers ? q : q - kLayers + 1;   // conv 1..5 and fc1 have input gradients
+        c->pf_off[q] = pf_n;
+        pf_n += l < kConvs ? (size_t)c->Kp[l] * kSpec[l].cout
+                           : (l == kConvs ? (size_t)kFc1In * kFc1Out : (size_t)kFc1Out * 16);
+    }
+    rc = rc ? rc : dalloc(c, &c->pf, pf_n);
+    rc = rc ? rc : dalloc(c, &c->x, (size_t)N * 60 * 80 * 4);
     rc = rc ? rc : dalloc(c, &c->gap, (size_t)N * kFc1In);
     rc = rc ? rc : dalloc(c, &c->h1, (size_t)N * kFc1Out);
+    rc = rc ? rc : dalloc(c, &c->dz1, (size_t)N * kFc1Out);
     rc = rc ? rc : dalloc(c, &c->out, (size_t)N * kOutPad);
-    rc = rc ? rc : dalloc(c, &c->dy, big);
-    rc = rc ? rc : dalloc(c, &c->dx, big);
-    rc = rc ? rc : dalloc(c, &c->dcol, big);
-    rc = rc ? rc : dalloc(c, &c->dz, big);
-    rc = rc ? rc : dalloc(c, &c->split, c->split_elems);
-    rc = rc ? rc : dalloc(c, &c->colpart, c->colpart_elems);
-    rc = rc ? rc : dalloc(c, &c->dob, (size_t)N * kOutPad);
-    rc = rc ? rc : dalloc(c, &c->dof, (size_t)N * kOutPad);
-    rc = rc ? rc : dalloc(c, &c->lossn, (size_t)N);
-    rc = rc ? rc : dalloc(c, &c->wts, (size_t)kOutPad);
+    rc = rc ? rc : dalloc(c, &c->part, part_elems(N));
     if (rc) {
         cnn_destroy(c);
         return rc;
@@ -1020,29 +1422,16 @@ int cnn_prepare_input(cnn_net c, const float* depth_a, const uint8_t* image_a, c
 int cnn_forward(cnn_net c, const void* x, int N, float* out)
 {
     if (!c || !x || N < 1 || N > c->max_batch) return CNN_ERR_ARG;
-    const bf16* in = (const bf16*)x;
-    int rc;
-    for (int l = 0; l < kConvs; ++l) {
-        const ConvSpec& s = kSpec[l];
-        const int M = N * s.ho * s.wo;
-        const size_t tot = (size_t)M * c->Kp[l];
-        hipLaunchKernelGGL(k_im2col, g1(tot), dim3(256), 0, c->stream, in, N, s.hi, s.wi, s.cin, s.ho, s.wo, c->Kp[l],
-                           c->xcol[l]);
-        if ((rc = gemm(c, false, c->xcol[l], c->Kp[l], false, c->pb + c->convW[l].off, s.cout, nullptr, c->y[l], s.cout,
-                       M, s.cout, c->Kp[l], c->p + c->convB[l].off, true,
-                       fwd_splits_n(N, s.ho * s.wo, s.cout, c->Kp[l]))))
-            return rc;
-        in = c->y[l];
-    }
-    hipLaunchKernelGGL(k_gap_fwd, g1((size_t)N * kFc1In), dim3(256), 0, c->stream, c->y[kConvs - 1], N, 2, kFc1In,
-                       c->gap);
-    if ((rc = gemm(c, false, c->gap, kFc1In, false, c->pb + c->fc1W.off, kFc1Out, nullptr, c->h1, kFc1Out, N, kFc1Out,
-                   kFc1In, c->p + c->fc1B.off, true, fwd_splits_n(N, 1, kFc1Out, kFc1In))))
-        return rc;
-    if ((rc = gemm(c, false, c->h1, kFc1Out, false, c->pb + c->fc2W.off, kOutPad, c->out, nullptr, kOutPad, N, kOutPad,
-                   kFc1Out, c->p + c->fc2B.off, false, fwd_splits_n(N, 1, kOutPad, kFc1Out))))
-        return rc;
-    if (out) CK(hipMemcpy2DAsync(out, kOut * 4, c->out, kOutPad * 4, kOut * 4, N, hipMemcpyDeviceToDevice, c->stream));
+    pack(c, (const bf16*)x, N);
+    const auto b = [&](const Param& p) { return c->p + p.off; };
+    launch_fwd<Conv0, 4, 2, 1, kRelu>(c, 0, c->x, N, b(c->convB[0]), c->y[0]);
+    launch_fwd<Conv1, 2, 4, 1, kRelu>(c, 1, c->y[0], N, b(c->convB[1]), c->y[1]);
+    launch_fwd<Conv2, 1, 3, 1, kRelu>(c, 2, c->y[1], N, b(c->convB[2]), c->y[2]);
+    launch_fwd<Conv3, 1, 4, 1, kRelu>(c, 3, c->y[2], N, b(c->convB[3]), c->y[3]);
+    launch_fwd<Conv4, 1, 1, 1, kRelu>(c, 4, c->y[3], N, b(c->convB[4]), c->y[4]);
+    launch_fwd<Conv5, 1, 1, 4, kReluGap, 9>(c, 5, c->y[4], N, b(c->convB[5]), c->y[5], c->gap);
+    launch_fwd<Fc1, 1, 4, 1, kRelu>(c, 6, c->gap, N, b(c->fc1B), c->h1);
+    launch_fwd<Fc2, 1, 1, 16, kHead, 30>(c, 7, c->h1, N, b(c->fc2B), nullptr, nullptr, c->out, out);
     return launch_check("forward");
 }
 
@@ -1189,52 +1578,35 @@ int cnn_set_infer_split(cnn_net c, int split)
 int cnn_backward(cnn_net c, int N, const float* target, const float* w, float* loss_n)
 {
     if (!c || !target || !w || N < 1 || N > c->max_batch) return CNN_ERR_ARG;
-    int rc;
-    float wp[kOutPad] = {0};
-    for (int j = 0; j < kOut; ++j) wp[j] = w[j];
-    CK(hipMemcpyAsync(c->wts, wp, sizeof wp, hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(k_loss, g1(N), dim3(256), 0, c->stream, c->out, kOutPad, target, c->wts, N, kOut, c->lossn,
-                       c->dob, c->dof);
-    if (loss_n) CK(hipMemcpyAsync(loss_n, c->lossn, N * 4, hipMemcpyDeviceToDevice, c->stream));
-    // fc2: dW2 = H1^T dO, db2 = colsum dO, dH1 = dO W2^T
-    if ((rc = gemm(c, true, c->h1, kFc1Out, false, c->dob, kOutPad, c->g + c->fc2W.off, nullptr, kOutPad, kFc1Out,
-                   kOutPad, N, nullptr, false, splits_for(N, kFc1Out * kOutPad))))
-        return rc;
-    if ((rc = colsum(c, c->dof, N, kOutPad, c->g + c->fc2B.off))) return rc;
-    if ((rc = gemm(c, false, c->dob, kOutPad, true, c->pb + c->fc2W.off, kOutPad, c->dy, nullptr, kFc1Out, N, kFc1Out,
-                   kOutPad, nullptr, false, 1)))
-        return rc;
-    // fc1 (ReLU): dZ1 = dH1 * (H1 > 0); dW1 = G^T dZ1; db1; dG = dZ1 W1^T
-    hipLaunchKernelGGL(k_relu_grad, g1((size_t)N * kFc1Out), dim3(256), 0, c->stream, c->dy, c->h1,
-                       (size_t)N * kFc1Out, c->dz, c->dx);
-    if ((rc = gemm(c, true, c->gap, kFc1In, false, c->dz, kFc1Out, c->g + c->fc1W.off, nullptr, kFc1Out, kFc1In,
-                   kFc1Out, N, nullptr, false, splits_for(N, kFc1In * kFc1Out))))
-        return rc;
-    if ((rc = colsum(c, c->dx, N, kFc1Out, c->g + c->fc1B.off))) return rc;
-    if ((rc = gemm(c, false, c->dz, kFc1Out, true, c->pb + c->fc1W.off, kFc1Out, c->dcol, nullptr, kFc1In, N, kFc1In,
-                   kFc1Out, nullptr, false, 1)))
-        return rc;
-    // GAP backward into dy of the last conv
-    hipLaunchKernelGGL(k_gap_bwd, g1((size_t)N * 2 * kFc1In), dim3(256), 0, c->stream, c->dcol, N, 2, kFc1In, c->dy);
-    for (int l = kConvs - 1; l >= 0; --l) {
-        const ConvSpec& s = kSpec[l];
-        const int M = N * s.ho * s.wo;
-        const size_t ny = (size_t)M * s.cout;
-        // dZ = dY * (Y > 0); fp32 copy in dx for the bias sums
-        hipLaunchKernelGGL(k_relu_grad, g1(ny), dim3(256), 0, c->stream, c->dy, c->y[l], ny, c->dz, c->dx);
-        if ((rc = gemm(c, true, c->xcol[l], c->Kp[l], false, c->dz, s.cout, c->g + c->convW[l].off, nullptr, s.cout,
-                       c->Kp[l], s.cout, M, nullptr, false, splits_for(M, c->Kp[l] * s.cout))))
-            return rc;
-        if ((rc = colsum(c, c->dx, M, s.cout, c->g + c->convB[l].off))) return rc;
-        if (l == 0) break;
-        // dXcol = dZ W^T, then col2im into dy of the layer below
-        if ((rc = gemm(c, false, c->dz, s.cout, true, c->pb + c->convW[l].off, s.cout, c->dcol, nullptr, c->Kp[l], M,
-                       c->Kp[l], s.cout, nullptr, false, 1)))
-            return rc;
-        const size_t nx = (size_t)N * s.hi * s.wi * s.cin;
-        hipLaunchKernelGGL(k_col2im, g1(nx), dim3(256), 0, c->stream, c->dcol, N, s.hi, s.wi, s.cin, s.ho, s.wo,
-                           c->Kp[l], c->dy);
-    }
+    if (c->fver != c->wver) pack(c, nullptr, 0);   // the gradients are those of the present weights
+    LossWeights lw;
+    for (int j = 0; j < kOut; ++j) lw.w[j] = w[j];
+    Parts P{c};
+    const auto g = [&](const Param& p) { return c->g + p.off; };
+    const auto wd = [&](int l) { return (const bf16*)(c->pf + c->pf_off[kLayers + l - 1]); };   // conv l, or fc1 as 6
+    const int chunks = cdiv(N, kHeadChunk);
+    float* pw2 = P.take((size_t)chunks * kFc1Out * kOutPad);
+    float* pb1 = P.take((size_t)chunks * kFc1Out);
+    float* pb2 = P.take((size_t)chunks * kOutPad);
+    hipLaunchKernelGGL(k_head_bwd, dim3(cdiv(kFc1Out, 256), chunks), dim3(256), 0, c->stream, c->out, target, lw, N,
+                       kFc1Out, c->h1, c->pb + c->fc2W.off, loss_n, c->dz1, pw2, pb1, pb2);
+    P.sum(pw2, chunks, kFc1Out * kOutPad, g(c->fc2W));
+    P.sum(pb1, chunks, kFc1Out, g(c->fc1B));
+    P.sum(pb2, chunks, kOutPad, g(c->fc2B));
+    launch_wgrad<Fc1, 128>(P, c->gap, c->dz1, N, g(c->fc1W));
+    launch_dgrad<Fc1, 1, 1>(P, c->dz1, wd(6), c->y[5], N, c->dz[5], g(c->convB[5]));
+    launch_wgrad<Conv5, 128>(P, c->y[4], c->dz[5], N * 2, g(c->convW[5]));
+    launch_dgrad<Conv5, 1, 1>(P, c->dz[5], wd(5), c->y[4], N, c->dz[4], g(c->convB[4]));
+    launch_wgrad<Conv4, 128>(P, c->y[3], c->dz[4], N * 6, g(c->convW[4]));
+    launch_dgrad<Conv4, 1, 1>(P, c->dz[4], wd(4), c->y[3], N, c->dz[3], g(c->convB[3]));
+    launch_wgrad<Conv3, 128>(P, c->y[2], c->dz[3], N * 20, g(c->convW[3]));
+    launch_dgrad<Conv3, 1, 3>(P, c->dz[3], wd(3), c->y[2], N, c->dz[2], g(c->convB[2]));
+    launch_wgrad<Conv2, 96>(P, c->y[1], c->dz[2], N * 80, g(c->convW[2]));
+    launch_dgrad<Conv2, 2, 4>(P, c->dz[2], wd(2), c->y[1], N, c->dz[1], g(c->convB[1]));
+    launch_wgrad<Conv1, 64>(P, c->y[0], c->dz[1], N * 300, g(c->convW[1]));
+    launch_dgrad<Conv1, 2, 2>(P, c->dz[1], wd(1), c->y[0], N, c->dz[0], g(c->convB[0]));
+    launch_wgrad<Conv0, 32>(P, c->x, c->dz[0], N * 1200, g(c->convW[0]));
+    hipLaunchKernelGGL(k_sum_parts, dim3(P.blocks), dim3(256), 0, c->stream, P.jobs);
     return launch_check("backward");
 }
 

@@ -85,6 +85,58 @@ def test_backward_matches_oracle(setup):
         assert rel(G[name], ge[name]) < 6e-2, (name, rel(G[name], ge[name]))
 
 
+def gradients(net, x, target, keep=True):
+    """Outputs, losses and gradients of one pass; keep False: the input lies 2
+    bytes off any wider alignment and is overwritten before the backward pass
+    (the forward keeps its own copy)."""
+    import torch
+    buf = torch.zeros(x.size + 8, dtype=torch.bfloat16, device="cuda")
+    off = 0 if keep else 1
+    xt = buf[off:off + x.size].reshape(x.shape)
+    xt.copy_(torch.from_numpy(np.ascontiguousarray(x)).to(torch.bfloat16))
+    out = net.forward(xt).cpu().numpy()
+    if not keep:
+        buf.zero_()
+    loss = net.backward(x.shape[0], torch.from_numpy(np.ascontiguousarray(target)).cuda()).cpu().numpy()
+    return out, loss, net.get_grads().astype(np.float64)
+
+
+@pytest.mark.parametrize("n", [1, 3, 17, 33, 64, 66])
+def test_gradients_at_the_edges_of_the_tiles(setup, n):
+    """Batches whose rows end inside a 16-row tile, a 64-row chunk and a
+    workgroup of every layer, with one sample and with rows split over
+    workgroups.  Up to 64 samples a sample's forward is the same in every
+    batch, so a batch's gradients are the mean of its samples' own but for
+    bf16 roundings (2^-9 each, of the outputs' gradients over n and of each
+    layer's): 1e-2.  Above, the forward's sums have another order and a
+    ReLU's mask may flip, which moves that sample's gradient by a few per
+    cent and the mean by 1/66 of it.  The one sample is checked against the
+    oracle with the same rounding points, as test_backward_matches_oracle."""
+    from slam_amd.warmstart import WarmStartNet
+    co = setup["co"]
+    net = WarmStartNet(max_batch=n)
+    net.init_params(seed=5)
+    rng = np.random.default_rng(n)
+    x = bf16_round(rng.uniform(0, 1, size=(n, 60, 80, 4)))
+    target = rng.normal(size=(n, 6)).astype(np.float32)
+    out, loss, flat = gradients(net, x, target, keep=False)
+    if n == 1:
+        ref_out, _ = co.forward(setup["p"], x, rnd=co.bf16)
+        ref_loss, ref = co.loss_and_grads(setup["p"], x, target, np.ones(6, np.float32), rnd=co.bf16)
+    else:
+        one = [gradients(net, x[i:i + 1], target[i:i + 1]) for i in range(n)]
+        ref_out = np.concatenate([o[0] for o in one])
+        ref_loss = np.mean([o[1] for o in one])
+        ref = co.unpack(np.mean([o[2] for o in one], axis=0))
+        if n <= 64:
+            assert np.array_equal(out, ref_out)
+    assert rel(out, ref_out) < 1e-2, rel(out, ref_out)
+    assert abs(loss.mean() - ref_loss) < 1e-2 * ref_loss
+    G = co.unpack(flat)
+    for name in ref:
+        assert rel(G[name], ref[name]) < 1e-2 and cos(G[name], ref[name]) > 0.9999, (name, rel(G[name], ref[name]))
+
+
 def test_training_reduces_loss():
     """2048 rendered pairs, 10 epochs on the GPU with the library's kernels:
     the training loss falls by 40 %, the validation loss falls, and the
