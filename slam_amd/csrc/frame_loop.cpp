@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "host_stage.h"
 #include "odom_internal.h"
 #include "slam_cnn.h"
 #include "slam_loop.h"
@@ -21,6 +22,8 @@ struct efloop_ctx {
     splat_handle pred = nullptr;
     surfel_handle model = nullptr;
     uint16_t* filtered = nullptr;    // device, the bilateral output
+    slam::HostStage uploads;         // host frames: each is copied to the device once
+    uint8_t *dev_rgb = nullptr, *dev_depth = nullptr;
     float pose[16];
     float last_pose[16];
     int tick = 0;
@@ -36,13 +39,35 @@ void free_loop(efloop_ctx* c)
     if (c->model) surfel_destroy(c->model);
     if (c->pred) splat_destroy(c->pred);
     if (c->odo) odom_destroy(c->odo);
-    if (c->filtered) (void)hipFree(c->filtered);
+    for (void* p : {(void*)c->filtered, (void*)c->dev_rgb, (void*)c->dev_depth})
+        if (p) (void)hipFree(p);
     delete c;
 }
 
 odom_frame_view device_view(const void* p, int w, int h, int bpp, int fmt)
 {
     return odom_frame_view{p, w * bpp, w, h, fmt, ODOM_MEM_DEVICE};
+}
+
+// The frame `v` of `bpp` bytes a pixel for the frame's stages: a host frame is
+// copied to `buf` (allocated on first use), once for all of them.  A view that
+// the stages would refuse stays as it is, for them to refuse.
+int to_device(efloop_ctx* c, const odom_frame_view* v, int fmt, int bpp, uint8_t** buf, odom_frame_view* out)
+{
+    *out = *v;
+    const size_t row = (size_t)c->w * bpp, pitch = v->pitch_bytes ? v->pitch_bytes : row;
+    if (v->mem != ODOM_MEM_HOST || !v->ptr || v->format != fmt || v->width != c->w || v->height != c->h ||
+        v->pitch_bytes < 0 || pitch < row || pitch % (bpp == 2 ? 2 : 1) != 0)
+        return ODOM_OK;
+    void* stream = nullptr;
+    if (int rc = odom_get_stream(c->odo, &stream)) return rc;
+    if (!*buf && hipMalloc((void**)buf, row * c->h) != hipSuccess) {
+        *buf = nullptr;
+        return ODOM_ERR_HIP;
+    }
+    if (c->uploads.upload(*buf, v->ptr, pitch, row, c->h, (hipStream_t)stream) != hipSuccess) return ODOM_ERR_HIP;
+    *out = device_view(*buf, c->w, c->h, bpp, fmt);
+    return ODOM_OK;
 }
 
 // max(|t|, angle(R)) of the motion between two rigid poses, in double
@@ -70,16 +95,21 @@ double motion(const float cur[16], const float last[16])
 // frame the model's initialisation and initFirstRGB, on later frames the
 // init calls of frame-to-model tracking against the filled-in prediction
 // (elastic_fusion_file.cpp:342-374).  *first: this was the first frame.
-int loop_begin_frame(efloop_ctx* c, const odom_frame_view* rgb, const odom_frame_view* depth, bool* first)
+// rgb and depth become the device's copies; the colour is copied while the
+// device works on the depth and the model.
+int loop_begin_frame(efloop_ctx* c, odom_frame_view* rgb, odom_frame_view* depth, bool* first)
 {
     const efloop_params& p = c->p;
-    int rc = odom_bilateral_depth(c->odo, depth, p.depth_cutoff, c->filtered, ODOM_MEM_DEVICE);
+    int rc = to_device(c, depth, ODOM_FMT_DEPTH_U16, 2, &c->dev_depth, depth);
+    if (rc) return rc;
+    rc = odom_bilateral_depth(c->odo, depth, p.depth_cutoff, c->filtered, ODOM_MEM_DEVICE);
     if (rc) return rc;
     const odom_frame_view filt = device_view(c->filtered, c->w, c->h, 2, ODOM_FMT_DEPTH_U16);
     c->tick += 1;
     *first = c->tick == 1;
     if (*first) {
-        rc = surfel_initialise(c->model, rgb, depth, &filt, p.depth_cutoff, c->tick, p.max_depth);
+        rc = to_device(c, rgb, ODOM_FMT_RGB8, 3, &c->dev_rgb, rgb);
+        if (!rc) rc = surfel_initialise(c->model, rgb, depth, &filt, p.depth_cutoff, c->tick, p.max_depth);
         if (!rc) rc = odom_init_first_rgb(c->odo, rgb);
         return rc;
     }
@@ -96,6 +126,7 @@ int loop_begin_frame(efloop_ctx* c, const odom_frame_view* rgb, const odom_frame
     rc = odom_init_icp_model(c->odo, &vv, &nv, p.max_depth, c->pose);
     if (!rc) rc = odom_init_rgb_model(c->odo, &iv);
     if (!rc) rc = odom_init_icp_depth(c->odo, &filt, p.max_depth);
+    if (!rc) rc = to_device(c, rgb, ODOM_FMT_RGB8, 3, &c->dev_rgb, rgb);
     if (!rc) rc = odom_init_rgb(c->odo, rgb);
     return rc;
 }
@@ -210,9 +241,11 @@ int efloop_destroy(efloop_handle c)
     return ODOM_OK;
 }
 
-int efloop_process(efloop_handle c, const odom_frame_view* rgb, const odom_frame_view* depth, float pose_out[16])
+int efloop_process(efloop_handle c, const odom_frame_view* rgb_in, const odom_frame_view* depth_in, float pose_out[16])
 {
-    if (!c || !rgb || !depth || !pose_out) return ODOM_ERR_ARG;
+    if (!c || !rgb_in || !depth_in || !pose_out) return ODOM_ERR_ARG;
+    odom_frame_view frame[2] = {*rgb_in, *depth_in};
+    odom_frame_view *rgb = &frame[0], *depth = &frame[1];
     bool first = false;
     int rc = loop_begin_frame(c, rgb, depth, &first);
     if (rc) return rc;
@@ -356,10 +389,12 @@ int efloop_batch_set_net(efloop_batch b, const float* params, size_t nparams, fl
     return ODOM_OK;
 }
 
-int efloop_batch_process(efloop_batch b, const odom_frame_view* rgb, const odom_frame_view* depth, float* poses_out)
+int efloop_batch_process(efloop_batch b, const odom_frame_view* rgb_in, const odom_frame_view* depth_in,
+                         float* poses_out)
 {
-    if (!b || !rgb || !depth || !poses_out) return ODOM_ERR_ARG;
+    if (!b || !rgb_in || !depth_in || !poses_out) return ODOM_ERR_ARG;
     const int n = (int)b->loops.size();
+    std::vector<odom_frame_view> rgb(rgb_in, rgb_in + n), depth(depth_in, depth_in + n);
     bool first = false;
     int rc = ODOM_OK;
     for (int i = 0; i < n && !rc; ++i) {

@@ -19,6 +19,7 @@
 #include <string>
 #include <vector>
 
+#include "host_stage.h"
 #include "host_wait.h"
 #include "timing_events.h"
 #include "odom_internal.h"
@@ -88,6 +89,7 @@ StepShape batch_shape(int kernel, int level)
 }  // namespace
 
 struct odom_ctx {
+    slam::HostStage uploads;         // host frames on their way to the device
     odom_params prm{};
     int w[kLevels], h[kLevels], n[kLevels];
     float fx[kLevels], fy[kLevels], cx[kLevels], cy[kLevels];
@@ -237,8 +239,7 @@ int resolve(odom_ctx* c, const odom_frame_view* v, int fmt_a, int fmt_b, void* s
     if (v->format == ODOM_FMT_DEPTH_U16 && (p % 2) != 0) return ODOM_ERR_ARG;
     *fmt_out = v->format;
     if (v->mem == ODOM_MEM_HOST) {
-        HIPCHK(c, hipMemcpy2DAsync(staging, row, v->ptr, p, row, v->height, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+        HIPCHK(c, c->uploads.upload(staging, v->ptr, p, row, v->height, c->stream));
         *dptr = staging;
         *pitch = row;
     } else if (v->mem == ODOM_MEM_DEVICE) {

@@ -38,6 +38,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include "host_stage.h"
 #include "slam_splat.h"
 #include "timing_events.h"
 
@@ -461,6 +462,7 @@ int cdiv(long long a, int b) { return (int)((a + b - 1) / b); }
 }  // namespace
 
 struct splat_ctx {
+    slam::HostStage uploads;         // host frames on their way to the device
     SplatCam cam{};
     hipStream_t own = nullptr;
     hipStream_t stream = nullptr;
@@ -525,8 +527,7 @@ int view_to_device(splat_ctx* c, const odom_frame_view* v, int fmt_a, int fmt_b,
     const int p = v->pitch_bytes ? v->pitch_bytes : row;
     if (p < row || (bpp == 2 && (p % 2) != 0)) return ODOM_ERR_ARG;
     if (v->mem == ODOM_MEM_HOST) {
-        SCHK(hipMemcpy2DAsync(staging, row, v->ptr, p, row, v->height, hipMemcpyHostToDevice, c->stream));
-        SCHK(hipStreamSynchronize(c->stream));
+        SCHK(c->uploads.upload(staging, v->ptr, p, row, v->height, c->stream));
         *d = (const uint8_t*)staging;
         *pitch = row;
     } else if (v->mem == ODOM_MEM_DEVICE) {
