@@ -27,8 +27,10 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
+#include "host_stage.h"
 #include "host_wait.h"
 #include "odom_math.h"
 #include "slam_surfel.h"
@@ -290,20 +292,91 @@ __device__ __forceinline__ int scan_pos(const int* prefix, const int* block_sums
     return prefix[i] + block_sums[i / kScanItems];
 }
 
+// ----------------------------------------------------------- compaction
+
+// Which of a pass's items are kept, for the pass that follows: a bit per item
+// (a 64-bit word per wave) and a count per 256.  The following pass finds an
+// item's place itself: a workgroup of kPack items adds the counts before its
+// first item (a few kB from the caches), then its own waves' bits.  Against
+// int flags, a two-level scan and its prefixes this leaves out two launches
+// per compaction (5 and 4 us at 640x480) and 8 bytes per item.
+constexpr int kPack = 1024;
+
+// Called by whole workgroups of 256; item = the workgroup's first + thread.
+__device__ __forceinline__ void keep_item(bool keep, unsigned long long* bits, int* counts)
+{
+    __shared__ int kept[4];
+    const int wave = threadIdx.x >> 6;
+    const unsigned long long m = __ballot(keep);
+    if ((threadIdx.x & 63) == 0) {
+        bits[(size_t)blockIdx.x * 4 + wave] = m;
+        kept[wave] = __popcll(m);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) counts[blockIdx.x] = (kept[0] + kept[1]) + (kept[2] + kept[3]);
+}
+
+// The place of item `block * kPack + thread` of n, or -1 if it is not kept;
+// *total: the kept items up to the end of this workgroup's.  Whole workgroups
+// of kPack.
+__device__ __forceinline__ int kept_place(int block, int n, const unsigned long long* bits, const int* counts,
+                                          int* total)
+{
+    __shared__ int before[kPack / 64], own[kPack / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i = block * kPack + threadIdx.x;
+    const unsigned long long m = (i & ~63) < n ? bits[i >> 6] : 0ull;
+    int s = 0;
+    for (int q = threadIdx.x; q < block * (kPack / 256); q += kPack) s += counts[q];
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) s += __shfl_xor(s, d, 64);
+    if (lane == 0) {
+        before[wave] = s;
+        own[wave] = __popcll(m);
+    }
+    __syncthreads();
+    int place = 0, all = 0;
+#pragma unroll
+    for (int q = 0; q < kPack / 64; ++q) {
+        place += before[q] + (q < wave ? own[q] : 0);
+        all += before[q] + own[q];
+    }
+    *total = all;
+    return (m >> lane) & 1ull ? place + __popcll(m & ((1ull << lane) - 1ull)) : -1;
+}
+
 // ------------------------------------------------------------ metric depth
 
-// depth_metric.frag:29-37 for the raw and the filtered frame.
+// depth_metric.frag:29-37 for the raw and the filtered frame: rows to columns
+// through LDS, so both the reads (64 bytes per row) and the writes (128 per
+// column) are contiguous.  5.7 us at 640x480 with a lane per row.
+constexpr int kMetricTile = 32;
+
 __global__ __launch_bounds__(256) void k_metric2(const uint8_t* raw, int rpitch, const uint8_t* filt, int fpitch,
                                                  float maxD, Img I, float* dr, float* df)
 {
-    const int d = blockIdx.x * 256 + threadIdx.x;
-    if (d >= I.w * I.h) return;
-    const int x = d / I.h, y = d - x * I.h;
+    __shared__ uint16_t t[2][kMetricTile][kMetricTile + 2];
+    const int x0 = blockIdx.x * kMetricTile, y0 = blockIdx.y * kMetricTile;
+    const int a = threadIdx.x % kMetricTile, b = threadIdx.x / kMetricTile;
     const unsigned lim = (unsigned)(maxD * 1000.0f);
-    const unsigned a = *reinterpret_cast<const uint16_t*>(raw + (size_t)y * rpitch + 2 * (size_t)x);
-    const unsigned b = *reinterpret_cast<const uint16_t*>(filt + (size_t)y * fpitch + 2 * (size_t)x);
-    dr[d] = (a > lim || a < 300u) ? 0.0f : (float)a / 1000.0f;
-    df[d] = (b > lim || b < 300u) ? 0.0f : (float)b / 1000.0f;
+#pragma unroll
+    for (int k = 0; k < kMetricTile; k += 256 / kMetricTile) {
+        const int x = x0 + a, y = y0 + b + k;
+        if (x < I.w && y < I.h) {
+            t[0][b + k][a] = *reinterpret_cast<const uint16_t*>(raw + (size_t)y * rpitch + 2 * (size_t)x);
+            t[1][b + k][a] = *reinterpret_cast<const uint16_t*>(filt + (size_t)y * fpitch + 2 * (size_t)x);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kMetricTile; k += 256 / kMetricTile) {
+        const int x = x0 + b + k, y = y0 + a;
+        if (x < I.w && y < I.h) {
+            const unsigned r = t[0][a][b + k], f = t[1][a][b + k];
+            dr[cm(I, x, y)] = (r > lim || r < 300u) ? 0.0f : (float)r / 1000.0f;
+            df[cm(I, x, y)] = (f > lim || f < 300u) ? 0.0f : (float)f / 1000.0f;
+        }
+    }
 }
 
 // ---------------------------------------------------------- initialise
@@ -484,19 +557,26 @@ struct DataArgs {
     const uint32_t* index;
     const float4* vert_conf;
     const float4* norm_rad;
-    float* pix;             // 12 floats per pixel (draw order)
-    int* flag_fresh;        // by draw index
-    unsigned* claim;        // per surfel: first draw index that matched it
+    float* pix;             // 12 floats per candidate pixel that updates or adds a surfel
+    unsigned long long* bits;   // which do (compaction)
+    int* counts;
+    unsigned* claim;        // per surfel: first candidate that matched it
     int count;              // surfels in the model the claims refer to
+    int parity, nx, ny;     // the candidates: every second pixel per axis, from `parity`
 };
 
-// data.vert:67-190 for one pixel.
+// data.vert:67-190 for one candidate: the pixels (i, j) whose centres' integer
+// parts (pixel_tc(i) * w lies within a few units in the last place of i + 0.5)
+// have the frame's parity in both axes, numbered in draw order.  The others
+// leave nothing behind, so they get no thread: 16 us at 640x480 with a thread
+// per pixel.
 __global__ __launch_bounds__(256) void k_data(DataArgs A)
 {
     const Img& I = A.I;
-    const int d = blockIdx.x * 256 + threadIdx.x;
-    if (d >= I.w * I.h) return;
-    const int i = d / I.h, j = d - i * I.h;
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    const int ei = A.ny > 0 ? e / A.ny : 0, ej = e - ei * A.ny;
+    const bool live = ei < A.nx && A.ny > 0;
+    const int i = min(2 * ei + A.parity, I.w - 1), j = min(2 * ej + A.parity, I.h - 1);
     const float u = pixel_tc(i, I.w), v = pixel_tc(j, I.h);
     const float x = u * I.cols, y = v * I.rows;
     const Cam4& c = A.c;
@@ -514,10 +594,10 @@ __global__ __launch_bounds__(256) void k_data(DataArgs A)
     o[11] = radius_of(pf[2], nl[2], c);
     int update = 0;
     unsigned best = 0;
-    const int tpar = (int)A.time % 2;
+    const int tpar = A.parity;
     const bool nb = fetch(A.dr, I, u - (1.0f / I.cols), v) != 0.0f && fetch(A.dr, I, u, v - (1.0f / I.rows)) != 0.0f &&
                     fetch(A.dr, I, u + (1.0f / I.cols), v) != 0.0f && fetch(A.dr, I, u, v + (1.0f / I.rows)) != 0.0f;
-    if ((int)x % 2 == tpar && (int)y % 2 == tpar && nb && pl[2] > 0.0f && pl[2] <= A.maxDepth) {
+    if (live && (int)x % 2 == tpar && (int)y % 2 == tpar && nb && pl[2] > 0.0f && pl[2] <= A.maxDepth) {
         int counter = 0;
         const float scale = 1.0f, wm = 2.0f;
         const float sx = (1.0f / (I.cols * scale)) * 0.5f;
@@ -599,17 +679,33 @@ __global__ __launch_bounds__(256) void k_data(DataArgs A)
         update = counter > 0 ? 1 : 2;
         o[7] = counter > 0 ? -1.0f : -2.0f;
     }
-    store12(A.pix + 12 * (size_t)d, o);
-    A.flag_fresh[d] = update > 0 ? 1 : 0;
+    if (update > 0) store12(A.pix + 12 * (size_t)e, o);
     // an index map predicted from a larger model can name surfels that are gone
-    if (update == 1 && best < (unsigned)A.count) atomicMin(A.claim + best, (unsigned)d);
+    if (update == 1 && best < (unsigned)A.count) atomicMin(A.claim + best, (unsigned)e);
+    keep_item(update > 0, A.bits, A.counts);
 }
 
-// update.vert:37-90 for the surfels a pixel claimed; clears the claims.
-__global__ __launch_bounds__(256) void k_update(float* model, int count, const float* pix, unsigned* claim, Img I,
-                                                float time)
+// Workgroups below `nb`: data.geom's transform feedback, every candidate with
+// an update or a new point in draw order to `fresh`, their number to *nfresh.
+// The others: update.vert:37-90 for the surfels a pixel claimed; clears the
+// claims.  (One launch: neither needs the other.)
+__global__ __launch_bounds__(kPack) void k_update_fresh(int nb, const float* pix, int n,
+                                                        const unsigned long long* bits, const int* counts,
+                                                        float* fresh, int* nfresh, float* model, int count,
+                                                        unsigned* claim, float time)
 {
-    const int k = blockIdx.x * 256 + threadIdx.x;
+    if ((int)blockIdx.x < nb) {
+        int total;
+        const int at = kept_place(blockIdx.x, n, bits, counts, &total);
+        if (at >= 0) {
+            float o[12];
+            load12(pix + 12 * ((size_t)blockIdx.x * kPack + threadIdx.x), o);
+            store12(fresh + 12 * (size_t)at, o);
+        }
+        if ((int)blockIdx.x == nb - 1 && threadIdx.x == 0) *nfresh = total;
+        return;
+    }
+    const int k = ((int)blockIdx.x - nb) * kPack + threadIdx.x;
     if (k >= count) return;
     const unsigned d = claim[k];
     if (d == kNoClaim) return;
@@ -646,18 +742,6 @@ __global__ __launch_bounds__(256) void k_update(float* model, int count, const f
     store12(model + 12 * (size_t)k, s);
 }
 
-// data.geom's transform feedback: every pixel with an update or a new point,
-// in draw order.
-__global__ __launch_bounds__(256) void k_fresh_scatter(const float* pix, const int* flags, const int* prefix,
-                                                       const int* block_sums, Img I, float* fresh)
-{
-    const int d = blockIdx.x * 256 + threadIdx.x;
-    if (d >= I.w * I.h || !flags[d]) return;
-    float o[12];
-    load12(pix + 12 * (size_t)d, o);
-    store12(fresh + 12 * (size_t)scan_pos(prefix, block_sums, d), o);
-}
-
 // --------------------------------------------------------------- clean
 
 struct CleanArgs {
@@ -672,22 +756,24 @@ struct CleanArgs {
     const uint32_t* index;
     const float4* vert_conf;
     const float4* color_time;
-    float* items;           // the surfel as the cleaning leaves it
-    int* flags;
+    unsigned long long* bits;   // which stay (compaction)
+    int* counts;
 };
 
-// copy_unstable.vert:48-102 (no deformation nodes).
-__global__ __launch_bounds__(256) void k_clean(CleanArgs A)
+// Item t of the cleaning: the model's surfels, then the new points, which are
+// given the frame's time.
+__device__ __forceinline__ void clean_item(const CleanArgs& A, int t, float (&s)[12])
 {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    const int nf = *A.nfresh;
-    if (t >= A.count + A.I.w * A.I.h) return;
-    if (t >= A.count + nf) {
-        A.flags[t] = 0;
-        return;
-    }
-    float s[12];
     load12(t < A.count ? A.model + 12 * (size_t)t : A.fresh + 12 * (size_t)(t - A.count), s);
+}
+
+__device__ __forceinline__ float clean_time(const CleanArgs& A, float s7) { return s7 == -2.0f ? A.time : s7; }
+
+// copy_unstable.vert:48-102 (no deformation nodes).
+__device__ __forceinline__ bool clean_keeps(const CleanArgs& A, int t)
+{
+    float s[12];
+    clean_item(A, t, s);
     const Img& I = A.I;
     float lp[3], ln[3];
     xpoint(A.Ti, s[0], s[1], s[2], lp);
@@ -720,33 +806,45 @@ __global__ __launch_bounds__(256) void k_clean(CleanArgs A)
         const bool runs = window_runs(u0, u1, sx, I.w, rx) && window_runs(v0, v1, sy, I.h, ry);
         if (runs && !rx.m[3] && !ry.m[3]) {
             // the usual 3 x 3 texels: every load issued before the first use
-            // (unused slots read a clamped, valid texel and weigh 0)
-            uint32_t id[9];
-            float4 vcs[9], cts[9];
+            // (unused slots read a clamped, valid texel and weigh 0).  A texel
+            // can count only if its confident surfel lies behind this one,
+            // which few do, so the other two maps are read only then.
+            float4 vcs[9];
+            bool any = false;
 #pragma unroll
             for (int a = 0; a < 3; ++a)
 #pragma unroll
-                for (int b = 0; b < 3; ++b) {
-                    const size_t q = cm(I, min(rx.t0 + a, I.w - 1), min(ry.t0 + b, I.h - 1));
-                    id[3 * a + b] = A.index[q];
-                    vcs[3 * a + b] = A.vert_conf[q];
-                    cts[3 * a + b] = A.color_time[q];
-                }
+                for (int b = 0; b < 3; ++b)
+                    vcs[3 * a + b] = A.vert_conf[cm(I, min(rx.t0 + a, I.w - 1), min(ry.t0 + b, I.h - 1))];
 #pragma unroll
-            for (int a = 0; a < 3; ++a)
+            for (int q = 0; q < 9; ++q) any |= vcs[q].w > A.confThreshold && vcs[q].z > lp[2];
+            if (any) {
+                uint32_t id[9];
+                float4 cts[9];
 #pragma unroll
-                for (int b = 0; b < 3; ++b) {
-                    const int times = rx.m[a] * ry.m[b];
-                    if (!times || id[3 * a + b] == 0) continue;
-                    const float4 vc = vcs[3 * a + b], ct = cts[3 * a + b];
-                    const float dx = vc.x - lp[0], dy = vc.y - lp[1];
-                    if (ct.z < s[6] && vc.w > A.confThreshold && vc.z > lp[2] && vc.z - lp[2] < 0.01f &&
-                        sqrtf(dx * dx + dy * dy) < s[11] * 1.4f)
-                        count += times;
-                    if (ct.w == tm && vc.w > A.confThreshold && vc.z > lp[2] && vc.z - lp[2] > 0.01f &&
-                        fabsf(ln[2]) > 0.85f)
-                        zcount += times;
-                }
+                for (int a = 0; a < 3; ++a)
+#pragma unroll
+                    for (int b = 0; b < 3; ++b) {
+                        const size_t q = cm(I, min(rx.t0 + a, I.w - 1), min(ry.t0 + b, I.h - 1));
+                        id[3 * a + b] = A.index[q];
+                        cts[3 * a + b] = A.color_time[q];
+                    }
+#pragma unroll
+                for (int a = 0; a < 3; ++a)
+#pragma unroll
+                    for (int b = 0; b < 3; ++b) {
+                        const int times = rx.m[a] * ry.m[b];
+                        if (!times || id[3 * a + b] == 0) continue;
+                        const float4 vc = vcs[3 * a + b], ct = cts[3 * a + b];
+                        const float dx = vc.x - lp[0], dy = vc.y - lp[1];
+                        if (ct.z < s[6] && vc.w > A.confThreshold && vc.z > lp[2] && vc.z - lp[2] < 0.01f &&
+                            sqrtf(dx * dx + dy * dy) < s[11] * 1.4f)
+                            count += times;
+                        if (ct.w == tm && vc.w > A.confThreshold && vc.z > lp[2] && vc.z - lp[2] > 0.01f &&
+                            fabsf(ln[2]) > 0.85f)
+                            zcount += times;
+                    }
+            }
         } else if (runs) {
 #pragma unroll
             for (int a = 0; a < 4; ++a)
@@ -760,23 +858,39 @@ __global__ __launch_bounds__(256) void k_clean(CleanArgs A)
     }
     int test = 1;
     if (count > 8 || zcount > 4) test = 0;
-    if (s[7] == -2.0f) s[7] = tm;
+    s[7] = clean_time(A, s[7]);
     if (s[7] == -1.0f || ((tm - s[7]) > 20.0f && s[3] < A.confThreshold)) test = 0;
     if (s[7] > 0.0f && tm - s[7] > A.timeDelta) test = 1;
-    store12(A.items + 12 * (size_t)t, s);
-    A.flags[t] = test;
+    return test != 0;
 }
 
-__global__ __launch_bounds__(256) void k_clean_scatter(const float* items, const int* flags, const int* prefix,
-                                                       const int* block_sums, int n, int max_surfels, float* out)
+__global__ __launch_bounds__(256) void k_clean(CleanArgs A)
 {
     const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= n || !flags[t]) return;
-    const int k = scan_pos(prefix, block_sums, t);
-    if (k >= max_surfels) return;
-    float s[12];
-    load12(items + 12 * (size_t)t, s);
-    store12(out + 12 * (size_t)k, s);
+    const bool keep = t < A.count + *A.nfresh && clean_keeps(A, t);
+    keep_item(keep, A.bits, A.counts);
+}
+
+// The surfels that stay, in order, read again from the model and the new
+// points rather than from a copy (24 + 5 + 4 + 8 us at 640x480 into 300k
+// surfels with the copy and a scan).  The number of them also goes to host
+// memory; the new points are appended.
+__global__ __launch_bounds__(kPack) void k_clean_pack(CleanArgs A, int n, int max_surfels, float* out, int* total,
+                                                      int* host_total, int* nfresh)
+{
+    int all;
+    const int at = kept_place(blockIdx.x, n, A.bits, A.counts, &all);
+    if (at >= 0 && at < max_surfels) {
+        float s[12];
+        clean_item(A, (int)(blockIdx.x * kPack + threadIdx.x), s);
+        s[7] = clean_time(A, s[7]);
+        store12(out + 12 * (size_t)at, s);
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        *total = all;
+        __hip_atomic_store(host_total, all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        *nfresh = 0;
+    }
 }
 
 __global__ __launch_bounds__(256) void k_fill_u64(unsigned long long* p, int n, unsigned long long v)
@@ -796,6 +910,7 @@ int cdiv(long long a, int b) { return (int)((a + b - 1) / b); }
 }  // namespace
 
 struct surfel_ctx {
+    slam::HostStage uploads;         // host frames on their way to the device
     Img I{};
     float cx = 0, cy = 0, fx = 0, fy = 0;
     int max_surfels = 0, count = 0;
@@ -812,12 +927,13 @@ struct surfel_ctx {
     float* pix = nullptr;
     float* fresh = nullptr;
     unsigned* claim = nullptr;
-    float* items = nullptr;           // max(max_surfels + npix) surfels: cleaning output before compaction
     float* feed_norm = nullptr;       // npix float4
-    int *flags = nullptr, *flags2 = nullptr;
+    int *flags = nullptr, *flags2 = nullptr;   // initialise: npix flags, prefixes and block sums
     int *prefix = nullptr, *prefix2 = nullptr;
     int *bsums = nullptr, *bsums2 = nullptr;
-    int* totals = nullptr;            // [0] scan total, [1] second scan total
+    unsigned long long* bits = nullptr;        // compaction: max_surfels + npix items
+    int* counts = nullptr;
+    int* totals = nullptr;            // [0] surfels kept (or the first scan's total), [1] new points pending
     int* h_count = nullptr;           // pinned landing buffer of the count readback
 };
 
@@ -836,8 +952,8 @@ namespace {
 void free_ctx(surfel_ctx* c)
 {
     void* b[] = {c->model[0], c->model[1], c->dr, c->df, c->raw_stage, c->filt_stage, c->rgb_stage, c->keys,
-                 c->index, c->vert_conf, c->color_time, c->norm_rad, c->pix, c->fresh, c->claim, c->items,
-                 c->feed_norm, c->flags, c->flags2, c->prefix, c->prefix2, c->bsums, c->bsums2, c->totals};
+                 c->index, c->vert_conf, c->color_time, c->norm_rad, c->pix, c->fresh, c->claim, c->bits,
+                 c->counts, c->feed_norm, c->flags, c->flags2, c->prefix, c->prefix2, c->bsums, c->bsums2, c->totals};
     for (void* p : b)
         if (p) (void)hipFree(p);
     if (c->h_count) (void)hipHostFree(c->h_count);
@@ -871,8 +987,7 @@ int view_dev(surfel_ctx* c, const odom_frame_view* v, int fmt, void* stage, cons
     const int p = v->pitch_bytes ? v->pitch_bytes : row;
     if (p < row || (bpp == 2 && (p % 2) != 0)) return ODOM_ERR_ARG;
     if (v->mem == ODOM_MEM_HOST) {
-        SCHK(hipMemcpy2DAsync(stage, row, v->ptr, p, row, v->height, hipMemcpyHostToDevice, c->stream));
-        SCHK(hipStreamSynchronize(c->stream));
+        SCHK(c->uploads.upload(stage, v->ptr, p, row, v->height, c->stream));
         *d = (const uint8_t*)stage;
         *pitch = row;
     } else if (v->mem == ODOM_MEM_DEVICE) {
@@ -893,8 +1008,7 @@ int frames(surfel_ctx* c, const odom_frame_view* rgb, const odom_frame_view* raw
     if (!rc) rc = view_dev(c, filt, ODOM_FMT_DEPTH_U16, c->filt_stage, &f, &fp);
     if (!rc) rc = view_dev(c, rgb, ODOM_FMT_RGB8, c->rgb_stage, &rv->p, &rv->pitch);
     if (rc) return rc;
-    const int npix = c->I.w * c->I.h;
-    hipLaunchKernelGGL(k_metric2, dim3(cdiv(npix, 256)), dim3(256), 0, c->stream, r, rp, f, fp, depth_cutoff, c->I,
+    hipLaunchKernelGGL(k_metric2, dim3(cdiv(c->I.w, kMetricTile), cdiv(c->I.h, kMetricTile)), dim3(256), 0, c->stream, r, rp, f, fp, depth_cutoff, c->I,
                        c->dr, c->df);
     return ODOM_OK;
 }
@@ -944,7 +1058,6 @@ void enqueue_index(surfel_ctx* c, const IndexArgs& A)
 void enqueue_fuse(surfel_ctx* c, const float pose[16], int time, const RGBView& rv, float max_depth,
                   float weighting)
 {
-    const int npix = c->I.w * c->I.h;
     DataArgs A;
     A.dr = c->dr;
     A.df = c->df;
@@ -959,16 +1072,18 @@ void enqueue_fuse(surfel_ctx* c, const float pose[16], int time, const RGBView& 
     A.vert_conf = c->vert_conf;
     A.norm_rad = c->norm_rad;
     A.pix = c->pix;
-    A.flag_fresh = c->flags2;
+    A.bits = c->bits;
+    A.counts = c->counts;
     A.claim = c->claim;
     A.count = c->count;
-    hipLaunchKernelGGL(k_data, dim3(cdiv(npix, 256)), dim3(256), 0, c->stream, A);
-    if (c->count > 0)
-        hipLaunchKernelGGL(k_update, dim3(cdiv(c->count, 256)), dim3(256), 0, c->stream, c->model[c->cur], c->count,
-                           c->pix, c->claim, c->I, (float)time);
-    scan(c, c->flags2, npix, c->prefix2, c->bsums2, c->totals + 1);
-    hipLaunchKernelGGL(k_fresh_scatter, dim3(cdiv(npix, 256)), dim3(256), 0, c->stream, c->pix, c->flags2, c->prefix2,
-                       c->bsums2, c->I, c->fresh);
+    // of the shader's float time; a negative time's remainder is no pixel's
+    A.parity = A.time < 2147483648.0f ? (int)A.time % 2 : 1;
+    A.nx = A.parity < 0 ? 0 : (c->I.w - A.parity + 1) / 2;
+    A.ny = A.parity < 0 ? 0 : (c->I.h - A.parity + 1) / 2;
+    const int n = A.nx * A.ny, nb = std::max(1, cdiv(n, kPack));
+    hipLaunchKernelGGL(k_data, dim3(std::max(1, cdiv(n, 256))), dim3(256), 0, c->stream, A);
+    hipLaunchKernelGGL(k_update_fresh, dim3(nb + cdiv(c->count, kPack)), dim3(kPack), 0, c->stream, nb, c->pix, n,
+                       c->bits, c->counts, c->fresh, c->totals + 1, c->model[c->cur], c->count, c->claim, (float)time);
 }
 
 void enqueue_clean(surfel_ctx* c, const float pose[16], int time, float conf_threshold, int time_delta)
@@ -992,12 +1107,11 @@ void enqueue_clean(surfel_ctx* c, const float pose[16], int time, float conf_thr
     A.index = c->index;
     A.vert_conf = c->vert_conf;
     A.color_time = c->color_time;
-    A.items = c->items;
-    A.flags = c->flags;
+    A.bits = c->bits;
+    A.counts = c->counts;
     hipLaunchKernelGGL(k_clean, dim3(cdiv(n, 256)), dim3(256), 0, c->stream, A);
-    scan(c, c->flags, n, c->prefix, c->bsums, c->totals);
-    hipLaunchKernelGGL(k_clean_scatter, dim3(cdiv(n, 256)), dim3(256), 0, c->stream, c->items, c->flags, c->prefix,
-                       c->bsums, n, c->max_surfels, c->model[c->cur ^ 1]);
+    hipLaunchKernelGGL(k_clean_pack, dim3(cdiv(n, kPack)), dim3(kPack), 0, c->stream, A, n, c->max_surfels,
+                       c->model[c->cur ^ 1], c->totals, c->h_count, c->totals + 1);
 }
 
 }  // namespace
@@ -1044,12 +1158,13 @@ int surfel_create(int width, int height, float cx, float cy, float fx, float fy,
     A((void**)&c->pix, np * 48);
     A((void**)&c->fresh, np * 48);
     A((void**)&c->claim, ms * 4);
-    A((void**)&c->items, ni * 48);
+    A((void**)&c->bits, (ni / 256 + 1) * 32);
+    A((void**)&c->counts, (ni / 256 + 1) * 4);
     A((void**)&c->feed_norm, np * 16);
-    A((void**)&c->flags, ni * 4);
-    A((void**)&c->flags2, ni * 4);
-    A((void**)&c->prefix, ni * 4);
-    A((void**)&c->prefix2, ni * 4);
+    A((void**)&c->flags, np * 4);
+    A((void**)&c->flags2, np * 4);
+    A((void**)&c->prefix, np * 4);
+    A((void**)&c->prefix2, np * 4);
     A((void**)&c->bsums, 4096 * 4);
     A((void**)&c->bsums2, 4096 * 4);
     A((void**)&c->totals, 16);
@@ -1144,11 +1259,9 @@ int surfel_clean(surfel_handle c, const float pose[16], int time, float conf_thr
 {
     if (!c || !pose) return ODOM_ERR_ARG;
     enqueue_clean(c, pose, time, conf_threshold, time_delta);
-    SCHK(hipMemsetAsync(c->totals + 1, 0, 4, c->stream));  // the new points are appended
     SCHK(hipGetLastError());
-    int n = 0;
-    const int rc = read_count(c, c->totals, &n);
-    if (rc) return rc;
+    SCHK(slam::poll_stream(c->stream));
+    const int n = *(volatile int*)c->h_count;
     c->cur ^= 1;
     c->count = n < c->max_surfels ? n : c->max_surfels;
     return ODOM_OK;
@@ -1274,7 +1387,6 @@ int surfel_profile(surfel_handle c, const float pose[16], int time, const odom_f
     }
     c->cur = cur0 ^ 1;
     c->count = n < c->max_surfels ? n : c->max_surfels;
-    SCHK(hipMemsetAsync(c->totals + 1, 0, 4, c->stream));
     SCHK(hipStreamSynchronize(c->stream));
     for (int k = 0; k < 4; ++k) us[k] = (float)(acc[k] * 1000.0 / reps);
     return ODOM_OK;

@@ -183,3 +183,32 @@ def test_bad_arguments_raise():
     m.predictIndices(T, 1, MAX_DEPTH, DELTA)
     assert not m.index_map()[0].any()
     assert m.clean(T, 1, CONF, DELTA) == 0
+
+
+@pytest.mark.parametrize("w,h", [(62, 66), (64, 64), (82, 50), (33, 31), (31, 33), (17, 200)])
+def test_compaction_at_the_edges_of_its_workgroups(orc, w, h):
+    """1 023, 1 024 and 1 025 candidate pixels (a quarter of the image, of
+    either parity from frame to frame), odd sizes and one narrow image: the
+    new points, the cleaned model and their order are the oracle's."""
+    cam = synth.Camera(w, h, 0.8 * w, 0.8 * w, w / 2.0, h / 2.0)
+    seq = sequence(cam, 65, 4)
+    args = (cam.width, cam.height, cam.cx, cam.cy, cam.fx, cam.fy)
+    gpu, ref = surfels.SurfelModel(*args, 5 * w * h), orc.SurfelModel(*args, 5 * w * h)
+    for k, (T, f) in enumerate(seq):
+        filt = orc.bilateral(f.depth, MAXD)
+        if k == 0:
+            assert gpu.initialise(f.rgb, f.depth, filt, DEPTH_CUTOFF, 1, MAX_DEPTH) == \
+                ref.initialise(f.rgb, f.depth, filt, DEPTH_CUTOFF, 1, MAX_DEPTH)
+            continue
+        for m in (gpu, ref):
+            m.predictIndices(T, k + 1, MAX_DEPTH, DELTA)
+            m.fuse(T, k + 1, f.rgb, f.depth, filt, DEPTH_CUTOFF, MAX_DEPTH, 1.0)
+        fg, fr = gpu.fresh(), ref.fresh()
+        assert fg.shape == fr.shape and same_bits(fg, fr), ("new points", k)
+        for m in (gpu, ref):
+            m.predictIndices(T, k + 1, MAX_DEPTH, DELTA)
+        # the second time nothing is left to append
+        for again in range(2):
+            assert gpu.clean(T, k + 1, CONF, DELTA) == ref.clean(T, k + 1, CONF, DELTA), (k, again)
+            assert same_bits(gpu.model(), ref.model()), ("cleaned model", k, again)
+        assert gpu.fresh().shape[0] == 0
