@@ -155,7 +155,7 @@ int loop_after_tracking(efloop_ctx* c, const odom_frame_view* rgb, const odom_fr
     if (!rc)
         rc = surfel_fuse(c->model, c->pose, tick, rgb, depth, &filt, p.depth_cutoff, p.max_depth, c->weighting);
     if (!rc) rc = surfel_predict_indices(c->model, c->pose, tick, p.max_depth, p.time_delta);
-    if (!rc) rc = surfel_clean(c->model, c->pose, tick, p.confidence, p.time_delta);
+    if (!rc) rc = slam::surfel_clean_enqueue(c->model, c->pose, tick, p.confidence, p.time_delta);
     return rc;
 }
 
@@ -165,13 +165,14 @@ int loop_predict(efloop_ctx* c, const odom_frame_view* rgb)
 {
     const efloop_params& p = c->p;
     const odom_frame_view filt = device_view(c->filtered, c->w, c->h, 2, ODOM_FMT_DEPTH_U16);
+    // the count of the cleaned model stays on the device: a wait for it here
+    // left the GPU idle until the prediction's launches came
     const float* mp;
+    const int* dev_n;
     int n = 0;
-    int rc = surfel_get_model(c->model, &mp);
-    if (!rc) rc = surfel_count(c->model, &n);
-    if (!rc)
-        rc = splat_combined_predict(c->pred, c->pose, mp, n, ODOM_MEM_DEVICE, p.max_depth, p.confidence, c->tick,
-                                    c->tick, p.time_delta);
+    slam::surfel_model_enqueued(c->model, &mp, &n, &dev_n);
+    int rc = slam::splat_predict_counted(c->pred, c->pose, mp, n, dev_n, p.max_depth, p.confidence, c->tick, c->tick,
+                                         p.time_delta);
     if (!rc) rc = splat_fill_in(c->pred, &filt, rgb, 0, 0);
     return rc;
 }

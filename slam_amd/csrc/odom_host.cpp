@@ -1455,6 +1455,15 @@ StepLaunch plan_launch(odom_batch_s* b, int hyp, PairDesc* dp, int kernel, int l
 // done: the last of them is finished for both refinements (k_solve), the
 // judge keeps one state per handle, and the finer levels continue with one
 // entry per handle (their first pass A reads the state the solve stored).
+// Where the fused prologue ends: its registers leave one workgroup of 512
+// threads (or two of 256) on a CU, and each further round of workgroups
+// repeats the whole solve (8 sequences at 640x480, level 0: 64 us for 1 600
+// workgroups, 10 us a round).  Past two rounds the solve is a launch of its
+// own (9 us) and the pass without it runs several workgroups per CU: 8
+// sequences in lockstep 12.0 -> 10.9 ms per 5 frames, 4 sequences 7.4 -> 6.9;
+// at two rounds or fewer the two forms are level.  The same bits either way.
+constexpr int kFusedThreads = 2 * 256 * 512;
+
 void batch_launches(odom_batch_s* b, const CallSpec& cs, PairDesc* const* dp, hipEvent_t* ev)
 {
     const TrackParams& P = cs.P;
@@ -1483,7 +1492,7 @@ void batch_launches(odom_batch_s* b, const CallSpec& cs, PairDesc* const* dp, hi
         if (ev) (void)hipEventRecord(ev[e++], b->stream);
         if (state_ready) {
             launch_step_a(La, level, iter, (int)k, prev, P, 1, nullptr, b->stream);
-        } else if (b->split_solve) {
+        } else if (b->split_solve || La.total_blocks * La.shape.threads > kFusedThreads) {
             launch_solve(cur, n * hyp, level, iter, (int)k, prev, P, La.shape.threads, b->stream);
             launch_step_a(La, level, iter, (int)k, prev, P, 1, nullptr, b->stream);
         } else {

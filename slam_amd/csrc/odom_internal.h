@@ -7,6 +7,8 @@
 
 #include "odom_device.h"
 #include "slam_odom.h"
+#include "slam_splat.h"
+#include "slam_surfel.h"
 
 namespace slam {
 
@@ -14,6 +16,19 @@ namespace slam {
 // odom_get_pose or odom_get_stats), without a device round trip; for a caller
 // that has just made one of those calls.  ODOM_ERR_ARG before any readback.
 int odom_stats_last_read(odom_handle c, odom_stats* s);
+
+// surfel_clean without its wait for the surfel count, for a caller that goes
+// on enqueuing: until a surfel_* call that needs the count waits for it, the
+// model has at most *upper surfels (those before and the new points), their
+// number in device memory at *dev_count (which may exceed *upper where the
+// buffer is full).
+int surfel_clean_enqueue(surfel_handle c, const float pose[16], int time, float conf_threshold, int time_delta);
+// The current model, its surfels (an upper bound) and, while a count is
+// outstanding, the device's count (else null).
+void surfel_model_enqueued(surfel_handle c, const float** dev_ptr, int* upper, const int** dev_count);
+// splat_combined_predict of a device model of min(n, *dev_count) surfels.
+int splat_predict_counted(splat_handle c, const float pose[16], const float* model, int n, const int* dev_count,
+                          float depth_cutoff, float conf_threshold, int time, int max_time, int time_delta);
 
 // Launch shape of a step kernel at one level (replaces GPUConfig.h's
 // threads/blocks table; chosen by the autotuner).

@@ -39,6 +39,7 @@
 #include <string.h>
 
 #include "host_stage.h"
+#include "odom_internal.h"
 #include "slam_splat.h"
 #include "timing_events.h"
 
@@ -279,13 +280,17 @@ __global__ __launch_bounds__(256) void k_fill_keys(unsigned long long* keys, int
 // a time, after the lanes' own small ones.
 constexpr int kBigSprite = 100;
 
-__global__ __launch_bounds__(256) void k_splat_raster(const float4* __restrict__ model, int n, SplatUniforms U,
+// dev_n: if set, the model has min(n, *dev_n) surfels (a count that the host
+// has not read).
+__global__ __launch_bounds__(256) void k_splat_raster(const float4* __restrict__ model, int n,
+                                                      const int* __restrict__ dev_n, SplatUniforms U,
                                                       const float4* __restrict__ rays, unsigned long long* keys,
                                                       unsigned long long* frag_count)
 {
     const int k = blockIdx.x * 256 + threadIdx.x;
     Surf s{};
     int i0 = 0, j0 = 0, ncols = 1, cnt = 0;
+    if (dev_n) n = min(n, *dev_n);
     if (k < n) {
         const size_t b = (size_t)k * 3;
         float xw, yw, size;
@@ -539,11 +544,11 @@ int view_to_device(splat_ctx* c, const odom_frame_view* v, int fmt_a, int fmt_b,
     return ODOM_OK;
 }
 
-int enqueue_predict(splat_ctx* c, const SplatUniforms& U, const float* model, int n, bool count)
+int enqueue_predict(splat_ctx* c, const SplatUniforms& U, const float* model, int n, const int* dev_n, bool count)
 {
     if (n > 0)
-        hipLaunchKernelGGL(k_splat_raster, dim3(cdiv(n, 256)), dim3(256), 0, c->stream, (const float4*)model, n, U,
-                           c->rays, c->keys, count ? c->frag_count : nullptr);
+        hipLaunchKernelGGL(k_splat_raster, dim3(cdiv(n, 256)), dim3(256), 0, c->stream, (const float4*)model, n,
+                           dev_n, U, c->rays, c->keys, count ? c->frag_count : nullptr);
     const int npix = c->cam.w * c->cam.h;
     hipLaunchKernelGGL(k_splat_resolve, dim3(cdiv(npix, 256)), dim3(256), 0, c->stream, (const float4*)model, U,
                        c->rays, c->keys, c->image, c->vertex, c->normal, c->time);
@@ -675,7 +680,7 @@ int splat_combined_predict(splat_handle c, const float pose[16], const float* mo
     }
     SplatUniforms U;
     make_uniforms(c, pose, depth_cutoff, conf_threshold, time, max_time, time_delta, &U);
-    return enqueue_predict(c, U, dmodel, n, false);
+    return enqueue_predict(c, U, dmodel, n, nullptr, false);
 }
 
 int splat_fill_in(splat_handle c, const odom_frame_view* depth, const odom_frame_view* rgb, int passthrough_geometry,
@@ -739,7 +744,7 @@ int splat_profile(splat_handle c, const float pose[16], const float* model_dev, 
         const bool last = r == reps - 1;
         if (last) SCHK(hipMemsetAsync(c->frag_count, 0, 8, c->stream));
         SCHK(hipEventRecord(ev[0], c->stream));
-        hipLaunchKernelGGL(k_splat_raster, dim3(cdiv(n, 256)), dim3(256), 0, c->stream, (const float4*)model_dev, n,
+        hipLaunchKernelGGL(k_splat_raster, dim3(cdiv(n, 256)), dim3(256), 0, c->stream, (const float4*)model_dev, n, nullptr,
                            U, c->rays, c->keys, last ? c->frag_count : nullptr);
         SCHK(hipEventRecord(ev[1], c->stream));
         hipLaunchKernelGGL(k_splat_resolve, dim3(cdiv(npix, 256)), dim3(256), 0, c->stream,
@@ -767,3 +772,15 @@ int splat_profile(splat_handle c, const float pose[16], const float* model_dev, 
 }
 
 }  // extern "C"
+
+namespace slam {
+
+int splat_predict_counted(splat_handle c, const float pose[16], const float* model, int n, const int* dev_count,
+                          float depth_cutoff, float conf_threshold, int time, int max_time, int time_delta)
+{
+    SplatUniforms U;
+    make_uniforms(c, pose, depth_cutoff, conf_threshold, time, max_time, time_delta, &U);
+    return enqueue_predict(c, U, model, n, dev_count, false);
+}
+
+}  // namespace slam

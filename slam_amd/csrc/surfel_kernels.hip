@@ -32,6 +32,7 @@
 
 #include "host_stage.h"
 #include "host_wait.h"
+#include "odom_internal.h"
 #include "odom_math.h"
 #include "slam_surfel.h"
 #include "timing_events.h"
@@ -913,7 +914,8 @@ struct surfel_ctx {
     slam::HostStage uploads;         // host frames on their way to the device
     Img I{};
     float cx = 0, cy = 0, fx = 0, fy = 0;
-    int max_surfels = 0, count = 0;
+    int max_surfels = 0, count = 0;  // while `pending`, count is the upper bound
+    bool pending = false;            // the cleaning's count is on its way to h_count
     hipStream_t own = nullptr, stream = nullptr;
     float* model[2] = {nullptr, nullptr};
     int cur = 0;
@@ -1021,6 +1023,17 @@ void scan(surfel_ctx* c, const int* flags, int n, int* prefix, int* bsums, int* 
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, c->stream, bsums, nb, total);
 }
 
+// The surfel count, waiting for it if a cleaning's is outstanding.
+int settle(surfel_ctx* c)
+{
+    if (!c->pending) return ODOM_OK;
+    SCHK(slam::poll_stream(c->stream));
+    const int n = *(volatile int*)c->h_count;
+    c->count = n < c->max_surfels ? n : c->max_surfels;
+    c->pending = false;
+    return ODOM_OK;
+}
+
 int read_count(surfel_ctx* c, const int* dev, int* out)
 {
     SCHK(hipMemcpyAsync(c->h_count, dev, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -1086,10 +1099,12 @@ void enqueue_fuse(surfel_ctx* c, const float pose[16], int time, const RGBView& 
                        c->bits, c->counts, c->fresh, c->totals + 1, c->model[c->cur], c->count, c->claim, (float)time);
 }
 
+// The most points that a frame adds: its candidate pixels.
+int max_fresh(const surfel_ctx* c) { return ((c->I.w + 1) / 2) * ((c->I.h + 1) / 2); }
+
 void enqueue_clean(surfel_ctx* c, const float pose[16], int time, float conf_threshold, int time_delta)
 {
-    const int npix = c->I.w * c->I.h;
-    const int n = c->count + npix;
+    const int n = c->count + max_fresh(c);
     CleanArgs A;
     A.model = c->model[c->cur];
     A.count = c->count;
@@ -1201,6 +1216,7 @@ int surfel_destroy(surfel_handle c)
 int surfel_set_stream(surfel_handle c, void* stream)
 {
     if (!c) return ODOM_ERR_ARG;
+    if (int rc = settle(c)) return rc;
     SCHK(hipStreamSynchronize(c->stream));
     c->stream = stream ? (hipStream_t)stream : c->own;
     return ODOM_OK;
@@ -1210,8 +1226,10 @@ int surfel_initialise(surfel_handle c, const odom_frame_view* rgb, const odom_fr
                       const odom_frame_view* filtered_depth, float depth_cutoff, int time, float max_depth)
 {
     if (!c) return ODOM_ERR_ARG;
+    int rc = settle(c);
+    if (rc) return rc;
     RGBView rv;
-    int rc = frames(c, rgb, raw_depth, filtered_depth, depth_cutoff, &rv);
+    rc = frames(c, rgb, raw_depth, filtered_depth, depth_cutoff, &rv);
     if (rc) return rc;
     const int npix = c->I.w * c->I.h;
     const Cam4 cam{c->cx, c->cy, 1.0f / c->fx, 1.0f / c->fy};  // FeedbackBuffer::compute's 1.0f / f
@@ -1237,6 +1255,7 @@ int surfel_initialise(surfel_handle c, const odom_frame_view* rgb, const odom_fr
 int surfel_predict_indices(surfel_handle c, const float pose[16], int time, float max_depth, int time_delta)
 {
     if (!c || !pose) return ODOM_ERR_ARG;
+    if (int rc = settle(c)) return rc;
     enqueue_index(c, index_args(c, pose, time, max_depth, time_delta));
     SCHK(hipGetLastError());
     return ODOM_OK;
@@ -1247,6 +1266,7 @@ int surfel_fuse(surfel_handle c, const float pose[16], int time, const odom_fram
                 float max_depth, float weighting)
 {
     if (!c || !pose) return ODOM_ERR_ARG;
+    if (int rc = settle(c)) return rc;
     RGBView rv;
     const int rc = frames(c, rgb, raw_depth, filtered_depth, depth_cutoff, &rv);
     if (rc) return rc;
@@ -1258,18 +1278,14 @@ int surfel_fuse(surfel_handle c, const float pose[16], int time, const odom_fram
 int surfel_clean(surfel_handle c, const float pose[16], int time, float conf_threshold, int time_delta)
 {
     if (!c || !pose) return ODOM_ERR_ARG;
-    enqueue_clean(c, pose, time, conf_threshold, time_delta);
-    SCHK(hipGetLastError());
-    SCHK(slam::poll_stream(c->stream));
-    const int n = *(volatile int*)c->h_count;
-    c->cur ^= 1;
-    c->count = n < c->max_surfels ? n : c->max_surfels;
-    return ODOM_OK;
+    const int rc = slam::surfel_clean_enqueue(c, pose, time, conf_threshold, time_delta);
+    return rc ? rc : settle(c);
 }
 
 int surfel_count(surfel_handle c, int* count)
 {
     if (!c || !count) return ODOM_ERR_ARG;
+    if (int rc = settle(c)) return rc;
     *count = c->count;
     return ODOM_OK;
 }
@@ -1277,6 +1293,7 @@ int surfel_count(surfel_handle c, int* count)
 int surfel_get_model(surfel_handle c, const float** dev_ptr)
 {
     if (!c || !dev_ptr) return ODOM_ERR_ARG;
+    if (int rc = settle(c)) return rc;
     *dev_ptr = c->model[c->cur];
     return ODOM_OK;
 }
@@ -1284,6 +1301,7 @@ int surfel_get_model(surfel_handle c, const float** dev_ptr)
 int surfel_read_model(surfel_handle c, float* host_dst, int max_surfels, int* count)
 {
     if (!c || !host_dst || !count || max_surfels < 0) return ODOM_ERR_ARG;
+    if (int rc = settle(c)) return rc;
     const int n = c->count < max_surfels ? c->count : max_surfels;
     if (n > 0)
         SCHK(hipMemcpyAsync(host_dst, c->model[c->cur], (size_t)n * 48, hipMemcpyDeviceToHost, c->stream));
@@ -1296,6 +1314,7 @@ int surfel_set_model(surfel_handle c, const float* model, int n, int mem)
 {
     if (!c || n < 0 || n > c->max_surfels || (n > 0 && !model)) return ODOM_ERR_ARG;
     if (mem != ODOM_MEM_HOST && mem != ODOM_MEM_DEVICE) return ODOM_ERR_ARG;
+    if (int rc = settle(c)) return rc;
     if (n > 0)
         SCHK(hipMemcpyAsync(c->model[c->cur], model, (size_t)n * 48,
                             mem == ODOM_MEM_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice, c->stream));
@@ -1333,7 +1352,8 @@ int surfel_read_fresh(surfel_handle c, float* host_dst, int max_points, int* cou
 {
     if (!c || !host_dst || !count || max_points < 0) return ODOM_ERR_ARG;
     int n = 0;
-    const int rc = read_count(c, c->totals + 1, &n);
+    int rc = settle(c);   // both counts land in the same buffer
+    if (!rc) rc = read_count(c, c->totals + 1, &n);
     if (rc) return rc;
     const int m = n < max_points ? n : max_points;
     if (m > 0) SCHK(hipMemcpyAsync(host_dst, c->fresh, (size_t)m * 48, hipMemcpyDeviceToHost, c->stream));
@@ -1347,8 +1367,10 @@ int surfel_profile(surfel_handle c, const float pose[16], int time, const odom_f
                    float max_depth, float weighting, float conf_threshold, int time_delta, int reps, float us[4])
 {
     if (!c || !pose || !us || reps < 1) return ODOM_ERR_ARG;
+    int rc = settle(c);
+    if (rc) return rc;
     RGBView rv;
-    int rc = frames(c, rgb, raw_depth, filtered_depth, depth_cutoff, &rv);
+    rc = frames(c, rgb, raw_depth, filtered_depth, depth_cutoff, &rv);
     if (rc) return rc;
     // keep the starting model: every rep fuses the same frame into it
     const int n0 = c->count, cur0 = c->cur;
@@ -1393,3 +1415,25 @@ int surfel_profile(surfel_handle c, const float pose[16], int time, const odom_f
 }
 
 }  // extern "C"
+
+namespace slam {
+
+int surfel_clean_enqueue(surfel_handle c, const float pose[16], int time, float conf_threshold, int time_delta)
+{
+    if (int rc = settle(c)) return rc;
+    enqueue_clean(c, pose, time, conf_threshold, time_delta);
+    SCHK(hipGetLastError());
+    c->cur ^= 1;
+    c->count = std::min(c->max_surfels, c->count + max_fresh(c));
+    c->pending = true;
+    return ODOM_OK;
+}
+
+void surfel_model_enqueued(surfel_handle c, const float** dev_ptr, int* upper, const int** dev_count)
+{
+    *dev_ptr = c->model[c->cur];
+    *upper = c->count;
+    *dev_count = c->pending ? c->totals : nullptr;
+}
+
+}  // namespace slam
