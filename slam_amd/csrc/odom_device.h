@@ -36,6 +36,7 @@ struct LevelDesc {
     const float* zsrc;               // next depth, NaN where the photometric
                                      // source pixel is statically invalid
     const short2* dxy;               // next image derivatives (dx, dy)
+    const float* znext;              // next depth (zsrc and dxy are formed from it and inext)
     const uint8_t* inext;            // next intensity
     const float* zlast;              // model (last) depth
     const uint8_t* ilast;            // model (last) intensity

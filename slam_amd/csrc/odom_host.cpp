@@ -188,7 +188,7 @@ int upload_pair(odom_ctx* c)
             L.invFx = 1.0f / c->fx[l];
             L.invFy = 1.0f / c->fy[l];
             L.vcur = c->vcur[l]; L.ncur = c->ncur[l]; L.vprev = c->vprev[l]; L.nprev = c->nprev[l];
-            L.zsrc = c->zsrc[l]; L.dxy = c->dxy[l]; L.inext = c->img[q][l];
+            L.zsrc = c->zsrc[l]; L.dxy = c->dxy[l]; L.inext = c->img[q][l]; L.znext = c->nextDepth[l];
             L.zlast = c->lastDepth[l]; L.ilast = c->lastImage[l];
             const float sobelScale = (float)(1.0 / pow(2.0, 3));
             const double minGrad[kLevels] = {5, 3, 1};
@@ -251,9 +251,12 @@ int resolve(odom_ctx* c, const odom_frame_view* v, int fmt_a, int fmt_b, void* s
     return ODOM_OK;
 }
 
-int enqueue_depth_pyramid_maps(odom_ctx* c, float cutoff)
+// src, pitch (elements): level 0, which depth[0] becomes.
+int enqueue_depth_pyramid_maps(odom_ctx* c, const uint16_t* src, int pitch, float cutoff)
 {
     VNLevels a{};
+    a.src = src;
+    a.src_pitch = pitch;
     for (int l = 0; l < kLevels; ++l) {
         a.depth[l] = c->depth[l];
         a.vmap[l] = c->vcur[l];
@@ -305,7 +308,9 @@ int enqueue_model(odom_ctx* c, const odom_frame_view* v, const odom_frame_view* 
 }
 
 // populateRGBDData, RGBDOdometryef.cpp:208-235 (maxDepthRGB 6.0, :37)
-int enqueue_populate(odom_ctx* c, const odom_frame_view* rgb, float** dstDepth, uint8_t** dstImage)
+// first: a sequence starts with this image.
+int enqueue_populate(odom_ctx* c, const odom_frame_view* rgb, float** dstDepth, uint8_t** dstImage,
+                     bool first = false)
 {
     const void* p;
     int pitch, fmt;
@@ -314,6 +319,7 @@ int enqueue_populate(odom_ctx* c, const odom_frame_view* rgb, float** dstDepth, 
     PyrJob py{};
     py.w0 = c->w[0];
     py.h0 = c->h[0];
+    py.fresh = first ? c->st : nullptr;
     if (dstDepth) {
         PyrSrc& q = py.p[py.count++];
         q.vz = c->vz;
@@ -650,9 +656,7 @@ int odom_init_icp_depth(odom_handle c, const odom_frame_view* depth, float cutof
     int pitch, fmt;
     int rc = resolve(c, depth, ODOM_FMT_DEPTH_U16, ODOM_FMT_DEPTH_U16, c->stage_u16, &p, &pitch, &fmt);
     if (rc) return rc;
-    HIPCHK(c, hipMemcpy2DAsync(c->depth[0], (size_t)c->w[0] * 2, p, pitch, (size_t)c->w[0] * 2, c->h[0],
-                               hipMemcpyDeviceToDevice, c->stream));
-    rc = enqueue_depth_pyramid_maps(c, cutoff);
+    rc = enqueue_depth_pyramid_maps(c, (const uint16_t*)p, pitch / 2, cutoff);
     if (rc == ODOM_OK) c->icp_cur = true;
     return rc;
 }
@@ -665,7 +669,7 @@ int odom_init_icp_raw_depth(odom_handle c, const odom_frame_view* raw, float max
     int rc = resolve(c, raw, ODOM_FMT_DEPTH_U16, ODOM_FMT_DEPTH_U16, c->stage_u16, &p, &pitch, &fmt);
     if (rc) return rc;
     launch_bilateral((const uint16_t*)p, pitch / 2, c->depth[0], c->w[0], c->h[0], maxD, c->stream);
-    rc = enqueue_depth_pyramid_maps(c, cutoff);
+    rc = enqueue_depth_pyramid_maps(c, c->depth[0], c->w[0], cutoff);
     if (rc == ODOM_OK) c->icp_cur = true;
     return rc;
 }
@@ -721,13 +725,7 @@ int odom_init_first_rgb(odom_handle c, const odom_frame_view* rgb)
 {
     if (!c) return ODOM_ERR_ARG;
     uint8_t* dst[kLevels] = {last_next_img(c, 0), last_next_img(c, 1), last_next_img(c, 2)};
-    // a sequence starts: no motion yet to extrapolate
-    double eye[16];
-    for (int k = 0; k < 16; ++k) eye[k] = (k % 5 == 0) ? 1.0 : 0.0;
-    if (int rc = write_field(c, c->st->lastRt, eye, 16)) return rc;
-    const int zero = 0;
-    if (int rc = write_field(c, &c->st->so3_fail, &zero, 1)) return rc;
-    return enqueue_populate(c, rgb, nullptr, dst);
+    return enqueue_populate(c, rgb, nullptr, dst, true);
 }
 
 int odom_set_pose(odom_handle c, const float trans[3], const float rot[9])
@@ -738,7 +736,8 @@ int odom_set_pose(odom_handle c, const float trans[3], const float rot[9])
         for (int b = 0; b < 3; ++b) pose[a * 4 + b] = rot[a * 3 + b];
         pose[a * 4 + 3] = trans[a];
     }
-    return write_field(c, c->st->pose_out, pose, 12);
+    launch_set_pose(c->st, pose, c->stream);
+    return check_launch(c);
 }
 
 int odom_get_pose(odom_handle c, float trans[3], float rot[9])
@@ -1471,6 +1470,11 @@ void batch_launches(odom_batch_s* b, const CallSpec& cs, PairDesc* const* dp, hi
     int hyp = cs.hyp;
     PairDesc* cur = dp[hyp - 1];
     if (cs.policy_start) launch_seed_policy(cur, n * hyp, hyp, cs.pred, cs.t_scale, cs.r_scale, b->stream);
+    // the pairs' derivatives and source masks (once for both refinements)
+    int groups[kLevels] = {0, 0, 0};
+    for (const auto* c : b->h)
+        for (int l = 0; l < kLevels; ++l) groups[l] = std::max(groups[l], (c->w[l] + 3) / 4 * c->h[l]);
+    if (P.rgb) launch_rgb_prep_pairs(dp[0], n, groups, b->stream);
     if (P.so3) launch_so3(cur, n * hyp, &P, b->so3_spin, b->stream);  // begin rides on the SO3 loop's end
     else launch_track_begin(cur, n * hyp, P, b->stream);
     std::vector<int> sched;
@@ -1522,21 +1526,14 @@ void batch_launches(odom_batch_s* b, const CallSpec& cs, PairDesc* const* dp, hi
         }                                                                                                \
     } while (0)
 
-// Everything before the batch's own launches: checks, the per-pair
-// derivative pass on each handle's stream, the cross-stream waits, and the
-// descriptor arrays the call uses.
+// Everything before the batch's own launches: checks, the cross-stream waits
+// and the descriptor arrays the call uses.
 int batch_prepare(odom_batch_s* b, const CallSpec& cs, PairDesc** dp)
 {
     for (auto* c : b->h)
         if (!inputs_ready(c, cs.P)) return ODOM_ERR_STATE;
     for (size_t i = 0; i < b->h.size(); ++i) {
         odom_ctx* c = b->h[i];
-        if (cs.P.rgb) {
-            PrepLevels a{};
-            prep_levels(c, a);
-            launch_rgb_prep(a, c->stream);
-            if (int rc = check_launch(c)) return rc;
-        }
         if (b->own_stream) {
             BCHK(b, hipEventRecord(b->ready[i], c->stream));
             BCHK(b, hipStreamWaitEvent(b->stream, b->ready[i], 0));

@@ -45,15 +45,17 @@ void launch_bilateral(const uint16_t* src, int src_pitch, uint16_t* dst, int w, 
                       hipStream_t s);
 // depth pyramid -> vertex+normal maps of all levels in one launch
 struct VNLevels {
-    uint16_t* depth[kLevels];       // level 0 is read; launch_depth_pyramid_maps writes levels 1, 2
+    uint16_t* depth[kLevels];       // written by launch_depth_pyramid_maps (level 0 unless it is src)
+    const uint16_t* src;            // level 0
+    int src_pitch;                  // in elements
     float* vmap[kLevels];
     float* nmap[kLevels];
     int w[kLevels], h[kLevels];
     float fx_inv[kLevels], fy_inv[kLevels], cx[kLevels], cy[kLevels];
     float cutoff;
 };
-// initICP's depth levels 1 and 2 from a.depth[0] and the three levels'
-// vertex and normal maps, in one launch.
+// initICP's depth levels from a.src and the three levels' vertex and normal
+// maps, in one launch.
 void launch_depth_pyramid_maps(const VNLevels& a, hipStream_t s);
 // RGBA32F vertex/normal maps -> planar pyramids (copyMaps + resize, optional
 // rigid transform), plus the vertex z plane kept for verticesToDepth.
@@ -85,6 +87,7 @@ struct PyrJob {
     PyrSrc p[2];
     int count;
     int w0, h0;
+    TrackState* fresh;              // if set: a sequence starts (no motion yet, no SO3 failure)
 };
 void launch_pyramid(const PyrJob& j, hipStream_t s);
 // derivatives (a12) + static photometric source mask, all levels of all pairs
@@ -97,6 +100,11 @@ struct PrepLevels {
     float minScale[kLevels];
 };
 void launch_rgb_prep(const PrepLevels& a, hipStream_t s);
+// The same for every pair; max_groups: the most groups of four pixels of a row
+// that any pair has, per level.
+void launch_rgb_prep_pairs(const PairDesc* pairs, int npairs, const int max_groups[kLevels], hipStream_t s);
+// The pose (3x4 row-major) that the next call starts from.
+void launch_set_pose(TrackState* st, const float pose[12], hipStream_t s);
 
 // ---- tracking (a14-a21) ----
 struct StepLaunch {

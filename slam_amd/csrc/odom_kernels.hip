@@ -620,6 +620,10 @@ __device__ void pyr_tile(const PyrSrc& P, int w0, int h0, int tx, int ty, unsign
 __global__ __launch_bounds__(kPyrThreads) void k_pyramid(PyrGrid g)
 {
     __shared__ __align__(16) unsigned char smem[(TileDims<0, kPyrThreads>::N0 + TileDims<0, kPyrThreads>::N1) * 4];
+    if (g.j.fresh && blockIdx.x == 0) {
+        if (threadIdx.x < 16) g.j.fresh->lastRt[threadIdx.x] = (threadIdx.x % 5 == 0) ? 1.0 : 0.0;
+        if (threadIdx.x == 0) g.j.fresh->so3_fail = 0;
+    }
     const int q = (int)blockIdx.x / g.tiles, t = (int)blockIdx.x - q * g.tiles;
     const int ty = t / g.tiles_x, tx = t - ty * g.tiles_x;
     const PyrSrc& P = g.j.p[q];
@@ -643,7 +647,7 @@ void launch_pyramid(const PyrJob& j, hipStream_t s)
 // margin of one output (in LDS only; the neighbouring tile stores those), and
 // the staged level-0 texels and level-1 values hold the others' margins.
 struct DepthMapsGrid {
-    VNLevels a;                   // a.depth[0] is the input; a.depth[1], a.depth[2] are written
+    VNLevels a;
     int tiles_x;
 };
 
@@ -662,7 +666,7 @@ __global__ __launch_bounds__(kMapsThreads) void k_depth_pyramid_maps(DepthMapsGr
     for (int r = 0; r < D::R0; ++r) {
         const int i = min(tid + r * kMapsThreads, D::N0 - 1);
         const int x = min(max(c0x - 6 + i % D::X0, 0), w0 - 1), y = min(max(c0y - 6 + i / D::X0, 0), h0 - 1);
-        raw[r] = gp((const uint16_t*)a.depth[0])[(size_t)y * w0 + x];
+        raw[r] = gp(a.src)[(size_t)y * a.src_pitch + x];
     }
 #pragma unroll
     for (int r = 0; r < D::R0; ++r) {
@@ -688,8 +692,11 @@ __global__ __launch_bounds__(kMapsThreads) void k_depth_pyramid_maps(DepthMapsGr
     for (int r = 0; r < 16 * kTile2X * kTile2Y / kMapsThreads; ++r) {
         const int i = tid + r * kMapsThreads;
         const int x = c0x + i % (4 * kTile2X), y = c0y + i / (4 * kTile2X);
-        if (x < w0 && y < h0)
+        if (x < w0 && y < h0) {
+            if (a.src != a.depth[0])
+                gp(a.depth[0])[(size_t)y * w0 + x] = (uint16_t)s0[(y - c0y + 6) * D::X0 + (x - c0x + 6)];
             vn_pixel(a, 0, x, y, [&](int u, int v) { return (uint16_t)s0[(v - c0y + 6) * D::X0 + (u - c0x + 6)]; });
+        }
     }
     __syncthreads();
     if (tid < D::R2X * D::R2Y) {
@@ -735,77 +742,166 @@ __constant__ float c_gsx[9] = {0.52201f, 0.00000f, -0.52201f, 0.79451f, -0.00000
 __constant__ float c_gsy[9] = {0.52201f, 0.79451f, 0.52201f, 0.00000f, 0.00000f, 0.00000f,
                                -0.52201f, -0.79451f, -0.52201f};
 
-// Pixel k of level l.
-__device__ __forceinline__ void rgb_prep_px(const PrepLevels& a, int l, int k)
+// Pixels 4 g..4 g + 3 of a row, group k of one level.  The 16 texels of a
+// pixel's window hold the nine of its derivatives, and four pixels' windows
+// lie in 8 bytes of each of four rows: one load a row instead of 25 a pixel,
+// which bound the pass (64 pairs of
+// 320x240 to 848x480: 217 us by bytes, 134 so).
+__device__ __forceinline__ int prep_groups(int w) { return (w + 3) / 4; }
+
+// Bytes x..x+7 from the start of row y of an image of n bytes (row length w):
+// any x; bytes outside the image are 0.
+__device__ __forceinline__ uint64_t row8(const uint8_t* __restrict__ img, int n, int w, int y, int x)
 {
-    const int w = a.w[l], h = a.h[l];
-    if (k >= w * h) return;
-    const int y = k / w, x = k - y * w;
-    const uint8_t* img = a.img[l];
-    float dxv = 0.0f, dyv = 0.0f;
-    if (x >= 1 && x < w - 1 && y >= 1 && y < h - 1) {
-        // interior: the nine taps in the same order with fixed weights
-        const float kx[9] = {0.52201f, 0.00000f, -0.52201f, 0.79451f, -0.00000f, -0.79451f,
-                             0.52201f, 0.00000f, -0.52201f};
-        const float ky[9] = {0.52201f, 0.79451f, 0.52201f, 0.00000f, 0.00000f, 0.00000f,
-                             -0.52201f, -0.79451f, -0.52201f};
-        int ki = 8;
+    const int want = y * w + x, at = min(max(want, 0), n - 8);
+    uint64_t v;
+    __builtin_memcpy(&v, img + at, 8);
+    return want < at ? v << (8 * (at - want)) : v >> (8 * min(want - at, 7));
+}
+
+__device__ __forceinline__ void rgb_prep_group(const uint8_t* __restrict__ img, const float* __restrict__ depth,
+                                               short2* __restrict__ dxy, float* __restrict__ zsrc, int w, int h,
+                                               float min_scale, int k)
+{
+    const int per_row = prep_groups(w), y = k / per_row, x0 = 4 * (k - y * per_row);
+    if (y >= h) return;
+    // rows y-2..y+1 from column x0-2; a row above the image is not tested, one
+    // below it not reached
+    uint64_t r[4];
 #pragma unroll
-        for (int j = -1; j <= 1; j++)
-#pragma unroll
-            for (int i = -1; i <= 1; i++) {
-                const float sv = (float)img[(size_t)(y + j) * w + x + i];
-                dxv = dxv + sv * kx[ki];
-                dyv = dyv + sv * ky[ki];
-                --ki;
-            }
+    for (int j = 0; j < 4; ++j) r[j] = row8(img, w * h, w, min(max(y - 2 + j, 0), h - 1), x0 - 2);
+    const size_t o = (size_t)y * w + x0;
+    const bool wide = (w & 3) == 0;     // every row's groups are whole and 16-byte aligned
+    float d[4];
+    if (wide) {
+        const float4 v = *(const float4*)(depth + o);
+        d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
     } else {
-        int ki = 8;
-        for (int j = max(y - 1, 0); j <= min(y + 1, h - 1); j++)
-            for (int i = max(x - 1, 0); i <= min(x + 1, w - 1); i++) {
-                const float sv = (float)img[(size_t)j * w + i];
-                dxv = dxv + sv * c_gsx[ki];
-                dyv = dyv + sv * c_gsy[ki];
-                --ki;
-            }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[i] = depth[o + min(i, w - 1 - x0)];
     }
-    const short sx = (short)dxv, sy = (short)dyv;
-    a.dxy[l][k] = make_short2(sx, sy);
-    float z = QNAN;
-    if (x < w - 5 && y < h - 1) {
-        // rows y-2..y+1 and columns x-2..x+1 inside the image (the upper
-        // bounds hold here), all 16 loads issued before any test
-        bool valid = true;
+    short2 g[4];
+    float zs[4];
 #pragma unroll
-        for (int du = -2; du < 2; ++du)
+    for (int i = 0; i < 4; ++i) {
+        const int x = x0 + i;
+        const auto tap = [&](int j, int c) { return (int)((r[j] >> (8 * c)) & 0xFFu); };   // row y-2+j, column x0-2+c
+        float dxv = 0.0f, dyv = 0.0f;
+        if (x >= 1 && x < w - 1 && y >= 1 && y < h - 1) {
+            // interior: the taps in the loops' order with fixed weights (those of weight 0 leave the sums as they are)
+            const float kx[9] = {0.52201f, 0.00000f, -0.52201f, 0.79451f, -0.00000f, -0.79451f,
+                                 0.52201f, 0.00000f, -0.52201f};
+            const float ky[9] = {0.52201f, 0.79451f, 0.52201f, 0.00000f, 0.00000f, 0.00000f,
+                                 -0.52201f, -0.79451f, -0.52201f};
+            int ki = 8;
 #pragma unroll
-            for (int dv = -2; dv < 2; ++dv) {
-                const uint8_t t = img[(size_t)max(y + du, 0) * w + max(x + dv, 0)];
-                valid = valid & ((y + du < 0) | (x + dv < 0) | (t > 0));
-            }
-        if (valid) {
+            for (int j = -1; j <= 1; j++)
+#pragma unroll
+                for (int c = -1; c <= 1; c++) {
+                    const float sv = (float)tap(j + 2, i + 2 + c);
+                    if (kx[ki] != 0.0f) dxv = dxv + sv * kx[ki];
+                    if (ky[ki] != 0.0f) dyv = dyv + sv * ky[ki];
+                    --ki;
+                }
+        } else if (x < w) {
+            int ki = 8;
+            for (int j = max(y - 1, 0); j <= min(y + 1, h - 1); j++)
+                for (int c = max(x - 1, 0); c <= min(x + 1, w - 1); c++) {
+                    const float sv = (float)img[(size_t)j * w + c];
+                    dxv = dxv + sv * c_gsx[ki];
+                    dyv = dyv + sv * c_gsy[ki];
+                    --ki;
+                }
+        }
+        const short sx = (short)dxv, sy = (short)dyv;
+        g[i] = make_short2(sx, sy);
+        zs[i] = QNAN;
+        if (x < w - 5 && y < h - 1) {
+            // rows y-2..y+1 and columns x-2..x+1 inside the image (the upper bounds hold here)
+            bool valid = true;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    valid = valid & ((y - 2 + j < 0) | (x - 2 + c < 0) | (tap(j, i + c) > 0));
             const float mTwo = (float)((int)sx * (int)sx + (int)sy * (int)sy);
-            if (mTwo >= a.minScale[l]) {
-                const float d1 = a.depth[l][k];
-                if (!isnan(d1)) z = d1;
-            }
+            if (valid && mTwo >= min_scale) zs[i] = d[i];    // a NaN depth stays NaN
         }
     }
-    a.zsrc[l][k] = z;
+    if (wide) {
+        int4 q;
+        __builtin_memcpy(&q, g, 16);
+        *(int4*)(dxy + o) = q;
+        *(float4*)(zsrc + o) = make_float4(zs[0], zs[1], zs[2], zs[3]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (x0 + i < w) {
+                dxy[o + i] = g[i];
+                zsrc[o + i] = zs[i];
+            }
+    }
+}
+
+__device__ __forceinline__ void rgb_prep_group(const PrepLevels& a, int l, int k)
+{
+    rgb_prep_group(a.img[l], a.depth[l], a.dxy[l], a.zsrc[l], a.w[l], a.h[l], a.minScale[l], k);
+}
+
+// Groups of every level, as segments of blocks of nt threads.
+Seg3 prep_seg(const int w[kLevels], const int h[kLevels], int nt)
+{
+    int n[kLevels];
+    for (int l = 0; l < kLevels; ++l) n[l] = (w[l] + 3) / 4 * h[l];
+    return make_seg(n, nt);
 }
 
 __global__ __launch_bounds__(256) void k_rgb_prep(PrepLevels a, Seg3 g)
 {
     const int l = seg_level(g, blockIdx.x);
-    rgb_prep_px(a, l, (blockIdx.x - g.b0[l]) * 256 + threadIdx.x);
+    rgb_prep_group(a, l, (blockIdx.x - g.b0[l]) * 256 + threadIdx.x);
 }
 
 void launch_rgb_prep(const PrepLevels& a, hipStream_t s)
 {
-    int n[kLevels];
-    for (int l = 0; l < kLevels; ++l) n[l] = a.w[l] * a.h[l];
-    const Seg3 g = make_seg(n, 256);
+    const Seg3 g = prep_seg(a.w, a.h, 256);
     hipLaunchKernelGGL(k_rgb_prep, dim3(g.b0[kLevels]), dim3(256), 0, s, a, g);
+}
+
+// One launch for all pairs of a batch (blockIdx.y): a 640x480 pair by itself
+// fills the card with 1 575 short workgroups for 7 us, mostly launch and
+// drain, and 64 of them took 64 launches (480 us of kernels; 134 us here).
+// A smaller pair's blocks past its own pixels return at once.
+__global__ __launch_bounds__(256) void k_rgb_prep_pairs(const PairDesc* __restrict__ pairs, Seg3 g)
+{
+    const int l = seg_level(g, blockIdx.x);
+    const LevelDesc& L = pairs[blockIdx.y].lv[l];
+    rgb_prep_group(L.inext, L.znext, const_cast<short2*>(L.dxy), const_cast<float*>(L.zsrc), L.w, L.h, L.minScale,
+                   (blockIdx.x - g.b0[l]) * 256 + threadIdx.x);
+}
+
+void launch_rgb_prep_pairs(const PairDesc* pairs, int npairs, const int max_groups[kLevels], hipStream_t s)
+{
+    const Seg3 g = make_seg(max_groups, 256);
+    hipLaunchKernelGGL(k_rgb_prep_pairs, dim3(g.b0[kLevels], npairs), dim3(256), 0, s, pairs, g);
+}
+
+// The pose as a kernel argument: a 48-byte copy from the caller's memory costs
+// the host three times a launch.
+struct Pose12 {
+    float v[12];
+};
+
+__global__ __launch_bounds__(64) void k_set_pose(TrackState* st, Pose12 p)
+{
+    if (threadIdx.x < 12) st->pose_out[threadIdx.x] = p.v[threadIdx.x];
+}
+
+void launch_set_pose(TrackState* st, const float pose[12], hipStream_t s)
+{
+    Pose12 p;
+    for (int k = 0; k < 12; ++k) p.v[k] = pose[k];
+    hipLaunchKernelGGL(k_set_pose, dim3(1), dim3(64), 0, s, st, p);
 }
 
 // ============================================================ reductions
@@ -2490,16 +2586,28 @@ struct So3Src {
     float g[2], v;
 };
 
+// The texel (x, y) and its four neighbours.
+struct So3Texels {
+    uint8_t c, l, r, u, d;
+};
+
 template <class Ptr>
-__device__ __forceinline__ void so3_grad(Ptr img, int w, int x, int y, float* g)
+__device__ __forceinline__ void so3_texels(Ptr img, int w, int x, int y, So3Texels& t)
 {
-    const float actu = (float)img[(size_t)y * w + x];
-    float back = (float)img[(size_t)y * w + x - 1];
-    float fore = (float)img[(size_t)y * w + x + 1];
-    g[0] = ((back + actu) / 2.0f) - ((fore + actu) / 2.0f);
-    back = (float)img[(size_t)(y - 1) * w + x];
-    fore = (float)img[(size_t)(y + 1) * w + x];
-    g[1] = ((back + actu) / 2.0f) - ((fore + actu) / 2.0f);
+    const size_t i = (size_t)y * w + x;
+    t.c = img[i];
+    t.l = img[i - 1];
+    t.r = img[i + 1];
+    t.u = img[i - w];
+    t.d = img[i + w];
+}
+
+__device__ __forceinline__ So3Src so3_half(const So3Texels& t)
+{
+    const float actu = (float)t.c;
+    return {{(((float)t.l + actu) / 2.0f) - (((float)t.r + actu) / 2.0f),
+             (((float)t.u + actu) / 2.0f) - (((float)t.d + actu) / 2.0f)},
+            actu};
 }
 
 __device__ __forceinline__ bool so3_interior(int w, int h, int x, int y)
@@ -2512,8 +2620,9 @@ __device__ __forceinline__ void so3_src(Ptr last, int w, int h, int x, int y, So
 {
     s.g[0] = s.g[1] = s.v = 0.0f;
     if (so3_interior(w, h, x, y)) {
-        so3_grad(last, w, x, y, s.g);
-        s.v = (float)last[(size_t)y * w + x];
+        So3Texels t;
+        so3_texels(last, w, x, y, t);
+        s = so3_half(t);
     }
 }
 
@@ -2529,15 +2638,13 @@ __device__ __forceinline__ bool so3_warp(const float* H, int w, int h, int x, in
     return wx >= 1 && wx < w - 1 && wy >= 1 && wy < h - 1 && so3_interior(w, h, x, y);
 }
 
-template <class Ptr>
-__device__ __forceinline__ void so3_row(Ptr next, int w, int wx, int wy, const So3Src& src, int x, int y,
-                                        const float* Ki, const float* KR, float* row)
+// nx: the next image's half at the warped pixel, src: the last image's.
+__device__ __forceinline__ void so3_row(const So3Src& nx, const So3Src& src, int x, int y, const float* Ki,
+                                        const float* KR, float* row)
 {
     const float xf = (float)x, yf = (float)y;
-    float gn[2];
-    so3_grad(next, w, wx, wy, gn);
-    const float gx = (gn[0] + src.g[0]) / 2.0f;
-    const float gy = (gn[1] + src.g[1]) / 2.0f;
+    const float gx = (nx.g[0] + src.g[0]) / 2.0f;
+    const float gy = (nx.g[1] + src.g[1]) / 2.0f;
     const float pt0 = Ki[0] * xf + Ki[1] * yf + Ki[2] * 1.0f;
     const float pt1 = Ki[3] * xf + Ki[4] * yf + Ki[5] * 1.0f;
     const float pt2 = Ki[6] * xf + Ki[7] * yf + Ki[8] * 1.0f;
@@ -2549,7 +2656,7 @@ __device__ __forceinline__ void so3_row(Ptr next, int w, int wx, int wy, const S
     row[0] = lp1 * pt2 - lp2 * pt1;
     row[1] = lp2 * pt0 - lp0 * pt2;
     row[2] = lp0 * pt1 - lp1 * pt0;
-    row[3] = -((float)next[(size_t)wy * w + wx] - src.v);
+    row[3] = -(nx.v - src.v);
 }
 
 // One pixel in full (the parity-check kernel).
@@ -2561,7 +2668,9 @@ __device__ __forceinline__ bool so3_pixel(Ptr last, Ptr next, int w, int h, int 
     if (!so3_warp(H, w, h, x, y, wx, wy)) return false;
     So3Src src;
     so3_src(last, w, h, x, y, src);
-    so3_row(next, w, wx, wy, src, x, y, Ki, KR, row);
+    So3Texels t;
+    so3_texels(next, w, wx, wy, t);
+    so3_row(so3_half(t), src, x, y, Ki, KR, row);
     return true;
 }
 
@@ -2639,6 +2748,57 @@ __device__ void so3_evaluate(So3Slot& S, const double* tot)
         S.R_lr[k] = nR[k];
         S.resultR[k] = (double)nR[k];
     }
+}
+
+// `CH` pixels of a thread, `stride` apart from idx, into acc in pixel order:
+// every texel load is issued before the first row (a branch around each
+// pixel's loads would wait for them one pixel after another), at a valid
+// texel where the pixel is skipped.  SRC: the pixels' halves are in src.
+// Launches of 64 pairs: 25.3 -> 23.5 us.  The one-launch loop does not move
+// (27 us at 640x480, 3 iterations; 155 at 1920x1080, 8 iterations): there the
+// rows' arithmetic on 16 CUs and the serial evaluation are the time, and more
+// workgroups would reorder the fp32 sums, on which the loop's exact tests
+// (equal counts, a smaller error) turn.
+template <int CH, bool SRC, class Ptr>
+__device__ __forceinline__ void so3_chunk(Ptr last, Ptr next, int w, int h, int n, int idx, int stride,
+                                          const So3Src* src, const float* H, const float* Ki, const float* KR,
+                                          float (&acc)[kSO3])
+{
+    int x[CH], y[CH];
+    bool ok[CH];
+    So3Texels tn[CH], tl[CH];
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+        const int i = idx + q * stride;
+        int wx, wy;
+        y[q] = i / w;
+        x[q] = i - y[q] * w;
+        ok[q] = so3_warp(H, w, h, x[q], y[q], wx, wy) && i < n;
+        so3_texels(next, w, ok[q] ? wx : 1, ok[q] ? wy : 1, tn[q]);
+        if (!SRC) so3_texels(last, w, ok[q] ? x[q] : 1, ok[q] ? y[q] : 1, tl[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+        if (!ok[q]) continue;
+        So3Src sv;
+        if constexpr (SRC) sv = src[q];
+        else sv = so3_half(tl[q]);
+        float row[4];
+        so3_row(so3_half(tn[q]), sv, x[q], y[q], Ki, KR, row);
+        acc_row4(acc, row);
+    }
+}
+
+// A thread's pixels of an iteration: those whose halves are in src, then the
+// rest (1920x1080: 13 more), four at a time.
+template <class Ptr>
+__device__ __forceinline__ void so3_rows(Ptr last, Ptr next, int w, int h, int n, int first, int stride,
+                                         const So3Src (&src)[kSO3Pre], const float* H, const float* Ki,
+                                         const float* KR, float (&acc)[kSO3])
+{
+    so3_chunk<kSO3Pre, true>(last, next, w, h, n, first, stride, src, H, Ki, KR, acc);
+    for (int i = first + kSO3Pre * stride; i < n; i += 4 * stride)
+        so3_chunk<4, false>(last, next, w, h, n, i, stride, src, H, Ki, KR, acc);
 }
 
 // With `begin`, block 0 of each pair of launch 10 also sets up the
@@ -2751,30 +2911,7 @@ __global__ __launch_bounds__(kSO3Threads) void k_so3_iter(const PairDesc* __rest
     float acc[kSO3];
 #pragma unroll
     for (int k = 0; k < kSO3; ++k) acc[k] = 0.0f;
-    // the preloaded pixels: all warps, then all next-image loads, then the
-    // rows in pixel order
-    int wx[kSO3Pre], wy[kSO3Pre];
-    bool ok[kSO3Pre];
-#pragma unroll
-    for (int j = 0; j < kSO3Pre; ++j) {
-        const int idx = first + j * stride;
-        const int y = idx / w, x = idx - y * w;
-        ok[j] = idx < n && so3_warp(Hr, w, h, x, y, wx[j], wy[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < kSO3Pre; ++j)
-        if (ok[j]) {
-            const int idx = first + j * stride;
-            const int y = idx / w, x = idx - y * w;
-            float row[4];
-            so3_row(next, w, wx[j], wy[j], src[j], x, y, Kir, KRr, row);
-            acc_row4(acc, row);
-        }
-    for (int idx = first + kSO3Pre * stride; idx < n; idx += stride) {
-        const int y = idx / w, x = idx - y * w;
-        float row[4];
-        if (so3_pixel(last, next, w, h, x, y, Hr, Kir, KRr, row)) acc_row4(acc, row);
-    }
+    so3_rows(last, next, w, h, n, first, stride, src, Hr, Kir, KRr, acc);
     block_partial<kSO3, kSO3Threads>(acc, D.part_a[it & 1] + (size_t)lb * kPartStride, s_red);
 }
 
@@ -2799,7 +2936,7 @@ __global__ __launch_bounds__(kSO3Threads) void k_so3_loop(const PairDesc* __rest
 {
     if ((int)blockIdx.x >= nloop) {
         const int b = (int)blockIdx.x - nloop, l = seg_level(pseg, b);
-        rgb_prep_px(prep, l, (b - pseg.b0[l]) * kSO3Threads + threadIdx.x);
+        rgb_prep_group(prep, l, (b - pseg.b0[l]) * kSO3Threads + threadIdx.x);
         return;
     }
     __shared__ So3Slot S;
@@ -2861,28 +2998,7 @@ __global__ __launch_bounds__(kSO3Threads) void k_so3_loop(const PairDesc* __rest
         float acc[kSO3];
 #pragma unroll
         for (int k = 0; k < kSO3; ++k) acc[k] = 0.0f;
-        int wx[kSO3Pre], wy[kSO3Pre];
-        bool ok[kSO3Pre];
-#pragma unroll
-        for (int j = 0; j < kSO3Pre; ++j) {
-            const int idx = first + j * stride;
-            const int y = idx / w, x = idx - y * w;
-            ok[j] = idx < n && so3_warp(Hr, w, h, x, y, wx[j], wy[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < kSO3Pre; ++j)
-            if (ok[j]) {
-                const int idx = first + j * stride;
-                const int y = idx / w, x = idx - y * w;
-                float row[4];
-                so3_row(next, w, wx[j], wy[j], src[j], x, y, Kir, KRr, row);
-                acc_row4(acc, row);
-            }
-        for (int idx = first + kSO3Pre * stride; idx < n; idx += stride) {
-            const int y = idx / w, x = idx - y * w;
-            float row[4];
-            if (so3_pixel(last, next, w, h, x, y, Hr, Kir, KRr, row)) acc_row4(acc, row);
-        }
+        so3_rows(last, next, w, h, n, first, stride, src, Hr, Kir, KRr, acc);
         const float* part = D.part_a[it & 1];
         block_partial<kSO3, kSO3Threads>(acc, (float*)part + (size_t)lb * kPartStride, s_red);
         // grid barrier of the pair's workgroups
@@ -2950,9 +3066,7 @@ void launch_so3(const PairDesc* pairs, int npairs, const TrackParams* begin, int
         Seg3 g{};
         if (prep) {
             a = *prep;
-            int n[kLevels];
-            for (int l = 0; l < kLevels; ++l) n[l] = a.w[l] * a.h[l];
-            g = make_seg(n, kSO3Threads);
+            g = prep_seg(a.w, a.h, kSO3Threads);
         }
         hipLaunchKernelGGL(k_so3_loop, dim3(nloop + (prep ? g.b0[kLevels] : 0)), dim3(kSO3Threads), 0, s, pairs,
                            begin ? 1 : 0, P, spin_limit, nloop, a, g);
