@@ -974,6 +974,9 @@ constexpr int kActPad = 4;
 constexpr int kInferBufA = 30 * 40 * (32 + kActPad);   // elements: the largest output (layer 1)
 constexpr int kInferBufB = 15 * 20 * (64 + kActPad);   // layer 2's output; also holds the input
 constexpr int kInferIn = 60 * 80 * 4;                  // the input sample
+// One LDS array holds both buffers and four zeros, which a tap outside the
+// image reads.
+constexpr int kInferZero = kInferBufA + kInferBufB;
 static_assert(kInferIn <= kInferBufB, "the input fits its buffer");
 
 struct InferParams {
@@ -1017,24 +1020,29 @@ __global__ __launch_bounds__(256) void k_pack_infer(PackArgs A)
 constexpr int kGroup = 24;
 
 // The k steps [k0, k1) of one work item (column tile nt, row tiles from
-// ch * CH) into acc.
+// ch * CH) into acc.  S: the LDS of the kernel, X its input's offset.  A step
+// lies in one tap (with 4 input channels: four of a lane's group each), so a
+// fragment's address is the row's base plus an offset that is the same in the
+// whole wave, and whether the tap lies in the image is a bit of the row's
+// mask; a tap outside reads zeros.  With the tap and the bounds formed per
+// lane and step the launch took 37.6 us, so 31.0 (the same bits).
 template <int CIN, int COUT, int HI, int WI, int HO, int WO, int XS, int CH, int GR, int k0, int k1>
-__device__ __forceinline__ void infer_conv_item(const bf16* __restrict__ X, const bf16* __restrict__ W, int nt,
+__device__ __forceinline__ void infer_conv_item(const bf16* __restrict__ S, int X, const bf16* __restrict__ W, int nt,
                                                 int ch, v4f (&acc)[CH])
 {
     constexpr int M = HO * WO, MT = (M + 15) / 16, NT = COUT / 16;
-    constexpr int KREAL = 9 * CIN;
     const int lane = threadIdx.x & 63;
-    const int rq = 4 * (lane >> 4);           // this lane's k offset within a 16-deep step
+    const int grp = lane >> 4;                // this lane's k offset within a 16-deep step: 4 grp
     // the rows of this lane's A fragments (one per row tile of the chunk)
-    int hob[CH], wob[CH];
-    bool mok[CH];
+    int base[CH], taps[CH];
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
         const int m = (ch * CH + i) * 16 + (lane & 15);
-        mok[i] = (ch * CH + i) < MT && m < M;
-        hob[i] = 2 * (m / WO) - 1;
-        wob[i] = 2 * (m % WO) - 1;
+        const int h = 2 * (m / WO) - 1, w = 2 * (m % WO) - 1;
+        base[i] = X + (h * WI + w) * XS + (CIN == 4 ? 0 : 4 * grp);
+        const int cols = (w >= 0 ? 1 : 0) | (w + 1 < WI ? 2 : 0) | (w + 2 < WI ? 4 : 0);
+        taps[i] = (h >= 0 ? cols : 0) | (h + 1 < HI ? cols << 3 : 0) | (h + 2 < HI ? cols << 6 : 0);
+        if ((ch * CH + i) >= MT || m >= M) taps[i] = 0;
     }
 #pragma unroll
     for (int i = 0; i < CH; ++i) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -1048,15 +1056,19 @@ __device__ __forceinline__ void infer_conv_item(const bf16* __restrict__ X, cons
 #pragma unroll
         for (int g = 0; g < GR; ++g) {
             if (g0 + g >= k1) break;
-            const int kq = (g0 + g) * 16 + rq;
-            const int c = kq % CIN, tap = kq / CIN;
-            const int kh = tap / 3, kw = tap - 3 * kh;
+            int tap, c;
+            if constexpr (CIN == 4) {
+                tap = 4 * (g0 + g) + grp;
+                c = 0;
+            } else {
+                static_assert(CIN % 16 == 0, "a step lies in one tap");
+                tap = (g0 + g) / (CIN / 16);
+                c = ((g0 + g) % (CIN / 16)) * 16;
+            }
+            const int kh = tap / 3, off = (kh * WI + tap - 3 * kh) * XS + c;
 #pragma unroll
             for (int i = 0; i < CH; ++i) {
-                v4s a = v4s{0, 0, 0, 0};
-                const int hi = hob[i] + kh, wi = wob[i] + kw;
-                if (mok[i] && kq < KREAL && hi >= 0 && hi < HI && wi >= 0 && wi < WI)
-                    a = *(const v4s*)&X[(hi * WI + wi) * XS + c];
+                const v4s a = *(const v4s*)&S[(taps[i] >> tap) & 1 ? base[i] + off : kInferZero];
                 acc[i] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[g], acc[i], 0, 0, 0);
             }
         }
@@ -1085,23 +1097,26 @@ __device__ __forceinline__ void infer_conv_store(bf16* __restrict__ Y, const flo
         }
 }
 
-// XS, YS: the pixel strides (elements) of X and Y.  CH: row tiles per work
+// XS, YS: the pixel strides (elements) of X and Y.  ROWS: row tiles per work
 // item (fewer when the layer has fewer, so no MFMA runs on an all-padding
-// tile).  Layers with at most half as many work items as waves (the deep,
+// tile), such that the items come out even over the 16 waves: 75 x 2 tiles in
+// 30 items of 5, 19 x 4 in 16 of 5, 5 x 6 in 12 of 3 (31.0 -> 29.0 us against
+// items of 4).  Layers with at most half as many work items as waves (the deep,
 // small ones) split each item's k steps in two halves on two waves; the
 // second half's sums go through LDS past the layer's output in Y (at
 // kKPartOff elements; Y is larger than the small outputs that split) and are
 // added to the first half's, in that order.
 constexpr int kKPartOff = 4096;
 
-template <int CIN, int COUT, int HI, int WI, int HO, int WO, int XS, int YS>
-__device__ __forceinline__ void infer_conv(const bf16* __restrict__ X, bf16* __restrict__ Y, const bf16* __restrict__ W,
+template <int CIN, int COUT, int HI, int WI, int HO, int WO, int XS, int YS, int ROWS>
+__device__ __forceinline__ void infer_conv(bf16* __restrict__ S, int X, int yoff, const bf16* __restrict__ W,
                                            const float* __restrict__ bias)
 {
-    constexpr int M = HO * WO, MT = (M + 15) / 16, NT = COUT / 16, CH = MT < 4 ? MT : 4;
+    constexpr int M = HO * WO, MT = (M + 15) / 16, NT = COUT / 16, CH = MT < ROWS ? MT : ROWS;
     constexpr int KREAL = 9 * CIN, KP = (KREAL + 31) / 32 * 32, KS = KP / 16;
     static_assert(COUT % 16 == 0 && CIN % 4 == 0 && KP % 16 == 0, "tile shapes");
-    const int wave = threadIdx.x >> 6;
+    bf16* Y = S + yoff;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int WAVES = kInferThreads / 64;
     constexpr int CHUNKS = (MT + CH - 1) / CH, ITEMS = NT * CHUNKS;
     constexpr bool SPLIT = 2 * ITEMS <= WAVES && KS >= 2 * kGroup;
@@ -1110,7 +1125,7 @@ __device__ __forceinline__ void infer_conv(const bf16* __restrict__ X, bf16* __r
         for (int item = wave; item < ITEMS; item += WAVES) {
             const int nt = item % NT, ch = item / NT;
             v4f acc[CH];
-            infer_conv_item<CIN, COUT, HI, WI, HO, WO, XS, CH, GR, 0, KS>(X, W, nt, ch, acc);
+            infer_conv_item<CIN, COUT, HI, WI, HO, WO, XS, CH, GR, 0, KS>(S, X, W, nt, ch, acc);
             infer_conv_store<COUT, HO, WO, YS, CH>(Y, bias, nt, ch, acc);
         }
     } else {
@@ -1128,9 +1143,9 @@ __device__ __forceinline__ void infer_conv(const bf16* __restrict__ X, bf16* __r
 #pragma unroll
             for (int i = 0; i < CH; ++i) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
         } else if (half == 0) {
-            infer_conv_item<CIN, COUT, HI, WI, HO, WO, XS, CH, GR, 0, KH>(X, W, nt, ch, acc);
+            infer_conv_item<CIN, COUT, HI, WI, HO, WO, XS, CH, GR, 0, KH>(S, X, W, nt, ch, acc);
         } else {
-            infer_conv_item<CIN, COUT, HI, WI, HO, WO, XS, CH, GR, KH, KS>(X, W, nt, ch, acc);
+            infer_conv_item<CIN, COUT, HI, WI, HO, WO, XS, CH, GR, KH, KS>(S, X, W, nt, ch, acc);
         }
         float* kp = (float*)(Y + kKPartOff) + ((size_t)item * CH * 64 + lane) * 4;
         if (live && half == 1)
@@ -1152,8 +1167,10 @@ __device__ __forceinline__ void infer_conv(const bf16* __restrict__ X, bf16* __r
 __global__ __launch_bounds__(kInferThreads) void k_cnn_infer(const bf16* __restrict__ x, InferParams P,
                                                              float* __restrict__ out, float* __restrict__ gap_out)
 {
-    __shared__ __align__(16) bf16 bufA[kInferBufA];
-    __shared__ __align__(16) bf16 bufB[kInferBufB];
+    __shared__ __align__(16) bf16 S[kInferZero + 4];
+    constexpr int A = 0, B = kInferBufA;
+    static_assert(kInferBufA % 8 == 0 && kInferZero % 4 == 0, "16-byte rows, 8-byte fragments");
+    bf16* bufB = S + B;
     __shared__ float s_h1[kFc1Out];
     __shared__ float s_gap[kFc1In];
     __shared__ float s_fc2[kInferThreads / 64][kOut];
@@ -1161,19 +1178,20 @@ __global__ __launch_bounds__(kInferThreads) void k_cnn_infer(const bf16* __restr
     // the input, 16 bytes per thread and step
     const uint4* src = (const uint4*)(x + (size_t)blockIdx.x * kInferIn);
     for (int i = t; i < kInferIn / 8; i += kInferThreads) ((uint4*)bufB)[i] = src[i];
+    if (t < 4) S[kInferZero + t] = 0;
     __syncthreads();
     constexpr int P4 = 4 + 0, P32 = 32 + kActPad, P64 = 64 + kActPad, P96 = 96 + kActPad, P128 = 128 + kActPad;
-    infer_conv<4, 32, 60, 80, 30, 40, P4, P32>(bufB, bufA, P.W[0], P.b[0]);
+    infer_conv<4, 32, 60, 80, 30, 40, P4, P32, 5>(S, B, A, P.W[0], P.b[0]);
     __syncthreads();
-    infer_conv<32, 64, 30, 40, 15, 20, P32, P64>(bufA, bufB, P.W[1], P.b[1]);
+    infer_conv<32, 64, 30, 40, 15, 20, P32, P64, 5>(S, A, B, P.W[1], P.b[1]);
     __syncthreads();
-    infer_conv<64, 96, 15, 20, 8, 10, P64, P96>(bufB, bufA, P.W[2], P.b[2]);
+    infer_conv<64, 96, 15, 20, 8, 10, P64, P96, 3>(S, B, A, P.W[2], P.b[2]);
     __syncthreads();
-    infer_conv<96, 128, 8, 10, 4, 5, P96, P128>(bufA, bufB, P.W[3], P.b[3]);
+    infer_conv<96, 128, 8, 10, 4, 5, P96, P128, 2>(S, A, B, P.W[3], P.b[3]);
     __syncthreads();
-    infer_conv<128, 128, 4, 5, 2, 3, P128, P128>(bufB, bufA, P.W[4], P.b[4]);
+    infer_conv<128, 128, 4, 5, 2, 3, P128, P128, 1>(S, B, A, P.W[4], P.b[4]);
     __syncthreads();
-    infer_conv<128, 128, 2, 3, 1, 2, P128, P128>(bufA, bufB, P.W[5], P.b[5]);
+    infer_conv<128, 128, 2, 3, 1, 2, P128, P128, 1>(S, A, B, P.W[5], P.b[5]);
     __syncthreads();
     // global average pooling over the 1 x 2 output (k_gap_fwd's arithmetic)
     if (t < kFc1In) {
