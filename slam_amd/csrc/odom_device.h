@@ -135,6 +135,7 @@ struct TrackState {
 // Uniform options of one track call.
 struct TrackParams {
     int icp, rgb, rgbOnly, so3;
+    int zcur;                        // every pair's current maps are a depth image's
     float icpWeight;
     float distThres, angleThres;
     float sobelScale;

@@ -137,6 +137,7 @@ struct odom_ctx {
     // call-order bookkeeping: which inputs have been provided at least once.
     // vtmp: the model vertex buffer that initRGB/initRGBModel read
     // (vmaps_tmp, RGBDOdometryef.cpp:208-235) has been filled.
+    bool from_depth = false;         // the current maps come from a depth image, not from given maps
     bool icp_cur = false, icp_model = false, rgb_next = false, rgb_last = false, vtmp = false;
     // captured tracking calls (odom_set_graph)
     bool use_graph = false;
@@ -342,6 +343,7 @@ TrackParams make_params(odom_ctx* c, int rgbOnly, float icpWeight, int pyramid, 
     P.rgb = (rgbOnly || icpWeight < 100) ? 1 : 0;
     P.rgbOnly = rgbOnly ? 1 : 0;
     P.so3 = so3 ? 1 : 0;
+    P.zcur = c->from_depth ? 1 : 0;
     P.icpWeight = icpWeight;
     P.distThres = c->prm.dist_thresh;
     P.angleThres = c->prm.angle_thresh;
@@ -424,7 +426,7 @@ std::vector<int> track_key(const odom_ctx* c, const TrackParams& P)
 {
     int w;
     memcpy(&w, &P.icpWeight, 4);
-    return {P.icp, P.rgb, P.rgbOnly, P.so3, P.seeded, P.iters[0], P.iters[1], P.iters[2], w, c->parity};
+    return {P.icp, P.rgb, P.rgbOnly, P.so3, P.zcur, P.seeded, P.iters[0], P.iters[1], P.iters[2], w, c->parity};
 }
 
 void drop_graphs(odom_ctx* c)
@@ -657,7 +659,7 @@ int odom_init_icp_depth(odom_handle c, const odom_frame_view* depth, float cutof
     int rc = resolve(c, depth, ODOM_FMT_DEPTH_U16, ODOM_FMT_DEPTH_U16, c->stage_u16, &p, &pitch, &fmt);
     if (rc) return rc;
     rc = enqueue_depth_pyramid_maps(c, (const uint16_t*)p, pitch / 2, cutoff);
-    if (rc == ODOM_OK) c->icp_cur = true;
+    if (rc == ODOM_OK) c->icp_cur = c->from_depth = true;
     return rc;
 }
 
@@ -670,7 +672,7 @@ int odom_init_icp_raw_depth(odom_handle c, const odom_frame_view* raw, float max
     if (rc) return rc;
     launch_bilateral((const uint16_t*)p, pitch / 2, c->depth[0], c->w[0], c->h[0], maxD, c->stream);
     rc = enqueue_depth_pyramid_maps(c, c->depth[0], c->w[0], cutoff);
-    if (rc == ODOM_OK) c->icp_cur = true;
+    if (rc == ODOM_OK) c->icp_cur = c->from_depth = true;
     return rc;
 }
 
@@ -678,6 +680,7 @@ int odom_init_icp_maps(odom_handle c, const odom_frame_view* v, const odom_frame
 {
     (void)cutoff;
     if (!c) return ODOM_ERR_ARG;
+    c->from_depth = false;
     const int rc = enqueue_model(c, v, n, nullptr, false);
     if (rc == ODOM_OK) c->icp_cur = c->vtmp = true;
     return rc;
@@ -1313,6 +1316,15 @@ struct CallSpec {
     float t_scale = 1.0f, r_scale = 1.0f;
 };
 
+// A batch's pass A reads z planes alone if every pair's maps are a depth
+// image's (TrackParams::zcur).
+int batch_from_depth(const odom_batch_s* b)
+{
+    for (const auto* c : b->h)
+        if (!c->from_depth) return 0;
+    return 1;
+}
+
 void batch_drop_graphs(odom_batch_s* b)
 {
     for (auto& g : b->graphs) (void)hipGraphExecDestroy(g.exec);
@@ -1571,7 +1583,7 @@ int bits(T v)
 std::vector<int> graph_key(const CallSpec& cs, const std::vector<int>& parities)
 {
     const TrackParams& P = cs.P;
-    std::vector<int> k = {P.icp, P.rgb, P.rgbOnly, P.so3, P.iters[0], P.iters[1], P.iters[2], bits(P.icpWeight),
+    std::vector<int> k = {P.icp, P.rgb, P.rgbOnly, P.so3, P.zcur, P.iters[0], P.iters[1], P.iters[2], bits(P.icpWeight),
                           P.seeded, bits(P.convT), bits(P.convR), bits(P.judgeTol), cs.hyp, cs.judge,
                           cs.policy_start ? 1 : 0, bits(cs.t_scale), bits(cs.r_scale)};
     uint64_t pp = (uint64_t)(uintptr_t)cs.pred;
@@ -1836,6 +1848,7 @@ int odom_track_batch(odom_batch b, int rgbOnly, float icpWeight, int pyramid, in
     if (!b) return ODOM_ERR_ARG;
     CallSpec cs;
     cs.P = make_params(b->h[0], rgbOnly, icpWeight, pyramid, fastOdom, so3);
+    cs.P.zcur = batch_from_depth(b);
     if (!cs.P.icp && !cs.P.rgb) return ODOM_ERR_ARG;  // RGBDOdometryef.cpp:558-561
     return batch_call(b, cs);
 }
@@ -1847,6 +1860,7 @@ int odom_track_batch_policy(odom_batch b, const float* pred, float t_scale, floa
     CallSpec cs;
     const int rc = policy_spec(b->h[0], pred, t_scale, r_scale, pol, rgbOnly, icpWeight, cs);
     if (rc) return rc;
+    cs.P.zcur = batch_from_depth(b);
     return batch_call(b, cs);
 }
 
@@ -1883,6 +1897,7 @@ int odom_batch_autotune(odom_batch b, int rgbOnly, float icpWeight)
 {
     if (!b) return ODOM_ERR_ARG;
     TrackParams P = make_params(b->h[0], rgbOnly, icpWeight, 1, 0, 0);
+    P.zcur = batch_from_depth(b);
     if (!P.icp && !P.rgb) return ODOM_ERR_ARG;
     for (auto* c : b->h)
         if (!inputs_ready(c, P)) return ODOM_ERR_STATE;
@@ -1961,6 +1976,7 @@ int odom_batch_profile_track(odom_batch b, int rgbOnly, float icpWeight, int pyr
     if (!b || !us_a || !us_b || !n_a || !n_b || !us_total) return ODOM_ERR_ARG;
     CallSpec cs;
     cs.P = make_params(b->h[0], rgbOnly, icpWeight, pyramid, fastOdom, so3);
+    cs.P.zcur = batch_from_depth(b);
     if (!cs.P.icp && !cs.P.rgb) return ODOM_ERR_ARG;
     PairDesc* dp[2];
     int rc = batch_prepare(b, cs, dp);
