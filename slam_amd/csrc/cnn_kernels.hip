@@ -51,26 +51,21 @@ inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 // one tap, loaded from the activations (or gradients) themselves, which the
 // caches hold.  The first operand of a product is the weights, so a lane's
 // four results are four consecutive channels of one position: an 8-byte bf16
-// store.  The passes up to the activations' gradients run 16-deep products in
-// ascending order of the reduction: a rounding that moves a bf16 activation
-// moves a ReLU's mask and, through Adam, whole weights, so the order of their
-// sums is part of what a training run reproduces.
+// store.  Every sum has one order, in 16-deep products ascending through parts
+// of a stated length: a rounding that moves a bf16 activation moves a ReLU's
+// mask and, through Adam, whole weights (other orders of any sum, the weight
+// gradients' too, moved the gradients four steps on by 1 to 8 % in some runs),
+// so the order of the sums is part of what a training run reproduces.
 //
 // Bound by latency and launches: a training step of 256 samples is 23 GFLOP
 // (10 us at the card's dense rate) and about 150 MB.  With im2col and col2im
 // buffers, 64x64 LDS-staged products, one-thread-per-column sums and 75
-// launches it took 2.1 ms, 0.9 ms of it in the sums over partial results.
-typedef __bf16 v8b __attribute__((ext_vector_type(8)));
-
+// launches it took 2.1 ms, 0.9 ms of it in the sums over partial results; now
+// 0.43 ms in 27 launches, with the same bits.
 __device__ __forceinline__ v4f mma16(uint2 a, uint2 b, v4f c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(v4s, a), __builtin_bit_cast(v4s, b), c, 0, 0,
                                                      0);
-}
-
-__device__ __forceinline__ v4f mma32(uint4 a, uint4 b, v4f c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8b, a), __builtin_bit_cast(v8b, b), c, 0, 0, 0);
 }
 
 __device__ __forceinline__ uint2 pack4(const float (&v)[4])
@@ -319,8 +314,8 @@ __global__ __launch_bounds__(256) void k_pack(PackJobs P)
 
 // Input gradient, through the ReLU of the layer below: dZl = (Yl > 0) ? dX : 0
 // with dX[h][w] = sum over the taps (kh, kw) with h = 2 ho - 1 + kh, w = 2 wo
-// - 1 + kw of dZ[ho][wo] W[tap]^T, and the sums of dZl over a workgroup's rows
-// (fp32, for the bias gradient) to part[workgroup][CIN].  Positions of one
+// - 1 + kw of dZ[ho][wo] W[tap]^T; dZl as bf16 for the products and as fp32
+// (dZf) for the bias gradient.  Positions of one
 // parity of (h, w) meet the same 1, 2, 2 or 4 taps, so each parity is a
 // product of its own (blockIdx.z, the longest first).  For the linear layer
 // above the average pooling (TAPS 1) both of a sample's two positions take
@@ -332,12 +327,11 @@ template <class L, int RT, int CT>
 __global__ __launch_bounds__(L::TAPS == 1 ? 64 : 256) void k_dgrad(const bf16* __restrict__ dZ,
                                                                    const bf16* __restrict__ Wp,
                                                                    const bf16* __restrict__ Yl, int N,
-                                                                   bf16* __restrict__ dZl, float* __restrict__ part)
+                                                                   bf16* __restrict__ dZl, float* __restrict__ dZf)
 {
     constexpr int WAVES = L::TAPS == 1 ? 1 : 4;
     constexpr int NT = L::CIN / 16, STEPS = L::COUT / 16, U = STEPS > 8 ? 24 : STEPS;
     static_assert(L::CIN % 16 == 0 && NT % CT == 0 && STEPS % U == 0, "whole tiles");
-    __shared__ float sums[WAVES][CT * 16];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row0 = ((int)blockIdx.x * WAVES + wave) * RT * 16, col0 = blockIdx.y * CT;
     const int ph = L::TAPS == 1 ? 0 : 1 - (int)(blockIdx.z >> 1), pw = L::TAPS == 1 ? 0 : 1 - (int)(blockIdx.z & 1);
@@ -404,8 +398,8 @@ __global__ __launch_bounds__(L::TAPS == 1 ? 64 : 256) void k_dgrad(const bf16* _
 #pragma unroll
                 for (int j = 0; j < CT; ++j) sum[i][j] = a + b ? sum[i][j] + acc[i][j] : acc[i][j];
         }
-    // mask, store and the sum over the tile's rows (lanes 0, 16, 32, 48 hold it)
-    const auto store = [&](int i, int j, v4f a, float (&s)[4]) {
+    // mask and store
+    const auto store = [&](int i, int j, v4f a) {
         const bool live = row0 + 16 * i + (lane & 15) < M;
         const int ch = (col0 + j) * 16 + 4 * (lane >> 4);
         constexpr int POS = L::TAPS == 1 ? 2 : 1;
@@ -419,30 +413,17 @@ __global__ __launch_bounds__(L::TAPS == 1 ? 64 : 256) void k_dgrad(const bf16* _
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 g[r] = live && bf_at(y, r) > 0.0f ? (L::TAPS == 1 ? a[r] / 2.0f : a[r]) : 0.0f;
-                s[r] += g[r];
             }
-            if (live) *(uint2*)(dZl + o) = pack4(g);
+            if (live) {
+                *(uint2*)(dZl + o) = pack4(g);
+                *(float4*)(dZf + o) = make_float4(g[0], g[1], g[2], g[3]);
+            }
         }
     };
 #pragma unroll
-    for (int j = 0; j < CT; ++j) {
-        float s[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
-        for (int i = 0; i < RT; ++i) store(i, j, sum[i][j], s);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-#pragma unroll
-            for (int d = 1; d < 16; d <<= 1) s[r] += __shfl_xor(s[r], d, 64);
-            if ((lane & 15) == 0) sums[wave][j * 16 + 4 * (lane >> 4) + r] = s[r];
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x < CT * 16) {
-        float s = sums[0][threadIdx.x];
-#pragma unroll
-        for (int q = 1; q < WAVES; ++q) s += sums[q][threadIdx.x];
-        part[(size_t)(blockIdx.z * gridDim.x + blockIdx.x) * L::CIN + col0 * 16 + threadIdx.x] = s;
-    }
+        for (int j = 0; j < CT; ++j) store(i, j, sum[i][j]);
 }
 
 // Weight gradient: dW = im2col(X)^T dZ over the rows of split blockIdx.z
@@ -509,11 +490,11 @@ __global__ __launch_bounds__(256) void k_wgrad(const bf16* __restrict__ X, const
         __syncthreads();
         if (m0 + kWgChunk < mend) load(m0 + kWgChunk);
 #pragma unroll
-        for (int s = 0; s < kWgChunk; s += 32) {
-            const int q = s + 8 * (lane >> 4);
-            const uint4 x = *(const uint4*)&Xs[wave * 16 + (lane & 15)][q];
+        for (int s = 0; s < kWgChunk; s += 16) {
+            const int q = s + 4 * (lane >> 4);
+            const uint2 x = *(const uint2*)&Xs[wave * 16 + (lane & 15)][q];
 #pragma unroll
-            for (int j = 0; j < NT; ++j) acc[j] = mma32(*(const uint4*)&Zs[j * 16 + (lane & 15)][q], x, acc[j]);
+            for (int j = 0; j < NT; ++j) acc[j] = mma16(*(const uint2*)&Zs[j * 16 + (lane & 15)][q], x, acc[j]);
         }
         __syncthreads();
     }
@@ -525,10 +506,9 @@ __global__ __launch_bounds__(256) void k_wgrad(const bf16* __restrict__ X, const
 }
 
 // The head's gradients: the weighted squared error over the first kHeadOut
-// outputs, loss = sum_j w_j (O - T)^2 and dO = 2 w_j (O - T) / N; then for the
-// linear layers dZ1 = (H1 > 0) ? dO W2^T : 0 (bf16) and, summed over the 16
-// samples of a chunk (blockIdx.y), H1^T dO, dZ1 and dO.  A thread is one
-// hidden unit, except in dO W2^T, which is formed as the other layers' products.
+// outputs, loss = sum_j w_j (O - T)^2 and dO = 2 w_j (O - T) / N; and dZ1 =
+// (H1 > 0) ? dO W2^T : 0; both as bf16 and, for the biases, fp32.  A workgroup
+// takes 16 samples (blockIdx.y) x 256 hidden units, four tiles a wave.
 constexpr int kHeadChunk = 16;
 struct LossWeights {
     float w[kHeadOut];
@@ -537,101 +517,138 @@ struct LossWeights {
 __global__ __launch_bounds__(256) void k_head_bwd(const float* __restrict__ O, const float* __restrict__ T,
                                                   LossWeights lw, int N, int H, const bf16* __restrict__ h1,
                                                   const bf16* __restrict__ W2, float* __restrict__ loss,
-                                                  bf16* __restrict__ dz1, float* __restrict__ partW2,
-                                                  float* __restrict__ partB1, float* __restrict__ partB2)
+                                                  bf16* __restrict__ dob, float* __restrict__ dof,
+                                                  bf16* __restrict__ dz1, float* __restrict__ dz1f)
 {
-    __shared__ float d16[kHeadChunk][kHeadOut], d32[kHeadChunk][kHeadOut];
     __shared__ __align__(8) bf16 db[kHeadChunk][kHeadPad];
-    __shared__ v4f gs[256 / 4][kHeadChunk + 1];
     const int r0 = blockIdx.y * kHeadChunk, rows = min(kHeadChunk, N - r0);
-    const int j = blockIdx.x * 256 + threadIdx.x;
     if (threadIdx.x < kHeadChunk)
         for (int q = 0; q < kHeadPad; ++q) db[threadIdx.x][q] = 0;
     if ((int)threadIdx.x < rows) {
         const int n = r0 + threadIdx.x;
         float l = 0.0f;
-        for (int q = 0; q < kHeadOut; ++q) {
-            const float e = O[(size_t)n * kHeadPad + q] - T[(size_t)n * kHeadOut + q];
-            l += lw.w[q] * e * e;
-            const float g = 2.0f * lw.w[q] * e / (float)N;
-            d32[threadIdx.x][q] = g;
-            db[threadIdx.x][q] = f2bf(g);
-            d16[threadIdx.x][q] = bf2f(f2bf(g));
+        for (int q = 0; q < kHeadPad; ++q) {
+            float g = 0.0f;
+            if (q < kHeadOut) {
+                const float e = O[(size_t)n * kHeadPad + q] - T[(size_t)n * kHeadOut + q];
+                l += lw.w[q] * e * e;
+                g = 2.0f * lw.w[q] * e / (float)N;
+                db[threadIdx.x][q] = f2bf(g);
+            }
+            if (blockIdx.x == 0) {
+                dob[(size_t)n * kHeadPad + q] = f2bf(g);
+                dof[(size_t)n * kHeadPad + q] = g;
+            }
         }
         if (loss && blockIdx.x == 0) loss[n] = l;
     }
     __syncthreads();
-    if (blockIdx.x == 0 && threadIdx.x < kHeadPad) {
-        float s = 0.0f;
-        if (threadIdx.x < kHeadOut)
-            for (int r = 0; r < rows; ++r) s += d32[r][threadIdx.x];
-        partB2[(size_t)blockIdx.y * kHeadPad + threadIdx.x] = s;
+    const int lane = threadIdx.x & 63, g4 = lane >> 4;
+    const int n = r0 + (lane & 15);
+    const uint2 x = g4 < 2 ? *(const uint2*)&db[lane & 15][4 * g4] : make_uint2(0, 0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int unit0 = (int)blockIdx.x * 256 + ((threadIdx.x >> 6) * 4 + q) * 16;
+        if (unit0 >= H) break;                            // whole tiles: H is a multiple of 16
+        const uint2 v = *(const uint2*)(W2 + (size_t)(unit0 + (lane & 15)) * kHeadPad + 4 * (g4 & 1));
+        const v4f a = mma16(g4 < 2 ? v : make_uint2(0, 0), x, v4f{0.f, 0.f, 0.f, 0.f});
+        if (n >= N) continue;
+        const size_t o = (size_t)n * H + unit0 + 4 * g4;
+        const uint2 y = *(const uint2*)(h1 + o);
+        float g[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) g[r] = bf_at(y, r) > 0.0f ? a[r] : 0.0f;
+        *(uint2*)(dz1 + o) = pack4(g);
+        *(float4*)(dz1f + o) = make_float4(g[0], g[1], g[2], g[3]);
     }
-    {
-        // dO W2^T of the workgroup's units, four tiles of 16 a wave
-        const int lane = threadIdx.x & 63, g4 = lane >> 4;
-        const uint2 x = g4 < 2 ? *(const uint2*)&db[lane & 15][4 * g4] : make_uint2(0, 0);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int tile = (threadIdx.x >> 6) * 4 + q, unit = min((int)blockIdx.x * 256 + tile * 16 + (lane & 15), H - 1);
-            const uint2 v = *(const uint2*)(W2 + (size_t)unit * kHeadPad + 4 * (g4 & 1));
-            gs[tile * 4 + g4][lane & 15] = mma16(g4 < 2 ? v : make_uint2(0, 0), x, v4f{0.f, 0.f, 0.f, 0.f});
-        }
-    }
-    __syncthreads();
-    if (j >= H) return;
-    bf16 hv[kHeadChunk];
-#pragma unroll
-    for (int r = 0; r < kHeadChunk; ++r) hv[r] = h1[(size_t)(r0 + min(r, rows - 1)) * H + j];
-    float sw[kHeadPad] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, sb = 0.0f;
-#pragma unroll
-    for (int r = 0; r < kHeadChunk; ++r) {
-        if (r >= rows) break;
-        const float h = bf2f(hv[r]);
-#pragma unroll
-        for (int q = 0; q < kHeadOut; ++q) sw[q] += h * d16[r][q];
-        const float g = h > 0.0f ? gs[threadIdx.x >> 2][r][threadIdx.x & 3] : 0.0f;
-        sb += g;
-        dz1[(size_t)(r0 + r) * H + j] = f2bf(g);
-    }
-    partB1[(size_t)blockIdx.y * H + j] = sb;
-    float* o = partW2 + ((size_t)blockIdx.y * H + j) * kHeadPad;
-    *(float4*)o = make_float4(sw[0], sw[1], sw[2], sw[3]);
-    *(float4*)(o + 4) = make_float4(sw[4], sw[5], sw[6], sw[7]);
 }
 
-// Every gradient's sum over its partial results, in one launch: 16 threads
-// share a group of four values, each sums every 16th part, and their sums are
-// added in order.
+// The head's weight gradient H1^T dO: 16 hidden units a wave, the samples in
+// chunks of `chunk` (a multiple of 16) whose sums are added in order.
+__global__ __launch_bounds__(256) void k_head_wgrad(const bf16* __restrict__ h1, const bf16* __restrict__ dob, int N,
+                                                    int H, int chunk, float* __restrict__ out)
+{
+    const int lane = threadIdx.x & 63, col = lane & 15, g4 = lane >> 4;
+    const int unit0 = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * 16;
+    if (unit0 >= H) return;
+    v4f sum = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int n0 = 0; n0 < N; n0 += chunk) {
+        const int end = min(N, n0 + chunk);
+        v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int n = n0; n < end; n += 16) {
+            uint32_t a[4], b[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int m = n + 4 * g4 + q, mc = min(m, N - 1);
+                const uint32_t h = h1[(size_t)mc * H + unit0 + col], d = dob[(size_t)mc * kHeadPad + (col & 7)];
+                a[q] = m < end ? h : 0u;
+                b[q] = m < end && col < kHeadPad ? d : 0u;
+            }
+            acc = mma16(make_uint2(a[0] | a[1] << 16, a[2] | a[3] << 16),
+                        make_uint2(b[0] | b[1] << 16, b[2] | b[3] << 16), acc);
+        }
+        sum = n0 ? sum + acc : acc;
+    }
+    if (col < kHeadPad)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[(size_t)(unit0 + 4 * g4 + r) * kHeadPad + col] = sum[r];
+}
+
+// Column sums of every layer's fp32 gradients (the biases'), in one launch: a
+// thread adds the rows of one chunk and column in order, 32 loads in flight.
 constexpr int kSumJobs = 2 * kLayers;
-struct SumJobs {
-    const float* part[kSumJobs];
-    float* dst[kSumJobs];
-    int parts[kSumJobs], n[kSumJobs], first[kSumJobs];   // values per part (of 4); first workgroup
+struct ColJobs {
+    const float* G[kLayers];
+    float* part[kLayers];                       // [chunks][N]
+    int M[kLayers], N[kLayers], rows[kLayers], chunks[kLayers], first[kLayers];
     int count;
 };
 
-__global__ __launch_bounds__(256) void k_sum_parts(SumJobs J)
+__global__ __launch_bounds__(64) void k_colsum(ColJobs J)
 {
     int s = 0;
     while (s + 1 < J.count && (int)blockIdx.x >= J.first[s + 1]) ++s;
-    const int lane = threadIdx.x & 15, share = threadIdx.x >> 4;
-    const int i = (((int)blockIdx.x - J.first[s]) * 16 + lane) * 4, n = J.n[s];
-    __shared__ v4f sums[16][16];
-    v4f a = v4f{0.f, 0.f, 0.f, 0.f};
-    if (i < n) {
-        const float* p = J.part[s] + i;
-        const int parts = J.parts[s];
-#pragma unroll 4
-        for (int z = share; z < parts; z += 16) a += *(const v4f*)(p + (size_t)z * n);
-    }
-    sums[share][lane] = a;
-    __syncthreads();
-    if (share == 0 && i < n) {
+    const int i = ((int)blockIdx.x - J.first[s]) * 64 + threadIdx.x, N = J.N[s];
+    if (i >= J.chunks[s] * N) return;
+    const int c = i / N, n = i - c * N;
+    const int r0 = c * J.rows[s], r1 = min(J.M[s], r0 + J.rows[s]);
+    const float* G = J.G[s] + n;
+    float a = 0.0f;
+    for (int r = r0; r < r1; r += 32) {
+        float v[32];
 #pragma unroll
-        for (int q = 1; q < 16; ++q) a += sums[q][lane];
-        *(v4f*)(J.dst[s] + i) = a;
+        for (int q = 0; q < 32; ++q) v[q] = G[(size_t)min(r + q, r1 - 1) * N];
+#pragma unroll
+        for (int q = 0; q < 32; ++q) a = r + q < r1 ? a + v[q] : a;
     }
+    J.part[s][i] = a;
+}
+
+// Every gradient's sum over its partial results, in order, in one launch: a
+// value a thread, 16 loads in flight.
+struct SumJobs {
+    const float* part[kSumJobs];
+    float* dst[kSumJobs];
+    int parts[kSumJobs], n[kSumJobs], first[kSumJobs];   // values per part; first workgroup
+    int count;
+};
+
+__global__ __launch_bounds__(64) void k_sum_parts(SumJobs J)
+{
+    int s = 0;
+    while (s + 1 < J.count && (int)blockIdx.x >= J.first[s + 1]) ++s;
+    const int i = ((int)blockIdx.x - J.first[s]) * 64 + threadIdx.x, n = J.n[s], parts = J.parts[s];
+    if (i >= n) return;
+    const float* p = J.part[s] + i;
+    float a = 0.0f;
+    for (int z = 0; z < parts; z += 16) {
+        float v[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) v[q] = p[(size_t)min(z + q, parts - 1) * n];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) a = z + q < parts ? a + v[q] : a;
+    }
+    J.dst[s][i] = a;
 }
 
 // Adam with decoupled weight decay on fp32 master weights; writes the bf16
@@ -762,8 +779,8 @@ struct cnn_net_s {
     bf16 *gap = nullptr, *h1 = nullptr;
     float* out = nullptr;            // [N][8]
     // backward scratch: gradients before the activations, partial sums
-    bf16 *dz[kConvs] = {}, *dz1 = nullptr;
-    float* part = nullptr;
+    bf16 *dz[kConvs] = {}, *dz1 = nullptr, *dob = nullptr;
+    float *dzf[kConvs] = {}, *dz1f = nullptr, *dof = nullptr, *part = nullptr;
     std::vector<void*> allocs;
 };
 
@@ -812,22 +829,24 @@ using Fc1 = Layer<1, kFc1In, kFc1Out>;
 using Fc2 = Layer<1, kFc1Out, kOutPad>;
 static_assert(kOut == kHeadOut && kOutPad == kHeadPad, "the head's outputs");
 
-// A weight gradient's rows are split until its workgroups give each of the
-// 256 CUs one or two (more splits only write more partial sums); with few
-// rows a single workgroup per tile writes the gradient itself.
-constexpr int kWgBlocks = 384;
+// The rows of a weight gradient's parts: up to 512 of 512 rows or more over
+// the layer's 64x64 output tiles.
+constexpr int wgrad_max_splits(int kp, int cout) { return std::max(1, 512 / std::max(1, kp * cout / 4096)); }
 
-template <class L, int BN>
-constexpr int wgrad_max_splits()
+inline int wgrad_rows(int M, int kp, int cout)
 {
-    return std::max(1, kWgBlocks / (((L::K + kWgTile - 1) / kWgTile) * (L::COUT / BN)));
+    const int splits = std::min(wgrad_max_splits(kp, cout), std::max(1, M / 512));
+    return cdiv(cdiv(M, splits), 32) * 32;
 }
 
-template <class L, int BN>
+template <class L>
 constexpr size_t wgrad_part_elems()
 {
-    return (size_t)wgrad_max_splits<L, BN>() * L::KP * L::COUT;
+    return (size_t)wgrad_max_splits(L::KP, L::COUT) * L::KP * L::COUT;
 }
+
+// The chunks of a bias gradient's rows.
+inline int col_chunks(int M) { return std::min(256, std::max(1, M / 64)); }
 
 // Workgroups along the rows of k_dgrad's largest parity class.
 template <class L, int RT>
@@ -892,8 +911,9 @@ void pack(cnn_net_s* c, const bf16* x, int N)
 struct Parts {
     cnn_net_s* c;
     SumJobs jobs{};
+    ColJobs cols{};
     size_t used = 0;
-    int blocks = 0;
+    int blocks = 0, col_blocks = 0;
 
     float* take(size_t n)
     {
@@ -901,7 +921,7 @@ struct Parts {
         used += n;
         return p;
     }
-    // dst = the sum of `parts` parts of n values (a multiple of 4) at p
+    // dst = the sum of `parts` parts of n values at p
     void sum(const float* p, int parts, int n, float* dst)
     {
         const int q = jobs.count++;
@@ -912,16 +932,26 @@ struct Parts {
         jobs.first[q] = blocks;
         blocks += cdiv(n, 64);
     }
+    // dst = the column sums of G [M][N]
+    void columns(const float* G, int M, int N, float* dst)
+    {
+        const int q = cols.count++, chunks = col_chunks(M);
+        cols.G[q] = G;
+        cols.part[q] = take((size_t)chunks * N);
+        cols.M[q] = M;
+        cols.N[q] = N;
+        cols.rows[q] = cdiv(M, chunks);
+        cols.chunks[q] = chunks;
+        cols.first[q] = col_blocks;
+        col_blocks += cdiv(chunks * N, 64);
+        sum(cols.part[q], chunks, N, dst);
+    }
 };
 
 template <class L, int BN>
 void launch_wgrad(Parts& w, const bf16* X, const bf16* dZ, int M, float* dst)
 {
-    const int kt = cdiv(L::K, kWgTile), chunks = cdiv(M, kWgChunk);
-    int splits = std::min(wgrad_max_splits<L, BN>(), chunks);
-    if (chunks <= 8 && kt * (L::COUT / BN) >= 48) splits = 1;
-    const int rows_per = cdiv(chunks, splits) * kWgChunk;
-    splits = cdiv(M, rows_per);
+    const int kt = cdiv(L::K, kWgTile), rows_per = wgrad_rows(M, L::KP, L::COUT), splits = cdiv(M, rows_per);
     float* out = splits == 1 ? dst : w.take((size_t)splits * L::KP * L::COUT);
     hipLaunchKernelGGL((k_wgrad<L, BN>), dim3(kt, L::COUT / BN, splits), dim3(256), 0, w.c->stream, X, dZ, M,
                        rows_per, out);
@@ -929,27 +959,22 @@ void launch_wgrad(Parts& w, const bf16* X, const bf16* dZ, int M, float* dst)
 }
 
 template <class L, int RT, int CT>
-void launch_dgrad(Parts& w, const bf16* dZ, const bf16* W, const bf16* Yl, int N, bf16* dZl, float* dbias)
+void launch_dgrad(Parts& w, const bf16* dZ, const bf16* W, const bf16* Yl, int N, bf16* dZl, float* dZf, float* dbias)
 {
     const int classes = L::TAPS == 1 ? 1 : 4, blocks = dgrad_blocks<L, RT>(N);
-    float* out = w.take((size_t)classes * blocks * L::CIN);
-    hipLaunchKernelGGL((k_dgrad<L, RT, CT>), dim3(blocks, L::CIN / 16 / CT, classes), dim3(L::TAPS == 1 ? 64 : 256), 0, w.c->stream, dZ, W, Yl, N, dZl, out);
-    w.sum(out, classes * blocks, L::CIN, dbias);
+    hipLaunchKernelGGL((k_dgrad<L, RT, CT>), dim3(blocks, L::CIN / 16 / CT, classes), dim3(L::TAPS == 1 ? 64 : 256), 0,
+                       w.c->stream, dZ, W, Yl, N, dZl, dZf);
+    w.columns(dZf, L::TAPS == 1 ? 2 * N : N * L::HI * L::WI, L::CIN, dbias);
 }
 
 // Room for the partial sums of a batch of N (all of cnn_backward's takes).
 size_t part_elems(int N)
 {
-    const size_t chunks = cdiv(N, kHeadChunk);
-    size_t n = wgrad_part_elems<Conv0, 32>() + wgrad_part_elems<Conv1, 64>() + wgrad_part_elems<Conv2, 96>() +
-               wgrad_part_elems<Conv3, 128>() + wgrad_part_elems<Conv4, 128>() + wgrad_part_elems<Conv5, 128>() +
-               wgrad_part_elems<Fc1, 128>();
-    n += chunks * ((size_t)kFc1Out * (kOutPad + 1) + kOutPad);
-    n += 4 * ((size_t)dgrad_blocks<Conv1, 2>(N) * Conv1::CIN + (size_t)dgrad_blocks<Conv2, 2>(N) * Conv2::CIN +
-              (size_t)dgrad_blocks<Conv3, 1>(N) * Conv3::CIN + (size_t)dgrad_blocks<Conv4, 1>(N) * Conv4::CIN +
-              (size_t)dgrad_blocks<Conv5, 1>(N) * Conv5::CIN) +
-         (size_t)dgrad_blocks<Fc1, 1>(N) * Fc1::CIN;
-    return n;
+    size_t n = wgrad_part_elems<Conv0>() + wgrad_part_elems<Conv1>() + wgrad_part_elems<Conv2>() +
+               wgrad_part_elems<Conv3>() + wgrad_part_elems<Conv4>() + wgrad_part_elems<Conv5>() +
+               wgrad_part_elems<Fc1>();
+    for (const auto& c : kSpec) n += (size_t)col_chunks(N * c.ho * c.wo) * c.cout;
+    return n + (size_t)col_chunks(N) * (kFc1Out + kOutPad);
 }
 
 }  // namespace
@@ -1319,6 +1344,7 @@ int cnn_create(int max_batch, cnn_net* out)
         const size_t n = (size_t)N * kSpec[l].ho * kSpec[l].wo * kSpec[l].cout;
         rc = dalloc(c, &c->y[l], n);
         rc = rc ? rc : dalloc(c, &c->dz[l], n);
+        rc = rc ? rc : dalloc(c, &c->dzf[l], n);
     }
     size_t pf_n = 0;
     for (int q = 0; q < kPackJobs; ++q) {
@@ -1332,6 +1358,9 @@ int cnn_create(int max_batch, cnn_net* out)
     rc = rc ? rc : dalloc(c, &c->gap, (size_t)N * kFc1In);
     rc = rc ? rc : dalloc(c, &c->h1, (size_t)N * kFc1Out);
     rc = rc ? rc : dalloc(c, &c->dz1, (size_t)N * kFc1Out);
+    rc = rc ? rc : dalloc(c, &c->dz1f, (size_t)N * kFc1Out);
+    rc = rc ? rc : dalloc(c, &c->dob, (size_t)N * kOutPad);
+    rc = rc ? rc : dalloc(c, &c->dof, (size_t)N * kOutPad);
     rc = rc ? rc : dalloc(c, &c->out, (size_t)N * kOutPad);
     rc = rc ? rc : dalloc(c, &c->part, part_elems(N));
     if (rc) {
@@ -1602,29 +1631,27 @@ int cnn_backward(cnn_net c, int N, const float* target, const float* w, float* l
     Parts P{c};
     const auto g = [&](const Param& p) { return c->g + p.off; };
     const auto wd = [&](int l) { return (const bf16*)(c->pf + c->pf_off[kLayers + l - 1]); };   // conv l, or fc1 as 6
-    const int chunks = cdiv(N, kHeadChunk);
-    float* pw2 = P.take((size_t)chunks * kFc1Out * kOutPad);
-    float* pb1 = P.take((size_t)chunks * kFc1Out);
-    float* pb2 = P.take((size_t)chunks * kOutPad);
-    hipLaunchKernelGGL(k_head_bwd, dim3(cdiv(kFc1Out, 256), chunks), dim3(256), 0, c->stream, c->out, target, lw, N,
-                       kFc1Out, c->h1, c->pb + c->fc2W.off, loss_n, c->dz1, pw2, pb1, pb2);
-    P.sum(pw2, chunks, kFc1Out * kOutPad, g(c->fc2W));
-    P.sum(pb1, chunks, kFc1Out, g(c->fc1B));
-    P.sum(pb2, chunks, kOutPad, g(c->fc2B));
+    hipLaunchKernelGGL(k_head_bwd, dim3(cdiv(kFc1Out, 256), cdiv(N, kHeadChunk)), dim3(256), 0, c->stream, c->out,
+                       target, lw, N, kFc1Out, c->h1, c->pb + c->fc2W.off, loss_n, c->dob, c->dof, c->dz1, c->dz1f);
+    hipLaunchKernelGGL(k_head_wgrad, dim3(cdiv(kFc1Out, 64)), dim3(256), 0, c->stream, c->h1, c->dob, N, kFc1Out,
+                       wgrad_rows(N, kFc1Out, kOutPad), g(c->fc2W));
+    P.columns(c->dof, N, kOutPad, g(c->fc2B));
+    P.columns(c->dz1f, N, kFc1Out, g(c->fc1B));
     launch_wgrad<Fc1, 128>(P, c->gap, c->dz1, N, g(c->fc1W));
-    launch_dgrad<Fc1, 1, 1>(P, c->dz1, wd(6), c->y[5], N, c->dz[5], g(c->convB[5]));
-    launch_wgrad<Conv5, 128>(P, c->y[4], c->dz[5], N * 2, g(c->convW[5]));
-    launch_dgrad<Conv5, 1, 1>(P, c->dz[5], wd(5), c->y[4], N, c->dz[4], g(c->convB[4]));
-    launch_wgrad<Conv4, 128>(P, c->y[3], c->dz[4], N * 6, g(c->convW[4]));
-    launch_dgrad<Conv4, 1, 1>(P, c->dz[4], wd(4), c->y[3], N, c->dz[3], g(c->convB[3]));
-    launch_wgrad<Conv3, 128>(P, c->y[2], c->dz[3], N * 20, g(c->convW[3]));
-    launch_dgrad<Conv3, 1, 3>(P, c->dz[3], wd(3), c->y[2], N, c->dz[2], g(c->convB[2]));
+    launch_dgrad<Fc1, 1, 1>(P, c->dz1, wd(6), c->y[5], N, c->dz[5], c->dzf[5], g(c->convB[5]));
+    launch_wgrad<Conv5, 32>(P, c->y[4], c->dz[5], N * 2, g(c->convW[5]));
+    launch_dgrad<Conv5, 1, 1>(P, c->dz[5], wd(5), c->y[4], N, c->dz[4], c->dzf[4], g(c->convB[4]));
+    launch_wgrad<Conv4, 32>(P, c->y[3], c->dz[4], N * 6, g(c->convW[4]));
+    launch_dgrad<Conv4, 1, 1>(P, c->dz[4], wd(4), c->y[3], N, c->dz[3], c->dzf[3], g(c->convB[3]));
+    launch_wgrad<Conv3, 64>(P, c->y[2], c->dz[3], N * 20, g(c->convW[3]));
+    launch_dgrad<Conv3, 1, 3>(P, c->dz[3], wd(3), c->y[2], N, c->dz[2], c->dzf[2], g(c->convB[2]));
     launch_wgrad<Conv2, 96>(P, c->y[1], c->dz[2], N * 80, g(c->convW[2]));
-    launch_dgrad<Conv2, 2, 4>(P, c->dz[2], wd(2), c->y[1], N, c->dz[1], g(c->convB[1]));
+    launch_dgrad<Conv2, 2, 4>(P, c->dz[2], wd(2), c->y[1], N, c->dz[1], c->dzf[1], g(c->convB[1]));
     launch_wgrad<Conv1, 64>(P, c->y[0], c->dz[1], N * 300, g(c->convW[1]));
-    launch_dgrad<Conv1, 2, 2>(P, c->dz[1], wd(1), c->y[0], N, c->dz[0], g(c->convB[0]));
+    launch_dgrad<Conv1, 2, 2>(P, c->dz[1], wd(1), c->y[0], N, c->dz[0], c->dzf[0], g(c->convB[0]));
     launch_wgrad<Conv0, 32>(P, c->x, c->dz[0], N * 1200, g(c->convW[0]));
-    hipLaunchKernelGGL(k_sum_parts, dim3(P.blocks), dim3(256), 0, c->stream, P.jobs);
+    hipLaunchKernelGGL(k_colsum, dim3(P.col_blocks), dim3(64), 0, c->stream, P.cols);
+    hipLaunchKernelGGL(k_sum_parts, dim3(P.blocks), dim3(64), 0, c->stream, P.jobs);
     return launch_check("backward");
 }
 
