@@ -11,8 +11,9 @@
 //   - points drawn at a surfel's texel of the update maps, where the depth
 //     test at equal depth keeps the first pixel drawn: an atomic minimum of
 //     the pixel's draw index per surfel;
-//   - transform feedback, which appends in draw order: flags, an exclusive
-//     scan in draw order, and a scatter.
+//   - transform feedback, which appends in draw order: a bit per item and a
+//     count per 256 items, from which the next pass finds each kept item's
+//     place (initialise: flags, an exclusive scan and a scatter).
 // Draw order is the reference's: pixels column by column (its uv buffers),
 // surfels by index.  The per-pixel maps of this file (metric depth, index map,
 // per-pixel fusion data) are stored in that order too, at d = x * height + y:
