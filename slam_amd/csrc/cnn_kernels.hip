@@ -147,7 +147,7 @@ __device__ __forceinline__ uint2 patch4(const bf16* __restrict__ X, const RowPos
 // Forward: Y = relu(im2col(X) W + b) as bf16, and for the last convolution the
 // mean over its two positions (GAP); or fp32 sums without ReLU, eight columns
 // per row and the first kHeadOut of them to `user` (HEAD).
-//   Wf: the weights in fragment order (k_pack): k step s, column tile j, lane
+//   Wf: the weights in fragment order (store_weight): k step s, column tile j, lane
 //   L hold W[16 s + 4 (L >> 4) + q][16 j + (L & 15)], q = 0..3.
 // A wave forms RT row tiles x CT column tiles, in chunks of `chunk` (an even
 // number of) k steps whose sums are added in order.  KS = 1: a workgroup is
@@ -263,53 +263,50 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_fwd(const bf16* __r
     }
 }
 
-// The weights [K][ld] of every layer in k_fwd's fragment order, columns from
-// ld to the tile's end as 0, and those of the layers with an input gradient in
-// k_dgrad's (the same for the transposed weights: row tile r, k step s, lane L
-// hold W[16 r + (L & 15)][16 s + 4 (L >> 4) + q]) (blockIdx.y = job); and a copy of the input,
-// which backward needs and which gives it the loads' alignment (the last
-// blockIdx.y).
-constexpr int kLayers = 8, kPackJobs = kLayers + 6;
-struct PackJobs {
-    const bf16* src[kPackJobs];
-    bf16* dst[kPackJobs];
-    int n[kPackJobs], nt[kPackJobs], ld[kPackJobs];   // n: fragments of 4 (KP / 16 * nt * 64)
-    const bf16* x;
-    bf16* xcopy;
-    int nx, jobs;                               // fragments of 8; kPackJobs, or 0 when packed already
+constexpr int kLayers = 8;
+
+// The bf16 weights in every form that a kernel reads: as they lie in the
+// parameter vector, in k_fwd's (and the inference's) fragment order, and for
+// the layers with an input gradient in k_dgrad's (the same for the transposed
+// weights: row tile r, k step s, lane L hold W[16 r + (L & 15)][16 s + 4 (L >> 4)
+// + q]).  Whoever writes a weight writes them all, so no call has to know
+// whether they are up to date, and a captured graph stays right when its
+// weights change.  first, n: a layer's weights [n / ld][ld] in the vector,
+// multiples of 64, so a wave's 64 parameters lie in one tensor.  k_fwd's
+// columns from ld to the tile's end stay 0.
+struct WeightForms {
+    bf16* flat;
+    bf16 *fwd[kLayers], *dgrad[kLayers];        // dgrad: null without an input gradient
+    int first[kLayers], n[kLayers], ld[kLayers];
 };
 
-__global__ __launch_bounds__(256) void k_pack(PackJobs P)
+// Whole waves of consecutive i, the first a multiple of 64.
+__device__ __forceinline__ void store_weight(const WeightForms& F, int i, bf16 b)
 {
-    const int l = blockIdx.y;
-    if (l == P.jobs) {
-        const bool wide = ((uintptr_t)P.x & 15) == 0;
-        for (int e = blockIdx.x * 256 + threadIdx.x; e < P.nx; e += gridDim.x * 256) {
-            const bf16* p = P.x + (size_t)e * 8;
-            uint4 v;
-            if (wide) v = *(const uint4*)p;
-            else v = make_uint4(p[0] | (uint32_t)p[1] << 16, p[2] | (uint32_t)p[3] << 16,
-                                p[4] | (uint32_t)p[5] << 16, p[6] | (uint32_t)p[7] << 16);
-            *(uint4*)(P.xcopy + (size_t)e * 8) = v;
-        }
-        return;
-    }
-    const int e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= P.n[l]) return;
-    const int lane = e & 63, tile = e >> 6, nt = P.nt[l], ld = P.ld[l];
-    if (l >= kLayers) {
-        const int row = (tile / nt) * 16 + (lane & 15), c = (tile % nt) * 16 + 4 * (lane >> 4);
-        *(uint2*)(P.dst[l] + (size_t)e * 4) = *(const uint2*)(P.src[l] + (size_t)row * ld + c);
-        return;
-    }
-    const int col = (tile % nt) * 16 + (lane & 15), k = (tile / nt) * 16 + 4 * (lane >> 4);
-    uint32_t o[2];
+    F.flat[i] = b;
+    const int base = __builtin_amdgcn_readfirstlane(i & ~63);
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        const bf16* p = P.src[l] + (size_t)(k + 2 * q) * ld + col;
-        o[q] = col < ld ? p[0] | (uint32_t)p[ld] << 16 : 0u;
+    for (int l = 0; l < kLayers; ++l) {
+        if ((unsigned)(base - F.first[l]) >= (unsigned)F.n[l]) continue;
+        const int e = i - F.first[l], ld = F.ld[l], k = e / ld, c = e - k * ld, tile = (k >> 4) * ((ld + 15) >> 4) + (c >> 4);
+        F.fwd[l][(tile * 64 + ((k >> 2) & 3) * 16 + (c & 15)) * 4 + (k & 3)] = b;
+        if (F.dgrad[l]) F.dgrad[l][(tile * 64 + ((c >> 2) & 3) * 16 + (k & 15)) * 4 + (c & 3)] = b;
     }
-    *(uint2*)(P.dst[l] + (size_t)e * 4) = make_uint2(o[0], o[1]);
+}
+
+// A copy of the input, which backward needs (the caller's may be gone by then)
+// and which gives it the loads' alignment.  n: fragments of 8.
+__global__ __launch_bounds__(256) void k_copy_input(const bf16* __restrict__ x, int n, bf16* __restrict__ to)
+{
+    const bool wide = ((uintptr_t)x & 15) == 0;
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) {
+        const bf16* p = x + (size_t)e * 8;
+        uint4 v;
+        if (wide) v = *(const uint4*)p;
+        else v = make_uint4(p[0] | (uint32_t)p[1] << 16, p[2] | (uint32_t)p[3] << 16,
+                            p[4] | (uint32_t)p[5] << 16, p[6] | (uint32_t)p[7] << 16);
+        *(uint4*)(to + (size_t)e * 8) = v;
+    }
 }
 
 // Input gradient, through the ReLU of the layer below: dZl = (Yl > 0) ? dX : 0
@@ -322,7 +319,7 @@ __global__ __launch_bounds__(256) void k_pack(PackJobs P)
 // half its gradient; it has few tiles and a long reduction, so its waves are
 // workgroups of their own, on as many CUs.  A wave forms RT row tiles x CT
 // column tiles; each tap's product is summed by itself, then the taps in order.
-//   Wp: the weights in k_dgrad's fragment order (k_pack).
+//   Wp: the weights in k_dgrad's fragment order (store_weight).
 template <class L, int RT, int CT>
 __global__ __launch_bounds__(L::TAPS == 1 ? 64 : 256) void k_dgrad(const bf16* __restrict__ dZ,
                                                                    const bf16* __restrict__ Wp,
@@ -652,34 +649,33 @@ __global__ __launch_bounds__(64) void k_sum_parts(SumJobs J)
 }
 
 // Adam with decoupled weight decay on fp32 master weights; writes the bf16
-// copy the GEMMs read.  Entries with mask 0 (reduction padding) stay 0.
+// copies that the products read.  Entries with mask 0 (reduction padding)
+// stay 0.  n: a multiple of 64.
 __global__ __launch_bounds__(256) void k_adam(float* __restrict__ p, const float* __restrict__ g,
-                                              float* __restrict__ m, float* __restrict__ v, bf16* __restrict__ pb,
-                                              const uint8_t* __restrict__ mask, size_t n, float lr, float b1, float b2,
+                                              float* __restrict__ m, float* __restrict__ v, WeightForms F,
+                                              const uint8_t* __restrict__ mask, int n, float lr, float b1, float b2,
                                               float eps, float bc1, float bc2, float wd)
 {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    if (mask && !mask[i]) {
-        p[i] = 0.0f;
-        pb[i] = 0;
-        return;
+    float pi = 0.0f;
+    if (!mask || mask[i]) {
+        const float gi = g[i];
+        const float mi = b1 * m[i] + (1.0f - b1) * gi;
+        const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
+        m[i] = mi;
+        v[i] = vi;
+        const float upd = (mi / bc1) / (sqrtf(vi / bc2) + eps);
+        pi = p[i] * (1.0f - lr * wd) - lr * upd;
     }
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float upd = (mi / bc1) / (sqrtf(vi / bc2) + eps);
-    const float pi = p[i] * (1.0f - lr * wd) - lr * upd;
     p[i] = pi;
-    pb[i] = f2bf(pi);
+    store_weight(F, i, f2bf(pi));
 }
 
-__global__ __launch_bounds__(256) void k_to_bf16(const float* __restrict__ a, size_t n, bf16* __restrict__ b)
+__global__ __launch_bounds__(256) void k_to_bf16(const float* __restrict__ a, int n, WeightForms F)
 {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) b[i] = f2bf(a[i]);
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) store_weight(F, i, f2bf(a[i]));
 }
 
 // Network input from frame data at twice the input resolution (2W x 2H):
@@ -756,11 +752,7 @@ struct cnn_net_s {
     size_t nparam = 0;
     float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
     bf16* pb = nullptr;
-    // the conv weights in the inference kernel's fragment order (k_pack_infer),
-    // repacked when the weights have changed since the last pack
-    bf16* pw = nullptr;
-    size_t pw_off[kConvs] = {};
-    unsigned long long wver = 1, pver = 0;
+    WeightForms forms{};             // where the bf16 weights go
     // the split inference head: pooled features, per-workgroup FC2 partials
     // and the per-sample arrival tickets (back to 0 after every launch)
     int infer_split = 1;
@@ -768,10 +760,6 @@ struct cnn_net_s {
     unsigned int* infer_ticket = nullptr;
     uint8_t* mask = nullptr;
     int step = 0;
-    // the weights in k_fwd's and k_dgrad's fragment orders (k_pack), repacked likewise
-    bf16* pf = nullptr;
-    size_t pf_off[kPackJobs] = {};
-    unsigned long long fver = 0;
     // a copy of the last forward's input (the caller's may be gone before
     // cnn_backward) and its activations, sized for max_batch
     bf16* x = nullptr;
@@ -877,34 +865,7 @@ void launch_fwd(cnn_net_s* c, int layer, const bf16* X, int N, const float* bias
     const int M = N * L::HO * L::WO;
     const dim3 grid(cdiv(M, (KS == 1 ? 64 : 16) * RT), cdiv(L::COUT, 16) / CT);
     hipLaunchKernelGGL((k_fwd<L, RT, CT, KS, OUT, PARTS>), grid, dim3(KS == 1 ? 256 : 64 * KS), 0, c->stream, X,
-                       c->pf + c->pf_off[layer], bias, M, fwd_chunk<L>(N), Y, gap, out, user);
-}
-
-// The packed weights, when they have changed since the last pack, and a copy
-// of N samples (none: x null).
-void pack(cnn_net_s* c, const bf16* x, int N)
-{
-    PackJobs J{};
-    J.x = x;
-    J.xcopy = c->x;
-    J.nx = x ? N * (60 * 80 * 4 / 8) : 0;
-    int frags = 0;
-    if (c->fver != c->wver) {
-        J.jobs = kPackJobs;
-        for (int q = 0; q < kPackJobs; ++q) {
-            const int l = q < kLayers ? q : q - kLayers + 1;
-            const Param& w = l < kConvs ? c->convW[l] : (l == kConvs ? c->fc1W : c->fc2W);
-            J.ld[q] = l < kConvs ? kSpec[l].cout : (l == kConvs ? kFc1Out : kOutPad);
-            J.nt[q] = cdiv(J.ld[q], 16);
-            J.n[q] = (int)(w.n / J.ld[q]) / 16 * J.nt[q] * 64;
-            J.src[q] = c->pb + w.off;
-            J.dst[q] = c->pf + c->pf_off[q];
-            frags = std::max(frags, J.n[q]);
-        }
-        c->fver = c->wver;
-    }
-    const int blocks = std::max(cdiv(frags, 256), std::min(cdiv(J.nx, 256), 2048));
-    hipLaunchKernelGGL(k_pack, dim3(blocks, J.jobs + 1), dim3(256), 0, c->stream, J);
+                       c->forms.fwd[layer], bias, M, fwd_chunk<L>(N), Y, gap, out, user);
 }
 
 // The partial sums of one backward pass, taken from c->part in order.
@@ -1005,7 +966,7 @@ constexpr int kInferZero = kInferBufA + kInferBufB;
 static_assert(kInferIn <= kInferBufB, "the input fits its buffer");
 
 struct InferParams {
-    const bf16* W[kConvs];                   // fragment order (k_pack_infer) bf16
+    const bf16* W[kConvs];                   // k_fwd's fragment order
     const float* b[kConvs];
     int Kp[kConvs];
     const bf16* fc1W;                        // [128][3840]
@@ -1013,27 +974,6 @@ struct InferParams {
     const bf16* fc2W;                        // [256][8]
     const float* fc2b;
 };
-
-// The conv weights [Kp][Cout] of every layer in the inference kernel's
-// fragment order (grid.y = layer).
-struct PackArgs {
-    const bf16* src[kConvs];
-    bf16* dst[kConvs];
-    size_t n[kConvs];
-    int nt[kConvs], cout[kConvs];
-};
-
-__global__ __launch_bounds__(256) void k_pack_infer(PackArgs A)
-{
-    const int l = blockIdx.y;
-    const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= A.n[l]) return;
-    const int q = (int)(e & 3), lane = (int)((e >> 2) & 63);
-    const size_t r = e >> 8;
-    const int nt = (int)(r % A.nt[l]), ks = (int)(r / A.nt[l]);
-    const int k = ks * 16 + 4 * (lane >> 4) + q, n = nt * 16 + (lane & 15);
-    A.dst[l][e] = A.src[l][(size_t)k * A.cout[l] + n];
-}
 
 // One convolution layer (3x3, stride 2, pad 1) from X (LDS, [HI][WI][CIN])
 // into Y (LDS, [HO][WO][COUT]).  Each wave takes (column tile, up to four row
@@ -1331,12 +1271,6 @@ int cnn_create(int max_batch, cnn_net* out)
     rc = rc ? rc : dalloc(c, &c->v, off);
     rc = rc ? rc : dalloc(c, &c->pb, off);
     rc = rc ? rc : dalloc(c, &c->mask, off);
-    size_t pw_n = 0;
-    for (int l = 0; l < kConvs; ++l) {
-        c->pw_off[l] = pw_n;
-        pw_n += (size_t)c->Kp[l] * kSpec[l].cout;
-    }
-    rc = rc ? rc : dalloc(c, &c->pw, pw_n);
     rc = rc ? rc : dalloc(c, &c->infer_gap, (size_t)N * kFc1In);
     rc = rc ? rc : dalloc(c, &c->infer_part, (size_t)N * kHeadGroups * kOutPad);
     rc = rc ? rc : dalloc(c, &c->infer_ticket, (size_t)N);
@@ -1346,14 +1280,22 @@ int cnn_create(int max_batch, cnn_net* out)
         rc = rc ? rc : dalloc(c, &c->dz[l], n);
         rc = rc ? rc : dalloc(c, &c->dzf[l], n);
     }
-    size_t pf_n = 0;
-    for (int q = 0; q < kPackJobs; ++q) {
-        const int l = q < kLayers ? q : q - kLayers + 1;   // conv 1..5 and fc1 have input gradients
-        c->pf_off[q] = pf_n;
-        pf_n += l < kConvs ? (size_t)c->Kp[l] * kSpec[l].cout
-                           : (l == kConvs ? (size_t)kFc1In * kFc1Out : (size_t)kFc1Out * 16);
+    size_t form_n[2 * kLayers] = {}, form_total = 0;
+    c->forms.flat = c->pb;
+    for (int l = 0; l < kLayers; ++l) {
+        const Param& w = l < kConvs ? c->convW[l] : (l == kConvs ? c->fc1W : c->fc2W);
+        const int ld = l < kConvs ? kSpec[l].cout : (l == kConvs ? kFc1Out : kOutPad);
+        c->forms.first[l] = (int)w.off;
+        c->forms.n[l] = (int)w.n;
+        c->forms.ld[l] = ld;
+        form_n[l] = w.n / ld * (cdiv(ld, 16) * 16);
+        form_n[kLayers + l] = l > 0 && l <= kConvs ? w.n : 0;   // conv 1..5 and fc1 have input gradients
+        form_total += form_n[l] + form_n[kLayers + l];
     }
-    rc = rc ? rc : dalloc(c, &c->pf, pf_n);
+    bf16* form = nullptr;
+    rc = rc ? rc : dalloc(c, &form, form_total);
+    for (size_t q = 0, at = 0; q < 2 * kLayers && !rc; at += form_n[q++])
+        (q < kLayers ? c->forms.fwd[q] : c->forms.dgrad[q - kLayers]) = form_n[q] ? form + at : nullptr;
     rc = rc ? rc : dalloc(c, &c->x, (size_t)N * 60 * 80 * 4);
     rc = rc ? rc : dalloc(c, &c->gap, (size_t)N * kFc1In);
     rc = rc ? rc : dalloc(c, &c->h1, (size_t)N * kFc1Out);
@@ -1379,7 +1321,7 @@ int cnn_create(int max_batch, cnn_net* out)
     if (hipMemcpy(c->mask, mk.data(), off, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(c->p, 0, off * 4) != hipSuccess || hipMemset(c->g, 0, off * 4) != hipSuccess ||
         hipMemset(c->m, 0, off * 4) != hipSuccess || hipMemset(c->v, 0, off * 4) != hipSuccess ||
-        hipMemset(c->pb, 0, off * 2) != hipSuccess ||
+        hipMemset(c->pb, 0, off * 2) != hipSuccess || hipMemset(form, 0, form_total * 2) != hipSuccess ||
         hipMemset(c->infer_ticket, 0, (size_t)N * sizeof(unsigned int)) != hipSuccess) {
         cnn_destroy(c);
         return CNN_ERR_HIP;
@@ -1430,8 +1372,7 @@ int cnn_set_params(cnn_net c, const float* host, size_t n)
 {
     if (!c || !host || n != c->nparam) return CNN_ERR_ARG;
     CK(hipMemcpy(c->p, host, n * 4, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_to_bf16, g1(n), dim3(256), 0, c->stream, c->p, n, c->pb);
-    c->wver++;
+    hipLaunchKernelGGL(k_to_bf16, g1(n), dim3(256), 0, c->stream, c->p, (int)n, c->forms);
     CK(hipMemset(c->m, 0, n * 4));
     CK(hipMemset(c->v, 0, n * 4));
     c->step = 0;
@@ -1469,7 +1410,9 @@ int cnn_prepare_input(cnn_net c, const float* depth_a, const uint8_t* image_a, c
 int cnn_forward(cnn_net c, const void* x, int N, float* out)
 {
     if (!c || !x || N < 1 || N > c->max_batch) return CNN_ERR_ARG;
-    pack(c, (const bf16*)x, N);
+    const int frags = N * (60 * 80 * 4 / 8);
+    hipLaunchKernelGGL(k_copy_input, dim3(std::min(cdiv(frags, 256), 2048)), dim3(256), 0, c->stream, (const bf16*)x,
+                       frags, c->x);
     const auto b = [&](const Param& p) { return c->p + p.off; };
     launch_fwd<Conv0, 4, 2, 1, kRelu>(c, 0, c->x, N, b(c->convB[0]), c->y[0]);
     launch_fwd<Conv1, 2, 4, 1, kRelu>(c, 1, c->y[0], N, b(c->convB[1]), c->y[1]);
@@ -1573,23 +1516,9 @@ int cnn_infer(cnn_net c, const void* x, int N, float* out)
 {
     if (!c || !x || !out || N < 1 || N > c->max_batch) return CNN_ERR_ARG;
     if ((uintptr_t)x % 16 != 0) return CNN_ERR_ARG;
-    if (c->pver != c->wver) {
-        PackArgs A;
-        size_t n = 0;
-        for (int l = 0; l < kConvs; ++l) {
-            A.src[l] = c->pb + c->convW[l].off;
-            A.dst[l] = c->pw + c->pw_off[l];
-            A.n[l] = (size_t)c->Kp[l] * kSpec[l].cout;
-            A.nt[l] = kSpec[l].cout / 16;
-            A.cout[l] = kSpec[l].cout;
-            n = std::max(n, A.n[l]);
-        }
-        hipLaunchKernelGGL(k_pack_infer, dim3((unsigned)((n + 255) / 256), kConvs), dim3(256), 0, c->stream, A);
-        c->pver = c->wver;
-    }
     InferParams P;
     for (int l = 0; l < kConvs; ++l) {
-        P.W[l] = c->pw + c->pw_off[l];
+        P.W[l] = c->forms.fwd[l];
         P.b[l] = c->p + c->convB[l].off;
         P.Kp[l] = c->Kp[l];
     }
@@ -1625,12 +1554,11 @@ int cnn_set_infer_split(cnn_net c, int split)
 int cnn_backward(cnn_net c, int N, const float* target, const float* w, float* loss_n)
 {
     if (!c || !target || !w || N < 1 || N > c->max_batch) return CNN_ERR_ARG;
-    if (c->fver != c->wver) pack(c, nullptr, 0);   // the gradients are those of the present weights
     LossWeights lw;
     for (int j = 0; j < kOut; ++j) lw.w[j] = w[j];
     Parts P{c};
     const auto g = [&](const Param& p) { return c->g + p.off; };
-    const auto wd = [&](int l) { return (const bf16*)(c->pf + c->pf_off[kLayers + l - 1]); };   // conv l, or fc1 as 6
+    const auto wd = [&](int l) { return (const bf16*)c->forms.dgrad[l]; };   // conv l, or fc1 as 6
     hipLaunchKernelGGL(k_head_bwd, dim3(cdiv(kFc1Out, 256), cdiv(N, kHeadChunk)), dim3(256), 0, c->stream, c->out,
                        target, lw, N, kFc1Out, c->h1, c->pb + c->fc2W.off, loss_n, c->dob, c->dof, c->dz1, c->dz1f);
     hipLaunchKernelGGL(k_head_wgrad, dim3(cdiv(kFc1Out, 64)), dim3(256), 0, c->stream, c->h1, c->dob, N, kFc1Out,
@@ -1661,9 +1589,8 @@ int cnn_adam_step(cnn_net c, float lr, float wd)
     c->step++;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     const float bc1 = 1.0f - powf(b1, (float)c->step), bc2 = 1.0f - powf(b2, (float)c->step);
-    hipLaunchKernelGGL(k_adam, g1(c->nparam), dim3(256), 0, c->stream, c->p, c->g, c->m, c->v, c->pb, c->mask,
-                       c->nparam, lr, b1, b2, eps, bc1, bc2, wd);
-    c->wver++;
+    hipLaunchKernelGGL(k_adam, g1(c->nparam), dim3(256), 0, c->stream, c->p, c->g, c->m, c->v, c->forms, c->mask,
+                       (int)c->nparam, lr, b1, b2, eps, bc1, bc2, wd);
     return launch_check("adam");
 }
 

@@ -224,3 +224,91 @@ def test_split_head_equals_one_launch_head():
         assert np.array_equal(net.infer(x).cpu().numpy(), one)
         assert np.array_equal(net.infer(x[:1].contiguous()).cpu().numpy(), one1)
     net.close()
+
+
+def captured(net, x, target, adam):
+    """A graph of forward, inference and backward (and an Adam step) on the
+    net's own stream, after a first pass of each, with its outputs."""
+    import torch
+    stream = torch.cuda.Stream()
+    net.set_stream(stream.cuda_stream)
+    out, inf = (torch.empty(x.shape[0], 6, device="cuda") for _ in range(2))
+
+    def step():
+        net.forward(x, out)
+        net.infer(x, inf)
+        net.backward(x.shape[0], target)
+        if adam:
+            net.adam(1e-3)
+
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        step()
+
+    def replay():
+        with torch.cuda.stream(stream):
+            graph.replay()
+        torch.cuda.synchronize()
+        return out.cpu().numpy(), inf.cpu().numpy(), net.get_grads()
+
+    return replay
+
+
+def eager(flat, x, target):
+    from slam_amd.warmstart import WarmStartNet
+    net = WarmStartNet(max_batch=x.shape[0])
+    net.set_params(flat)
+    out, inf = net.forward(x).cpu().numpy(), net.infer(x).cpu().numpy()
+    net.backward(x.shape[0], target)
+    return out, inf, net.get_grads()
+
+
+@pytest.mark.parametrize("warm", [False, True])
+def test_captured_calls_use_the_present_weights(setup, warm):
+    """Weights set after the capture (before it: a first pass, or none) are
+    those of the next replay, and an eager pass between capture and replay has
+    them too: bit for bit the eager calls of another net."""
+    import torch
+    from slam_amd.warmstart import WarmStartNet, he_init
+    x, target = setup["xt"], torch.from_numpy(setup["target"]).cuda()
+    net = WarmStartNet(max_batch=4)
+    weights = [he_init(net.layout, net.nparam, seed) for seed in (21, 22, 23)]
+    net.set_params(weights[0])
+    if warm:
+        net.forward(x)
+        net.infer(x)
+    replay = captured(net, x, target, adam=False)
+    torch.cuda.synchronize()
+    ref = eager(weights[0], x, target)
+    net.forward(x)
+    inf = net.infer(x)
+    torch.cuda.synchronize()
+    assert np.array_equal(inf.cpu().numpy(), ref[1])
+    for flat in weights + weights[:1]:
+        net.set_params(flat)
+        ref = eager(flat, x, target)
+        for _ in range(2):
+            for mine, theirs in zip(replay(), ref):
+                assert np.array_equal(mine, theirs)
+
+
+def test_replayed_training_steps_move_the_weights_of_later_calls(setup):
+    """Adam steps inside a graph: each replay, and eager calls between the
+    replays, work with the weights that the last step left."""
+    import torch
+    from slam_amd.warmstart import WarmStartNet
+    x, target = setup["xt"], torch.from_numpy(setup["target"]).cuda()
+    net = WarmStartNet(max_batch=4)
+    net.init_params(seed=24)
+    replay = captured(net, x, target, adam=True)
+    for _ in range(3):
+        before = net.get_params()
+        got, ref = replay(), eager(before, x, target)
+        for mine, theirs in zip(got, ref):
+            assert np.array_equal(mine, theirs)
+        ref = eager(net.get_params(), x, target)
+        assert not np.array_equal(got[0], ref[0])
+        out, inf = net.forward(x), net.infer(x)
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), ref[0]) and np.array_equal(inf.cpu().numpy(), ref[1])
