@@ -59,7 +59,9 @@ int efloop_destroy(efloop_handle h);
 int efloop_process(efloop_handle h, const odom_frame_view *rgb, const odom_frame_view *depth, float pose_out[16]);
 
 /* The loop's components (owned by the loop), its frame count and the last
- * fusion weighting. */
+ * fusion weighting.  surfel_set_stream and splat_set_stream may move a
+ * component to another stream between frames: the loop orders its stages over
+ * the streams with events. */
 int efloop_get_handles(efloop_handle h, odom_handle *odom, splat_handle *prediction, surfel_handle *model);
 int efloop_get_state(efloop_handle h, int *tick, float *last_weighting, float *last_icp_error);
 

@@ -24,6 +24,7 @@ struct efloop_ctx {
     uint16_t* filtered = nullptr;    // device, the bilateral output
     slam::HostStage uploads;         // host frames: each is copied to the device once
     uint8_t *dev_rgb = nullptr, *dev_depth = nullptr;
+    hipEvent_t order = nullptr;      // between the components' streams, where they differ
     float pose[16];
     float last_pose[16];
     int tick = 0;
@@ -41,7 +42,27 @@ void free_loop(efloop_ctx* c)
     if (c->odo) odom_destroy(c->odo);
     for (void* p : {(void*)c->filtered, (void*)c->dev_rgb, (void*)c->dev_depth})
         if (p) (void)hipFree(p);
+    if (c->order) (void)hipEventDestroy(c->order);
     delete c;
+}
+
+hipStream_t odom_stream(const efloop_ctx* c)
+{
+    void* s = nullptr;
+    (void)odom_get_stream(c->odo, &s);
+    return (hipStream_t)s;
+}
+
+// What `b` is given from here on runs after what `a` has been given so far.
+// The components share the odometry's stream, but surfel_set_stream and
+// splat_set_stream may have moved theirs, and then no host wait orders the
+// cleaning and the prediction, or a frame's copies and their readers.
+int order(efloop_ctx* c, hipStream_t a, hipStream_t b)
+{
+    if (a == b) return ODOM_OK;
+    if (hipEventRecord(c->order, a) != hipSuccess || hipStreamWaitEvent(b, c->order, 0) != hipSuccess)
+        return ODOM_ERR_HIP;
+    return ODOM_OK;
 }
 
 odom_frame_view device_view(const void* p, int w, int h, int bpp, int fmt)
@@ -59,13 +80,11 @@ int to_device(efloop_ctx* c, const odom_frame_view* v, int fmt, int bpp, uint8_t
     if (v->mem != ODOM_MEM_HOST || !v->ptr || v->format != fmt || v->width != c->w || v->height != c->h ||
         v->pitch_bytes < 0 || pitch < row || pitch % (bpp == 2 ? 2 : 1) != 0)
         return ODOM_OK;
-    void* stream = nullptr;
-    if (int rc = odom_get_stream(c->odo, &stream)) return rc;
     if (!*buf && hipMalloc((void**)buf, row * c->h) != hipSuccess) {
         *buf = nullptr;
         return ODOM_ERR_HIP;
     }
-    if (c->uploads.upload(*buf, v->ptr, pitch, row, c->h, (hipStream_t)stream) != hipSuccess) return ODOM_ERR_HIP;
+    if (c->uploads.upload(*buf, v->ptr, pitch, row, c->h, odom_stream(c)) != hipSuccess) return ODOM_ERR_HIP;
     *out = device_view(*buf, c->w, c->h, bpp, fmt);
     return ODOM_OK;
 }
@@ -100,7 +119,10 @@ double motion(const float cur[16], const float last[16])
 int loop_begin_frame(efloop_ctx* c, odom_frame_view* rgb, odom_frame_view* depth, bool* first)
 {
     const efloop_params& p = c->p;
-    int rc = to_device(c, depth, ODOM_FMT_DEPTH_U16, 2, &c->dev_depth, depth);
+    // the frame overwrites what the last one's update and fill-in read
+    int rc = order(c, slam::surfel_stream(c->model), odom_stream(c));
+    if (!rc) rc = order(c, slam::splat_stream(c->pred), odom_stream(c));
+    if (!rc) rc = to_device(c, depth, ODOM_FMT_DEPTH_U16, 2, &c->dev_depth, depth);
     if (rc) return rc;
     rc = odom_bilateral_depth(c->odo, depth, p.depth_cutoff, c->filtered, ODOM_MEM_DEVICE);
     if (rc) return rc;
@@ -109,6 +131,7 @@ int loop_begin_frame(efloop_ctx* c, odom_frame_view* rgb, odom_frame_view* depth
     *first = c->tick == 1;
     if (*first) {
         rc = to_device(c, rgb, ODOM_FMT_RGB8, 3, &c->dev_rgb, rgb);
+        if (!rc) rc = order(c, odom_stream(c), slam::surfel_stream(c->model));
         if (!rc) rc = surfel_initialise(c->model, rgb, depth, &filt, p.depth_cutoff, c->tick, p.max_depth);
         if (!rc) rc = odom_init_first_rgb(c->odo, rgb);
         return rc;
@@ -151,7 +174,8 @@ int loop_after_tracking(efloop_ctx* c, const odom_frame_view* rgb, const odom_fr
     if (!c->tracking_ok) return ODOM_OK;
     const odom_frame_view filt = device_view(c->filtered, c->w, c->h, 2, ODOM_FMT_DEPTH_U16);
     const int tick = c->tick;
-    int rc = surfel_predict_indices(c->model, c->pose, tick, p.max_depth, p.time_delta);
+    int rc = order(c, odom_stream(c), slam::surfel_stream(c->model));
+    if (!rc) rc = surfel_predict_indices(c->model, c->pose, tick, p.max_depth, p.time_delta);
     if (!rc)
         rc = surfel_fuse(c->model, c->pose, tick, rgb, depth, &filt, p.depth_cutoff, p.max_depth, c->weighting);
     if (!rc) rc = surfel_predict_indices(c->model, c->pose, tick, p.max_depth, p.time_delta);
@@ -171,8 +195,10 @@ int loop_predict(efloop_ctx* c, const odom_frame_view* rgb)
     const int* dev_n;
     int n = 0;
     slam::surfel_model_enqueued(c->model, &mp, &n, &dev_n);
-    int rc = slam::splat_predict_counted(c->pred, c->pose, mp, n, dev_n, p.max_depth, p.confidence, c->tick, c->tick,
-                                         p.time_delta);
+    int rc = order(c, odom_stream(c), slam::splat_stream(c->pred));
+    if (!rc) rc = order(c, slam::surfel_stream(c->model), slam::splat_stream(c->pred));
+    if (!rc) rc = slam::splat_predict_counted(c->pred, c->pose, mp, n, dev_n, p.max_depth, p.confidence, c->tick,
+                                              c->tick, p.time_delta);
     if (!rc) rc = splat_fill_in(c->pred, &filt, rgb, 0, 0);
     return rc;
 }
@@ -220,6 +246,7 @@ int efloop_create(int width, int height, float cx, float cy, float fx, float fy,
     if (!rc) rc = surfel_set_stream(c->model, stream);
     if (!rc && p->use_graph) rc = odom_set_graph(c->odo, 1);
     if (!rc && hipMalloc((void**)&c->filtered, (size_t)width * height * 2) != hipSuccess) rc = ODOM_ERR_HIP;
+    if (!rc && hipEventCreateWithFlags(&c->order, hipEventDisableTiming) != hipSuccess) rc = ODOM_ERR_HIP;
     for (int k = 0; k < 16; ++k) c->pose[k] = (k % 5 == 0) ? 1.0f : 0.0f;
     if (!rc) {
         const float t[3] = {0.0f, 0.0f, 0.0f};

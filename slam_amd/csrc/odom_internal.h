@@ -30,6 +30,10 @@ void surfel_model_enqueued(surfel_handle c, const float** dev_ptr, int* upper, c
 int splat_predict_counted(splat_handle c, const float pose[16], const float* model, int n, const int* dev_count,
                           float depth_cutoff, float conf_threshold, int time, int max_time, int time_delta);
 
+// The streams that the handles' work goes to.
+hipStream_t surfel_stream(surfel_handle c);
+hipStream_t splat_stream(splat_handle c);
+
 // Launch shape of a step kernel at one level (replaces GPUConfig.h's
 // threads/blocks table; chosen by the autotuner).
 struct StepShape {

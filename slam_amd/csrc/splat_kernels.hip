@@ -783,4 +783,6 @@ int splat_predict_counted(splat_handle c, const float pose[16], const float* mod
     return enqueue_predict(c, U, model, n, dev_count, false);
 }
 
+hipStream_t splat_stream(splat_handle c) { return c->stream; }
+
 }  // namespace slam

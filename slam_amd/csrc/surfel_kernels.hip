@@ -1437,4 +1437,6 @@ void surfel_model_enqueued(surfel_handle c, const float** dev_ptr, int* upper, c
     *dev_count = c->pending ? c->totals : nullptr;
 }
 
+hipStream_t surfel_stream(surfel_handle c) { return c->stream; }
+
 }  // namespace slam
