@@ -14,8 +14,10 @@
  *   every frame: the prediction and fill-in for the next one (predict()).
  * The prediction the reference makes right after tracking (:399) feeds only
  * the loop-closure search and is not made.  All work runs on the odometry's
- * stream; the call waits where the reference reads results on the host (the
- * pose and the surfel count).  Part of libslam_odom.so.
+ * stream.  The call waits for the pose; the surfel count stays on the device
+ * until surfel_count or another call asks for it, and the cleaning and the
+ * prediction may still run when the call returns (an error of theirs is
+ * reported by the next call).  Part of libslam_odom.so.
  */
 #ifndef SLAM_LOOP_H
 #define SLAM_LOOP_H
@@ -55,7 +57,10 @@ int efloop_create(int width, int height, float cx, float cy, float fx, float fy,
 int efloop_destroy(efloop_handle h);
 
 /* One frame: depth ODOM_FMT_DEPTH_U16 (mm), colour ODOM_FMT_RGB8, host or
- * device.  pose_out: the tracked camera-to-model pose, 4x4 row-major. */
+ * device.  pose_out: the tracked camera-to-model pose, 4x4 row-major.  Host
+ * images and a device depth image may be overwritten or freed as soon as the
+ * call returns; a device colour image, which the fill-in reads last, once the
+ * loop's next call has returned or its odometry's stream was synchronised. */
 int efloop_process(efloop_handle h, const odom_frame_view *rgb, const odom_frame_view *depth, float pose_out[16]);
 
 /* The loop's components (owned by the loop), its frame count and the last

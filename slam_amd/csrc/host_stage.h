@@ -14,6 +14,8 @@
 
 #include <algorithm>
 
+#include "host_wait.h"
+
 namespace slam {
 
 class HostStage {
@@ -69,15 +71,6 @@ private:
         bool used = false;
     };
 
-    static hipError_t wait(Slot& q)
-    {
-        for (;;) {
-            const hipError_t e = hipEventQuery(q.ev);
-            if (e != hipErrorNotReady) return e;
-            __builtin_ia32_pause();
-        }
-    }
-
     static hipError_t ready(Slot& q)
     {
         if (!q.pin) {
@@ -93,7 +86,7 @@ private:
             }
         }
         if (!q.used) return hipSuccess;
-        if (hipError_t e = wait(q)) return e;
+        if (hipError_t e = poll_event(q.ev)) return e;
         q.used = false;
         return hipSuccess;
     }

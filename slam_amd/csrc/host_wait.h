@@ -22,4 +22,14 @@ inline hipError_t poll_stream(hipStream_t s)
     }
 }
 
+// The same for an event.
+inline hipError_t poll_event(hipEvent_t ev)
+{
+    for (;;) {
+        const hipError_t e = hipEventQuery(ev);
+        if (e != hipErrorNotReady) return e;
+        __builtin_ia32_pause();
+    }
+}
+
 }  // namespace slam

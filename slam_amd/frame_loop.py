@@ -9,8 +9,11 @@ model update, and the next prediction (elastic_fusion_file.cpp:335-420,
 tracking calls batched and, with the learned start, one network forward for
 all of them; a FrameLoop with any other tracking policy is a batch of one.
 Every stage of a sequence runs on one HIP stream (its odometry's); the host
-reads back only what the reference's loop reads: the tracked pose and the
-model's surfel count.  The prediction that the reference makes right after
+waits for the tracked pose only.  The model's surfel count, which the
+reference's loop reads back too, stays on the device until it is asked for.
+A device colour image is read until the next call has returned, so the loops
+hold on to the last frame's tensors; its contents must not change before then.
+The prediction that the reference makes right after
 tracking (elastic_fusion_file.cpp:399) feeds only the loop-closure search, so
 it is not made; the one at the end of the frame (:601) is.
 """
@@ -180,7 +183,7 @@ class FrameLoop:
     def close(self) -> None:
         if getattr(self, "_h", None):
             lib().efloop_destroy(self._h)
-            self._h = None
+            self._h = self._keep = None
 
     def __del__(self):
         try:
@@ -193,7 +196,12 @@ class FrameLoop:
         r, kr = frame_view(rgb, FMT_RGB8)
         d, kd = frame_view(depth, FMT_DEPTH_U16)
         pose = np.zeros(16, np.float32)
-        _check("efloop_process", lib().efloop_process(self._h, ctypes.byref(r), ctypes.byref(d), _p(pose)))
+        last, self._keep = getattr(self, "_keep", None), (kr, kd)
+        try:
+            _check("efloop_process", lib().efloop_process(self._h, ctypes.byref(r), ctypes.byref(d), _p(pose)))
+        except Exception:
+            self._keep += (last,)        # a failed call may not have waited
+            raise
         T = pose.reshape(4, 4)
         self.poses.append(T.copy())
         return T
@@ -237,7 +245,7 @@ class BatchFrameLoop:
     def close(self) -> None:
         if getattr(self, "_h", None):
             lib().efloop_batch_destroy(self._h)
-            self._h = None
+            self._h = self._keep = None
 
     def __del__(self):
         try:
@@ -255,7 +263,12 @@ class BatchFrameLoop:
             rv[i], dv[i] = r, d
             keep += [kr, kd]
         out = np.zeros((self.n, 16), np.float32)
-        _check("efloop_batch_process", lib().efloop_batch_process(self._h, rv, dv, _p(out)))
+        last, self._keep = getattr(self, "_keep", None), keep
+        try:
+            _check("efloop_batch_process", lib().efloop_batch_process(self._h, rv, dv, _p(out)))
+        except Exception:
+            self._keep = keep + [last]   # a failed call may not have waited
+            raise
         poses = [out[i].reshape(4, 4).copy() for i in range(self.n)]
         for i, T in enumerate(poses):
             self.poses[i].append(T)

@@ -1,14 +1,15 @@
 """Frames in host memory reach the device through pinned slots of 1 MiB: the
 device's copy has the host's bytes for row pitches with and without padding and
 for images below, at and above a slot, and the caller's memory is free as soon
-as the call returns."""
+as the call returns.  A device frame's depth is too, and the Python loops hold
+on to its colour until the next call."""
 import ctypes
 
 import numpy as np
 import pytest
 
 from slam_amd import synth
-from slam_amd.frame_loop import FrameLoop, LoopParams
+from slam_amd.frame_loop import BatchFrameLoop, FrameLoop, LoopParams
 from slam_amd.odometry import FMT_RGBA32F, MEM_HOST, FrameView, RGBDOdometry, lib
 
 pytestmark = pytest.mark.gpu
@@ -56,3 +57,35 @@ def test_loop_over_host_frames_equals_device_frames():
         b = dev.process(torch.from_numpy(f.rgb).cuda(), torch.from_numpy(f.depth).cuda())
         assert np.array_equal(a, b)
     assert np.array_equal(host.model.model().view(np.uint32), dev.model.model().view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [1, 3])
+def test_loop_leaves_device_frames_alone_after_the_call(n):
+    """Depth tensors are overwritten as soon as the call returns, colour
+    tensors are dropped and their size is allocated and filled again."""
+    import torch
+    cam = synth.CAM_640
+    scene = synth.Scene(9)
+    poses = synth.spline_trajectory(5, seed=9, max_step_m=0.01, max_step_deg=0.5)
+    frames = [scene.render(T, cam, noise_seed=k, model=False) for k, T in enumerate(poses)]
+    args = (cam.width, cam.height, cam.cx, cam.cy, cam.fx, cam.fy)
+    p = LoopParams(max_surfels=1_500_000)
+    make = (lambda: FrameLoop(*args, p)) if n == 1 else (lambda: BatchFrameLoop(n, *args, p))
+    host, dev = make(), make()
+    for f in frames:
+        rgbs = [torch.from_numpy(f.rgb).cuda() for _ in range(n)]
+        depths = [torch.from_numpy(f.depth).cuda() for _ in range(n)]
+        torch.cuda.synchronize()
+        if n == 1:
+            a, b = host.process(f.rgb, f.depth), dev.process(rgbs[0], depths[0])
+        else:
+            a, b = host.process([f.rgb] * n, [f.depth] * n), dev.process(rgbs, depths)
+        for d in depths:
+            d.fill_(1000)
+        del rgbs
+        again = [torch.full(f.rgb.shape, 77, dtype=torch.uint8, device="cuda") for _ in range(2 * n)]
+        assert np.array_equal(np.asarray(a), np.asarray(b))
+        del again
+    models = [(host.model, dev.model)] if n == 1 else list(zip(host.models, dev.models))
+    for x, y in models:
+        assert np.array_equal(x.model().view(np.uint32), y.model().view(np.uint32))
