@@ -98,21 +98,17 @@ odom_frame_view device_view(const void* p, int w, int h, int bpp, int fmt)
 }
 
 // The frame `v` of `bpp` bytes a pixel for the frame's stages: a host frame is
-// copied to `buf` (allocated on first use), once for all of them.  A view that
+// copied to `buf`, once for all of them.  A view that
 // the stages would refuse stays as it is, for them to refuse.
-int to_device(efloop_ctx* c, const odom_frame_view* v, int fmt, int bpp, uint8_t** buf, odom_frame_view* out)
+int to_device(efloop_ctx* c, const odom_frame_view* v, int fmt, int bpp, uint8_t* buf, odom_frame_view* out)
 {
     *out = *v;
     const size_t row = (size_t)c->w * bpp, pitch = v->pitch_bytes ? v->pitch_bytes : row;
     if (v->mem != ODOM_MEM_HOST || !v->ptr || v->format != fmt || v->width != c->w || v->height != c->h ||
         v->pitch_bytes < 0 || pitch < row || pitch % (bpp == 2 ? 2 : 1) != 0)
         return ODOM_OK;
-    if (!*buf && hipMalloc((void**)buf, row * c->h) != hipSuccess) {
-        *buf = nullptr;
-        return ODOM_ERR_HIP;
-    }
-    if (c->uploads.upload(*buf, v->ptr, pitch, row, c->h, odom_stream(c)) != hipSuccess) return ODOM_ERR_HIP;
-    *out = device_view(*buf, c->w, c->h, bpp, fmt);
+    if (c->uploads.upload(buf, v->ptr, pitch, row, c->h, odom_stream(c)) != hipSuccess) return ODOM_ERR_HIP;
+    *out = device_view(buf, c->w, c->h, bpp, fmt);
     return ODOM_OK;
 }
 
@@ -150,7 +146,7 @@ int loop_begin_frame(efloop_ctx* c, odom_frame_view* rgb, odom_frame_view* depth
     // the frame overwrites what the last one's update and fill-in read
     int rc = order(c, slam::surfel_stream(c->model), odom_stream(c));
     if (!rc) rc = order(c, slam::splat_stream(c->pred), odom_stream(c));
-    if (!rc) rc = to_device(c, depth, ODOM_FMT_DEPTH_U16, 2, &c->dev_depth, depth);
+    if (!rc) rc = to_device(c, depth, ODOM_FMT_DEPTH_U16, 2, c->dev_depth, depth);
     if (rc) return rc;
     rc = odom_bilateral_depth(c->odo, depth, p.depth_cutoff, c->filtered, ODOM_MEM_DEVICE);
     if (rc) return rc;
@@ -158,7 +154,7 @@ int loop_begin_frame(efloop_ctx* c, odom_frame_view* rgb, odom_frame_view* depth
     c->tick += 1;
     *first = c->tick == 1;
     if (*first) {
-        rc = to_device(c, rgb, ODOM_FMT_RGB8, 3, &c->dev_rgb, rgb);
+        rc = to_device(c, rgb, ODOM_FMT_RGB8, 3, c->dev_rgb, rgb);
         if (!rc) rc = order(c, odom_stream(c), slam::surfel_stream(c->model));
         if (!rc) rc = surfel_initialise(c->model, rgb, depth, &filt, p.depth_cutoff, c->tick, p.max_depth);
         if (!rc) rc = odom_init_first_rgb(c->odo, rgb);
@@ -177,7 +173,7 @@ int loop_begin_frame(efloop_ctx* c, odom_frame_view* rgb, odom_frame_view* depth
     rc = odom_init_icp_model(c->odo, &vv, &nv, p.max_depth, c->pose);
     if (!rc) rc = odom_init_rgb_model(c->odo, &iv);
     if (!rc) rc = odom_init_icp_depth(c->odo, &filt, p.max_depth);
-    if (!rc) rc = to_device(c, rgb, ODOM_FMT_RGB8, 3, &c->dev_rgb, rgb);
+    if (!rc) rc = to_device(c, rgb, ODOM_FMT_RGB8, 3, c->dev_rgb, rgb);
     if (!rc) rc = odom_init_rgb(c->odo, rgb);
     return rc;
 }
@@ -274,7 +270,11 @@ int efloop_create(int width, int height, float cx, float cy, float fx, float fy,
     if (!rc) rc = splat_set_stream(c->pred, stream);
     if (!rc) rc = surfel_set_stream(c->model, stream);
     if (!rc && p->use_graph) rc = odom_set_graph(c->odo, 1);
-    if (!rc && hipMalloc((void**)&c->filtered, (size_t)width * height * 2) != hipSuccess) rc = ODOM_ERR_HIP;
+    const size_t npix = (size_t)width * height;
+    if (!rc && (hipMalloc((void**)&c->filtered, npix * 2) != hipSuccess ||
+                hipMalloc((void**)&c->dev_rgb, npix * 3) != hipSuccess ||
+                hipMalloc((void**)&c->dev_depth, npix * 2) != hipSuccess || c->uploads.create() != hipSuccess))
+        rc = ODOM_ERR_HIP;
     for (hipEvent_t* e : {&c->order, &c->fused})
         if (!rc && hipEventCreateWithFlags(e, hipEventDisableTiming) != hipSuccess) rc = ODOM_ERR_HIP;
     for (int k = 0; k < 16; ++k) c->pose[k] = (k % 5 == 0) ? 1.0f : 0.0f;

@@ -4,8 +4,11 @@
 // row: one 640x480 colour image took about 4.6 ms, and the frame loop made
 // five such copies per frame (23 ms of a 23 ms frame).  Here the host copies
 // the rows into one of two pinned slots and enqueues the slot's copy, so the
-// caller's memory is free on return, the host does not wait for the device,
-// and one slot fills while the other is in flight.
+// caller's memory is free on return and one slot fills while the other is in
+// flight.  The host waits only for a slot: an image of up to two slots does not
+// wait for the device unless the images before it are still on their way, but
+// the third slot of a larger one waits until the first has been copied, and so
+// for the work queued ahead of it.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -26,10 +29,27 @@ public:
     // The owner has synchronised the streams of its uploads.
     ~HostStage()
     {
-        for (auto& s : slots_) {
+        for (auto& s : slots_)
             if (s.ev) (void)hipEventDestroy(s.ev);
-            if (s.pin) (void)hipHostFree(s.pin);
+        if (pin_) (void)hipHostFree(pin_);
+    }
+
+    // The slots (2 MiB of pinned memory, about 50 us), with the owner's other
+    // memory, so that no upload allocates.
+    hipError_t create()
+    {
+        if (hipError_t e = hipHostMalloc((void**)&pin_, 2 * kSlot, hipHostMallocDefault)) {
+            pin_ = nullptr;
+            return e;
         }
+        for (int k = 0; k < 2; ++k) {
+            slots_[k].pin = pin_ + k * kSlot;
+            if (hipError_t e = hipEventCreateWithFlags(&slots_[k].ev, hipEventDisableTiming)) {
+                slots_[k].ev = nullptr;
+                return e;
+            }
+        }
+        return hipSuccess;
     }
 
     // rows x row bytes at `src` (pitch bytes apart) to contiguous device
@@ -73,24 +93,13 @@ private:
 
     static hipError_t ready(Slot& q)
     {
-        if (!q.pin) {
-            if (hipError_t e = hipHostMalloc((void**)&q.pin, kSlot, hipHostMallocDefault)) {
-                q.pin = nullptr;
-                return e;
-            }
-        }
-        if (!q.ev) {
-            if (hipError_t e = hipEventCreateWithFlags(&q.ev, hipEventDisableTiming)) {
-                q.ev = nullptr;
-                return e;
-            }
-        }
         if (!q.used) return hipSuccess;
         if (hipError_t e = poll_event(q.ev)) return e;
         q.used = false;
         return hipSuccess;
     }
 
+    uint8_t* pin_ = nullptr;
     Slot slots_[2];
     int next_ = 0;
 };

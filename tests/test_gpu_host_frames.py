@@ -89,3 +89,24 @@ def test_loop_leaves_device_frames_alone_after_the_call(n):
     models = [(host.model, dev.model)] if n == 1 else list(zip(host.models, dev.models))
     for x, y in models:
         assert np.array_equal(x.model().view(np.uint32), y.model().view(np.uint32))
+
+
+def test_host_frames_allocate_no_device_memory():
+    """The loop's and the handles' memory is theirs from create on: the first
+    host frames take none."""
+    import torch
+    w, h = 1920, 1080
+    args = (w, h, w / 2.0, h / 2.0, 0.8 * w, 0.8 * w)
+    rgb = np.full((h, w, 3), 90, np.uint8)
+    depth = np.full((h, w), 1500, np.uint16)
+    loop, odo = FrameLoop(*args, LoopParams(max_surfels=3_000_000, use_graph=False)), RGBDOdometry(*args)
+    warm = FrameLoop(64, 48, 32.0, 24.0, 50.0, 50.0, LoopParams(max_surfels=10_000, use_graph=False))
+    for _ in range(2):                       # the runtime's own pools
+        warm.process(rgb[:48, :64].copy(), depth[:48, :64].copy())
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    odo.initFirstRGB(rgb)
+    for _ in range(2):
+        loop.process(rgb, depth)
+    torch.cuda.synchronize()
+    assert torch.cuda.mem_get_info()[0] == free
