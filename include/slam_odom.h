@@ -276,8 +276,9 @@ int odom_batch_get_step_shape(odom_batch b, int kernel, int level, int *threads,
 int odom_batch_autotune(odom_batch b, int rgb_only, float icp_weight);
 /* 1 (default): each iteration's solve runs once per pair in a kernel of its
  * own before the ICP pass; 0: every block of the ICP pass repeats it in its
- * prologue (the single-pair form) as long as the launch's blocks run at once.
- * The same results either way. */
+ * prologue (the single-pair form) where the launch has at most two rounds of
+ * blocks (two times 512 threads per compute unit), and the solve is a kernel
+ * of its own past that.  The same results either way. */
 int odom_batch_set_split_solve(odom_batch b, int enable);
 /* Capture each distinct call (options and image parities) as a hipGraph on
  * first use and replay it afterwards. */

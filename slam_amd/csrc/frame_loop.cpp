@@ -353,10 +353,12 @@ int efloop_get_state(efloop_handle c, int* tick, float* last_weighting, float* l
 // prediction, odometry handle and stream); their tracking calls run as one
 // batched call per frame (odom_track_batch_policy), with the learned start's
 // network input and forward for all n sequences in one launch each on the
-// batch's stream.  Every sequence's launches are those of the same sequence
-// tracked alone (a batch of one): the batch gives each pair the block count
-// of a single-pair call and the handles' launch shapes, and the network's
-// inference (one workgroup per sample) is the same for a sample in any batch.
+// batch's stream.  Every sequence's sums are those of the same sequence tracked
+// alone (a batch of one): the batch gives each pair the block count of a
+// single-pair call and the handles' launch shapes (the solve moves to a launch
+// of its own where many sequences fill the card, with the same bits), and the
+// network's inference (one workgroup per sample) is the same for a sample in
+// any batch.
 struct efloop_batch_s {
     std::vector<efloop_ctx*> loops;
     odom_batch batch = nullptr;
@@ -399,7 +401,7 @@ int efloop_batch_create(int n, int width, int height, float cx, float cy, float 
     std::vector<odom_handle> hs(n);
     for (int i = 0; i < n && !rc; ++i) hs[i] = b->loops[i]->odo;
     if (!rc) rc = odom_batch_create(hs.data(), n, &b->batch);
-    // the single-pair call's block counts, shapes and fused prologue
+    // the single-pair call's block counts and shapes, and its fused prologue up to two rounds of blocks
     if (!rc) rc = odom_batch_set_blocks(b->batch, 0);
     for (int k = 0; k < 2 && !rc; ++k)
         for (int l = 0; l < 3 && !rc; ++l) {

@@ -1293,11 +1293,12 @@ struct odom_batch_s {
     hipEvent_t done = nullptr;
     std::vector<hipEvent_t> ready;
     int target_blocks = 0;           // 0: each entry gets its single-call block count
+    int cus = 256;                   // the device's compute units
     StepShape shape[2][kLevels];
     BatchPlan plan[kMaxHyp];         // plan[k]: k + 1 entries per handle
     PairDesc* h_stage = nullptr;     // pinned upload buffer (kMaxHyp entries per handle)
     bool use_graph = false;
-    bool split_solve = true;         // k_solve + unfused pass A (else the fused prologue in every block)
+    bool split_solve = true;         // k_solve + unfused pass A (else the fused prologue, up to two rounds of blocks)
     int so3_spin = kSO3SpinDefault;  // the SO3 loop setting of the batch's first handle
     struct G { std::vector<int> key; hipGraphExec_t exec; };
     std::vector<G> graphs;
@@ -1459,6 +1460,18 @@ StepLaunch plan_launch(odom_batch_s* b, int hyp, PairDesc* dp, int kernel, int l
     return L;
 }
 
+// Where the fused prologue ends: its registers leave one workgroup of 512
+// threads (or two of 256) on a CU, and each further round of workgroups
+// repeats the whole solve.  Past two rounds the solve is a launch of its own
+// and the pass without it runs several workgroups per CU.  Pass A with its
+// solve, fused and split, 1 to 12 pairs of 320x240 to 1920x1080 at the single
+// pair's shapes: up to one round 9.9-32.7 us fused and 11.7-34.4 split; from
+// one to two 14-60 us, within 12 % either way; past two rounds the split form
+// wins everywhere (2.2-2.3 rounds: 41.7 against 34.7 at 848x480, 35.8 against
+// 29.1 at 640x480, 20.8 against 16.8 at 320x240; 8 to 9 rounds: 110 against 74).
+// The same bits either way.
+constexpr int kFusedPerCu = 512;
+
 // The launches of one batched getIncrementalTransformation (the sequence of
 // enqueue_track over every pair at once), with the start and judge of a
 // policy call.  dp[k]: the descriptor array of plan k + 1 (dp[1] only for
@@ -1466,15 +1479,6 @@ StepLaunch plan_launch(odom_batch_s* b, int hyp, PairDesc* dp, int kernel, int l
 // done: the last of them is finished for both refinements (k_solve), the
 // judge keeps one state per handle, and the finer levels continue with one
 // entry per handle (their first pass A reads the state the solve stored).
-// Where the fused prologue ends: its registers leave one workgroup of 512
-// threads (or two of 256) on a CU, and each further round of workgroups
-// repeats the whole solve (8 sequences at 640x480, level 0: 64 us for 1 600
-// workgroups, 10 us a round).  Past two rounds the solve is a launch of its
-// own (9 us) and the pass without it runs several workgroups per CU: 8
-// sequences in lockstep 12.0 -> 10.9 ms per 5 frames, 4 sequences 7.4 -> 6.9;
-// at two rounds or fewer the two forms are level.  The same bits either way.
-constexpr int kFusedThreads = 2 * 256 * 512;
-
 void batch_launches(odom_batch_s* b, const CallSpec& cs, PairDesc* const* dp, hipEvent_t* ev)
 {
     const TrackParams& P = cs.P;
@@ -1508,7 +1512,7 @@ void batch_launches(odom_batch_s* b, const CallSpec& cs, PairDesc* const* dp, hi
         if (ev) (void)hipEventRecord(ev[e++], b->stream);
         if (state_ready) {
             launch_step_a(La, level, iter, (int)k, prev, P, 1, nullptr, b->stream);
-        } else if (b->split_solve || La.total_blocks * La.shape.threads > kFusedThreads) {
+        } else if (b->split_solve || La.total_blocks * La.shape.threads > 2 * b->cus * kFusedPerCu) {
             launch_solve(cur, n * hyp, level, iter, (int)k, prev, P, La.shape.threads, b->stream);
             launch_step_a(La, level, iter, (int)k, prev, P, 1, nullptr, b->stream);
         } else {
@@ -1664,8 +1668,8 @@ int policy_spec(odom_ctx* c0, const float* pred, float t_scale, float r_scale, c
 int batch_new(const odom_handle* handles, int n, bool own_stream, odom_batch_s** out);
 
 // The handle's own batch of one for its policy calls: the handle's stream,
-// shapes and graph setting, the single-call block counts and the fused
-// prologue, so its launches are those of odom_track_async.
+// shapes and graph setting, the single-call block counts and (up to two rounds
+// of workgroups) the fused prologue, so its sums are those of odom_track_async.
 int self_batch(odom_ctx* c, odom_batch_s** out)
 {
     if (!c->self_batch) {
@@ -1695,14 +1699,12 @@ int batch_new(const odom_handle* handles, int n, bool own_stream, odom_batch_s**
     b->h.assign(handles, handles + n);
     b->own_stream = own_stream;
     b->so3_spin = handles[0]->so3_spin;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+        b->cus = cus;
     if (own_stream) {
-        int dev = 0, cus = 256;
-        if (hipGetDevice(&dev) == hipSuccess) {
-            hipDeviceProp_t prop;
-            if (hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0)
-                cus = prop.multiProcessorCount;
-        }
-        b->target_blocks = 4 * cus;
+        b->target_blocks = 4 * b->cus;
         for (int k = 0; k < 2; ++k)
             for (int l = 0; l < kLevels; ++l) b->shape[k][l] = batch_shape(k, l);
     } else {
