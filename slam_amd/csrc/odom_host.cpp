@@ -1487,10 +1487,15 @@ void batch_launches(odom_batch_s* b, const CallSpec& cs, PairDesc* const* dp, hi
     PairDesc* cur = dp[hyp - 1];
     if (cs.policy_start) launch_seed_policy(cur, n * hyp, hyp, cs.pred, cs.t_scale, cs.r_scale, b->stream);
     // the pairs' derivatives and source masks (once for both refinements)
-    int groups[kLevels] = {0, 0, 0};
-    for (const auto* c : b->h)
-        for (int l = 0; l < kLevels; ++l) groups[l] = std::max(groups[l], (c->w[l] + 3) / 4 * c->h[l]);
-    if (P.rgb) launch_rgb_prep_pairs(dp[0], n, groups, b->stream);
+    if (P.rgb) {
+        long long pixels = 0;
+        for (const auto* c : b->h) pixels += c->n[0];
+        const int G = rgb_prep_group_size(pixels);
+        int groups[kLevels] = {0, 0, 0};
+        for (const auto* c : b->h)
+            for (int l = 0; l < kLevels; ++l) groups[l] = std::max(groups[l], cdiv(c->w[l], G) * c->h[l]);
+        launch_rgb_prep_pairs(dp[0], n, G, groups, b->stream);
+    }
     if (P.so3) launch_so3(cur, n * hyp, &P, b->so3_spin, b->stream);  // begin rides on the SO3 loop's end
     else launch_track_begin(cur, n * hyp, P, b->stream);
     std::vector<int> sched;

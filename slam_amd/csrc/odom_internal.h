@@ -104,9 +104,11 @@ struct PrepLevels {
     float minScale[kLevels];
 };
 void launch_rgb_prep(const PrepLevels& a, hipStream_t s);
-// The same for every pair; max_groups: the most groups of four pixels of a row
-// that any pair has, per level.
-void launch_rgb_prep_pairs(const PairDesc* pairs, int npairs, const int max_groups[kLevels], hipStream_t s);
+// The same for every pair, G pixels of a row a thread; max_groups: the most
+// groups of G that any pair has, per level.
+void launch_rgb_prep_pairs(const PairDesc* pairs, int npairs, int G, const int max_groups[kLevels], hipStream_t s);
+// G of a launch over so many level-0 pixels (1 or 4).
+int rgb_prep_group_size(long long pixels);
 // The pose (3x4 row-major) that the next call starts from.
 void launch_set_pose(TrackState* st, const float pose[12], hipStream_t s);
 

@@ -737,53 +737,52 @@ void launch_depth_pyramid_maps(const VNLevels& a, hipStream_t s)
 // j < cols-5, i < rows-1, the 4x4 window of nextImage > 0, gradient
 // magnitude >= minScale, nextDepth not NaN).  zsrc = nextDepth where all of
 // them hold, NaN elsewhere.
-__constant__ float c_gsx[9] = {0.52201f, 0.00000f, -0.52201f, 0.79451f, -0.00000f, -0.79451f,
-                               0.52201f, 0.00000f, -0.52201f};
-__constant__ float c_gsy[9] = {0.52201f, 0.79451f, 0.52201f, 0.00000f, 0.00000f, 0.00000f,
-                               -0.52201f, -0.79451f, -0.52201f};
-
-// Pixels 4 g..4 g + 3 of a row, group k of one level.  The 16 texels of a
-// pixel's window hold the nine of its derivatives, and four pixels' windows
-// lie in 8 bytes of each of four rows: one load a row instead of 25 a pixel,
-// which bound the pass (64 pairs of
-// 320x240 to 848x480: 217 us by bytes, 134 so).
-__device__ __forceinline__ int prep_groups(int w) { return (w + 3) / 4; }
-
-// Bytes x..x+7 from the start of row y of an image of n bytes (row length w):
+//
+// G pixels of a row per thread.  The 16 texels of a pixel's window hold the
+// nine of its derivatives, and G pixels' windows lie in 4 (G = 1) or 8 (G = 4)
+// bytes of each of four rows: one load a row instead of 25 a pixel, and a
+// pixel next to the border takes its taps from the same bytes.
+// The bytes of T from column x of row y of an image of n bytes (row length w):
 // any x; bytes outside the image are 0.
-__device__ __forceinline__ uint64_t row8(const uint8_t* __restrict__ img, int n, int w, int y, int x)
+template <class T>
+__device__ __forceinline__ T row_bytes(const uint8_t* __restrict__ img, int n, int w, int y, int x)
 {
-    const int want = y * w + x, at = min(max(want, 0), n - 8);
-    uint64_t v;
-    __builtin_memcpy(&v, img + at, 8);
-    return want < at ? v << (8 * (at - want)) : v >> (8 * min(want - at, 7));
+    constexpr int B = sizeof(T);
+    const int want = y * w + x, at = min(max(want, 0), n - B);
+    T v;
+    __builtin_memcpy(&v, img + at, B);
+    return want < at ? v << (8 * (at - want)) : v >> (8 * min(want - at, B - 1));
 }
 
+// Group k of one level.
+template <int G>
 __device__ __forceinline__ void rgb_prep_group(const uint8_t* __restrict__ img, const float* __restrict__ depth,
                                                short2* __restrict__ dxy, float* __restrict__ zsrc, int w, int h,
                                                float min_scale, int k)
 {
-    const int per_row = prep_groups(w), y = k / per_row, x0 = 4 * (k - y * per_row);
+    static_assert(G == 1 || G == 4, "a pixel, or a 16-byte store");
+    using Row = std::conditional_t<G == 1, uint32_t, uint64_t>;
+    const int per_row = (w + G - 1) / G, y = k / per_row, x0 = G * (k - y * per_row);
     if (y >= h) return;
     // rows y-2..y+1 from column x0-2; a row above the image is not tested, one
     // below it not reached
-    uint64_t r[4];
+    Row r[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) r[j] = row8(img, w * h, w, min(max(y - 2 + j, 0), h - 1), x0 - 2);
+    for (int j = 0; j < 4; ++j) r[j] = row_bytes<Row>(img, w * h, w, min(max(y - 2 + j, 0), h - 1), x0 - 2);
     const size_t o = (size_t)y * w + x0;
-    const bool wide = (w & 3) == 0;     // every row's groups are whole and 16-byte aligned
-    float d[4];
+    const bool wide = G == 4 && (w & 3) == 0;   // every row's groups are whole and 16-byte aligned
+    float d[G];
     if (wide) {
         const float4 v = *(const float4*)(depth + o);
-        d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
+        __builtin_memcpy(d, &v, 4 * G);
     } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) d[i] = depth[o + min(i, w - 1 - x0)];
+        for (int i = 0; i < G; ++i) d[i] = depth[o + min(i, w - 1 - x0)];
     }
-    short2 g[4];
-    float zs[4];
+    short2 g[G];
+    float zs[G];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < G; ++i) {
         const int x = x0 + i;
         const auto tap = [&](int j, int c) { return (int)((r[j] >> (8 * c)) & 0xFFu); };   // row y-2+j, column x0-2+c
         float dxv = 0.0f, dyv = 0.0f;
@@ -804,13 +803,19 @@ __device__ __forceinline__ void rgb_prep_group(const uint8_t* __restrict__ img, 
                     --ki;
                 }
         } else if (x < w) {
+            // a tap outside the image takes no weight from the list
+            const bool rows[3] = {y >= 1, true, y < h - 1}, cols[3] = {x >= 1, true, x < w - 1};
             int ki = 8;
-            for (int j = max(y - 1, 0); j <= min(y + 1, h - 1); j++)
-                for (int c = max(x - 1, 0); c <= min(x + 1, w - 1); c++) {
-                    const float sv = (float)img[(size_t)j * w + c];
-                    dxv = dxv + sv * c_gsx[ki];
-                    dyv = dyv + sv * c_gsy[ki];
-                    --ki;
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    const int kr = (ki >= 3 ? 1 : 0) + (ki >= 6 ? 1 : 0), kc = ki - 3 * kr;
+                    const float mx = kr == 1 ? 0.79451f : 0.52201f, my = kc == 1 ? 0.79451f : 0.52201f;
+                    const float sv = rows[j] && cols[c] ? (float)tap(j + 1, i + 1 + c) : 0.0f;
+                    dxv = dxv + sv * (kc == 0 ? mx : (kc == 2 ? -mx : 0.0f));
+                    dyv = dyv + sv * (kr == 0 ? my : (kr == 2 ? -my : 0.0f));
+                    ki -= rows[j] && cols[c] ? 1 : 0;
                 }
         }
         const short sx = (short)dxv, sy = (short)dyv;
@@ -829,13 +834,15 @@ __device__ __forceinline__ void rgb_prep_group(const uint8_t* __restrict__ img, 
         }
     }
     if (wide) {
-        int4 q;
-        __builtin_memcpy(&q, g, 16);
+        int4 q{};
+        float4 zq{};
+        __builtin_memcpy(&q, g, 4 * G);
+        __builtin_memcpy(&zq, zs, 4 * G);
         *(int4*)(dxy + o) = q;
-        *(float4*)(zsrc + o) = make_float4(zs[0], zs[1], zs[2], zs[3]);
+        *(float4*)(zsrc + o) = zq;
     } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < G; ++i)
             if (x0 + i < w) {
                 dxy[o + i] = g[i];
                 zsrc[o + i] = zs[i];
@@ -843,47 +850,63 @@ __device__ __forceinline__ void rgb_prep_group(const uint8_t* __restrict__ img, 
     }
 }
 
+// G of a launch over so many level-0 pixels.  A small launch waits for one
+// wave's chain of loads and instructions, which four pixels a thread make
+// longer; a large one is bound by its loads and stores, of which they need
+// fewer.  One pixel against four, in us: 160x100 4.8 and 7.6, 333x251 5.1 and
+// 7.2, 842x478 8.1 and 9.1; 640x480 with 848x480 (714k) 11.2 and 10.8,
+// 1280x801 11.4 and 10.3, 1920x1080 18.6 and 15.0, 64 pairs (20M) 194 and 104.
+int rgb_prep_group_size(long long pixels) { return pixels < 600000 ? 1 : 4; }
+
+template <int G>
 __device__ __forceinline__ void rgb_prep_group(const PrepLevels& a, int l, int k)
 {
-    rgb_prep_group(a.img[l], a.depth[l], a.dxy[l], a.zsrc[l], a.w[l], a.h[l], a.minScale[l], k);
+    rgb_prep_group<G>(a.img[l], a.depth[l], a.dxy[l], a.zsrc[l], a.w[l], a.h[l], a.minScale[l], k);
 }
 
-// Groups of every level, as segments of blocks of nt threads.
-Seg3 prep_seg(const int w[kLevels], const int h[kLevels], int nt)
-{
-    int n[kLevels];
-    for (int l = 0; l < kLevels; ++l) n[l] = (w[l] + 3) / 4 * h[l];
-    return make_seg(n, nt);
-}
-
+template <int G>
 __global__ __launch_bounds__(256) void k_rgb_prep(PrepLevels a, Seg3 g)
 {
     const int l = seg_level(g, blockIdx.x);
-    rgb_prep_group(a, l, (blockIdx.x - g.b0[l]) * 256 + threadIdx.x);
+    rgb_prep_group<G>(a, l, (blockIdx.x - g.b0[l]) * 256 + threadIdx.x);
+}
+
+// The segments of one pair's groups, in blocks of nt threads.
+Seg3 prep_seg(const PrepLevels& a, int G, int nt)
+{
+    int n[kLevels];
+    for (int l = 0; l < kLevels; ++l) n[l] = cdiv(a.w[l], G) * a.h[l];
+    return make_seg(n, nt);
 }
 
 void launch_rgb_prep(const PrepLevels& a, hipStream_t s)
 {
-    const Seg3 g = prep_seg(a.w, a.h, 256);
-    hipLaunchKernelGGL(k_rgb_prep, dim3(g.b0[kLevels]), dim3(256), 0, s, a, g);
+    const int G = rgb_prep_group_size((long long)a.w[0] * a.h[0]);
+    const Seg3 g = prep_seg(a, G, 256);
+    const dim3 grid(g.b0[kLevels]);
+    if (G == 1) hipLaunchKernelGGL(k_rgb_prep<1>, grid, dim3(256), 0, s, a, g);
+    else hipLaunchKernelGGL(k_rgb_prep<4>, grid, dim3(256), 0, s, a, g);
 }
 
 // One launch for all pairs of a batch (blockIdx.y): a 640x480 pair by itself
 // fills the card with 1 575 short workgroups for 7 us, mostly launch and
-// drain, and 64 of them took 64 launches (480 us of kernels; 134 us here).
+// drain, and 64 of them took 64 launches (480 us of kernels; 104 us here).
 // A smaller pair's blocks past its own pixels return at once.
+template <int G>
 __global__ __launch_bounds__(256) void k_rgb_prep_pairs(const PairDesc* __restrict__ pairs, Seg3 g)
 {
     const int l = seg_level(g, blockIdx.x);
     const LevelDesc& L = pairs[blockIdx.y].lv[l];
-    rgb_prep_group(L.inext, L.znext, const_cast<short2*>(L.dxy), const_cast<float*>(L.zsrc), L.w, L.h, L.minScale,
-                   (blockIdx.x - g.b0[l]) * 256 + threadIdx.x);
+    rgb_prep_group<G>(L.inext, L.znext, const_cast<short2*>(L.dxy), const_cast<float*>(L.zsrc), L.w, L.h, L.minScale,
+                      (blockIdx.x - g.b0[l]) * 256 + threadIdx.x);
 }
 
-void launch_rgb_prep_pairs(const PairDesc* pairs, int npairs, const int max_groups[kLevels], hipStream_t s)
+void launch_rgb_prep_pairs(const PairDesc* pairs, int npairs, int G, const int max_groups[kLevels], hipStream_t s)
 {
     const Seg3 g = make_seg(max_groups, 256);
-    hipLaunchKernelGGL(k_rgb_prep_pairs, dim3(g.b0[kLevels], npairs), dim3(256), 0, s, pairs, g);
+    const dim3 grid(g.b0[kLevels], npairs);
+    if (G == 1) hipLaunchKernelGGL(k_rgb_prep_pairs<1>, grid, dim3(256), 0, s, pairs, g);
+    else hipLaunchKernelGGL(k_rgb_prep_pairs<4>, grid, dim3(256), 0, s, pairs, g);
 }
 
 // The pose as a kernel argument: a 48-byte copy from the caller's memory costs
@@ -2966,7 +2989,7 @@ __global__ __launch_bounds__(kSO3Threads) void k_so3_loop(const PairDesc* __rest
 {
     if ((int)blockIdx.x >= nloop) {
         const int b = (int)blockIdx.x - nloop, l = seg_level(pseg, b);
-        rgb_prep_group(prep, l, (b - pseg.b0[l]) * kSO3Threads + threadIdx.x);
+        rgb_prep_group<1>(prep, l, (b - pseg.b0[l]) * kSO3Threads + threadIdx.x);
         return;
     }
     __shared__ So3Slot S;
@@ -3096,7 +3119,7 @@ void launch_so3(const PairDesc* pairs, int npairs, const TrackParams* begin, int
         Seg3 g{};
         if (prep) {
             a = *prep;
-            g = prep_seg(a.w, a.h, kSO3Threads);
+            g = prep_seg(a, 1, kSO3Threads);
         }
         hipLaunchKernelGGL(k_so3_loop, dim3(nloop + (prep ? g.b0[kLevels] : 0)), dim3(kSO3Threads), 0, s, pairs,
                            begin ? 1 : 0, P, spin_limit, nloop, a, g);

@@ -1,4 +1,4 @@
-"""Derivatives and source masks, four pixels of a row a thread, and the SO3
+"""Derivatives and source masks, one or four pixels of a row a thread, and the SO3
 sums, four pixels at a time past the first three: widths of every remainder of
 4 on every level, small images, and levels 2 of 3 to 10 pixels a thread,
 against the oracle; and the pairs of a batch (one launch for all) against
@@ -65,6 +65,29 @@ def check_level(img, depth, dxy, zsrc, level):
             ok = x < w - 5 and y < h - 1 and np.all(img[max(y - 2, 0):y + 2, max(x - 2, 0):x + 2] > 0) and \
                 np.float32(int(dx) ** 2 + int(dy) ** 2) >= scale and not np.isnan(depth[y, x])
             assert zsrc[y, x] == depth[y, x] if ok else np.isnan(zsrc[y, x]), (x, y)
+
+
+@pytest.mark.parametrize("w,h,n", [(403, 351, 5), (404, 350, 5), (397, 373, 5), (1001, 601, 1)])
+def test_four_pixels_a_thread_equal_one(orc, w, h, n):
+    """From 600 000 pixels a launch on a thread takes four pixels of a row: a
+    batch of that many against single calls below, and a single call above;
+    every remainder of 4 on some level, and borders on all sides."""
+    cam = camera(w, h)
+    args = (w, h, cam.cx, cam.cy, cam.fx, cam.fy)
+    T0, T1, f0, f1 = make_pair(cam, 23)
+    filt = RGBDOdometry(*args).bilateral(f1.depth, 5.0)
+    odos = [fed(RGBDOdometry(*args), T0, f0, f1, filt) for _ in range(n + 1)]
+    odos[0].getIncrementalTransformation(T0[:3, 3], T0[:3, :3], False, 10.0, True, False, False)
+    for o in odos[1:]:
+        o.set_pose(T0[:3, 3], T0[:3, :3])
+    Batch(odos[1:]).track(False, 10.0, True, False, False)
+    assert w * h * n >= 600_000 > (w * h if n > 1 else 0)
+    for level in range(3):
+        a, m = odos[0].read_buffer("dxy", level), odos[0].read_buffer("zsrc", level)
+        for o in odos[1:]:
+            assert np.array_equal(a, o.read_buffer("dxy", level)), level
+            assert np.array_equal(m.view(np.uint32), o.read_buffer("zsrc", level).view(np.uint32)), level
+    check_level(odos[0].read_buffer("next_image", 2).astype(np.int32), odos[0].read_buffer("next_depth", 2), a, m, 2)
 
 
 @pytest.mark.parametrize("w,h", [(640, 624), (736, 712), (1280, 960)])
