@@ -2807,11 +2807,8 @@ __device__ void so3_evaluate(So3Slot& S, const double* tot)
 // every texel load is issued before the first row (a branch around each
 // pixel's loads would wait for them one pixel after another), at a valid
 // texel where the pixel is skipped.  SRC: the pixels' halves are in src.
-// Launches of 64 pairs: 25.3 -> 23.5 us.  The one-launch loop does not move
-// (27 us at 640x480, 3 iterations; 155 at 1920x1080, 8 iterations): there the
-// rows' arithmetic on 16 CUs and the serial evaluation are the time, and more
-// workgroups would reorder the fp32 sums, on which the loop's exact tests
-// (equal counts, a smaller error) turn.
+// For k_so3_iter, whose workgroups share CUs: launches of 64 pairs 25.3 -> 23.5
+// us.
 template <int CH, bool SRC, class Ptr>
 __device__ __forceinline__ void so3_chunk(Ptr last, Ptr next, int w, int h, int n, int idx, int stride,
                                           const So3Src* src, const float* H, const float* Ki, const float* KR,
@@ -2852,6 +2849,44 @@ __device__ __forceinline__ void so3_rows(Ptr last, Ptr next, int w, int h, int n
     so3_chunk<kSO3Pre, true>(last, next, w, h, n, first, stride, src, H, Ki, KR, acc);
     for (int i = first + kSO3Pre * stride; i < n; i += 4 * stride)
         so3_chunk<4, false>(last, next, w, h, n, i, stride, src, H, Ki, KR, acc);
+}
+
+// The same pixel by pixel, for the one-launch loop: its few workgroups have a
+// CU each, and the rows' arithmetic and the serial evaluation are its time (3
+// to 8 iterations), so the loads of skipped pixels cost more than the waits
+// they save.  Against four at a time 20.8 and 22.1 us at 211x160, 21.8 and 23.2
+// at 333x251, 148 and 155 at 1920x1080, 75 and 82 for two VGA pairs (640x480
+// level at 26.5).  More workgroups would reorder the fp32 sums, on which the
+// loop's exact tests (equal counts, a smaller error) turn.
+template <class Ptr>
+__device__ __forceinline__ void so3_rows_each(Ptr last, Ptr next, int w, int h, int n, int first, int stride,
+                                              const So3Src (&src)[kSO3Pre], const float* H, const float* Ki,
+                                              const float* KR, float (&acc)[kSO3])
+{
+    int wx[kSO3Pre], wy[kSO3Pre];
+    bool ok[kSO3Pre];
+#pragma unroll
+    for (int j = 0; j < kSO3Pre; ++j) {
+        const int idx = first + j * stride;
+        const int y = idx / w, x = idx - y * w;
+        ok[j] = idx < n && so3_warp(H, w, h, x, y, wx[j], wy[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < kSO3Pre; ++j)
+        if (ok[j]) {
+            const int idx = first + j * stride;
+            const int y = idx / w, x = idx - y * w;
+            float row[4];
+            So3Texels t;
+            so3_texels(next, w, wx[j], wy[j], t);
+            so3_row(so3_half(t), src[j], x, y, Ki, KR, row);
+            acc_row4(acc, row);
+        }
+    for (int idx = first + kSO3Pre * stride; idx < n; idx += stride) {
+        const int y = idx / w, x = idx - y * w;
+        float row[4];
+        if (so3_pixel(last, next, w, h, x, y, H, Ki, KR, row)) acc_row4(acc, row);
+    }
 }
 
 // With `begin`, block 0 of each pair of launch 10 also sets up the
@@ -3051,7 +3086,7 @@ __global__ __launch_bounds__(kSO3Threads) void k_so3_loop(const PairDesc* __rest
         float acc[kSO3];
 #pragma unroll
         for (int k = 0; k < kSO3; ++k) acc[k] = 0.0f;
-        so3_rows(last, next, w, h, n, first, stride, src, Hr, Kir, KRr, acc);
+        so3_rows_each(last, next, w, h, n, first, stride, src, Hr, Kir, KRr, acc);
         const float* part = D.part_a[it & 1];
         block_partial<kSO3, kSO3Threads>(acc, (float*)part + (size_t)lb * kPartStride, s_red);
         // grid barrier of the pair's workgroups
