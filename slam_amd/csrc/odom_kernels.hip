@@ -292,11 +292,20 @@ __device__ __forceinline__ void mean4(const float* a, const float* b, const floa
     for (int k = 0; k < 3; ++k) o[k] = bad ? QNAN : m[k];
 }
 
-// 2x2 mean of the texels at i, i + 1, i + ld, i + ld + 1 of planar LDS values.
+// 2x2 mean of four texels (x, y), (x+1, y), (x, y+1), (x+1, y+1).
+__device__ __forceinline__ Cam6 mean_cam(const Cam6 (&q)[4])
+{
+    Cam6 o;
+    mean4(q[0].v, q[1].v, q[2].v, q[3].v, false, o.v);
+    mean4(q[0].n, q[1].n, q[2].n, q[3].n, true, o.n);
+    return o;
+}
+
+// The mean of the texels at i, i + 1, i + ld, i + ld + 1 of planar LDS values.
 template <int N>
 __device__ __forceinline__ Cam6 mean_lds(const float (&p)[6][N], int i, int ld)
 {
-    Cam6 q[4], o;
+    Cam6 q[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
 #pragma unroll
@@ -304,9 +313,7 @@ __device__ __forceinline__ Cam6 mean_lds(const float (&p)[6][N], int i, int ld)
             q[k].v[m] = p[m][i + (k & 1) + (k >> 1) * ld];
             q[k].n[m] = p[3 + m][i + (k & 1) + (k >> 1) * ld];
         }
-    mean4(q[0].v, q[1].v, q[2].v, q[3].v, false, o.v);
-    mean4(q[0].n, q[1].n, q[2].n, q[3].n, true, o.n);
-    return o;
+    return mean_cam(q);
 }
 
 // Transform (when set) and store output i of level l.
@@ -334,31 +341,42 @@ __device__ __forceinline__ void model_store(const ModelLevels& a, int l, size_t 
     nm[i] = c.n[0]; nm[i + P] = c.n[1]; nm[i + 2 * P] = c.n[2];
 }
 
-// A workgroup computes all levels of a 64x16 tile of level 0, one texel per
-// thread: the untransformed values go through LDS to the 32x8 level-1 and
-// 16x4 level-2 outputs (2x2 means, each level of the one below), so each
-// texel is read once: bound by its bytes at 1920x1080 (140 MB, 27 us; 37 us
-// when level-1 workgroups read the texels again), by latency at 640x480
-// (8.3 us either way).
+// The transform of a launch, if it has one.
+__device__ __forceinline__ void model_pose(const ModelLevels& a, float (&R)[9], float (&t)[3])
+{
+    if (!a.transform) return;
+    if (a.pose_dev) {
+        const GLOBAL_AS float* pd = gp(a.pose_dev);
+        for (int r = 0; r < 3; ++r) {
+            for (int k = 0; k < 3; ++k) R[3 * r + k] = pd[4 * r + k];
+            t[r] = pd[4 * r + 3];
+        }
+    } else {
+        for (int k = 0; k < 9; ++k) R[k] = a.R[k];
+        for (int k = 0; k < 3; ++k) t[k] = a.t[k];
+    }
+}
+
+// Two forms of the same sums.  A workgroup of the tile form computes all
+// levels of a 64x16 tile of level 0, one texel per thread: the untransformed
+// values go through LDS to the 32x8 level-1 and 16x4 level-2 outputs (2x2
+// means, each level of the one below), so each texel is read once.  In the
+// other form level 1 has workgroups of its own, which read the texels again
+// (128 bytes a thread) and form level 2 from LDS, and a thread of the rest
+// moves one texel: more bytes, but one phase fewer in a row.  The tile form is
+// ahead where the bytes count (1920x1080: 140 MB, 27 against 37 us; 1280x801
+// 14.7 and 16.4; 842x478 8.5 and 9.1), the other where the phases do (640x480
+// with a transform 9.3 and 8.1; 333x251 5.5 and 4.7; 160x100 4.3 and 3.4): the
+// line lies between 640x480 and 842x478.
+constexpr int kTileMapsFrom = 350000;   // pixels
 constexpr int kMMX = 64, kMMY = 16;
 
-__global__ __launch_bounds__(kMMX * kMMY) void k_model_maps(ModelLevels a, int tiles_x)
+__global__ __launch_bounds__(kMMX * kMMY) void k_model_maps_tile(ModelLevels a, int tiles_x)
 {
     __shared__ float s0[6][kMMX * kMMY];
     __shared__ float s1[6][kMMX * kMMY / 4];
     float R[9], t[3];
-    if (a.transform) {
-        if (a.pose_dev) {
-            const GLOBAL_AS float* pd = gp(a.pose_dev);
-            for (int r = 0; r < 3; ++r) {
-                for (int k = 0; k < 3; ++k) R[3 * r + k] = pd[4 * r + k];
-                t[r] = pd[4 * r + 3];
-            }
-        } else {
-            for (int k = 0; k < 9; ++k) R[k] = a.R[k];
-            for (int k = 0; k < 3; ++k) t[k] = a.t[k];
-        }
-    }
+    model_pose(a, R, t);
     const int tx = (int)blockIdx.x % tiles_x, ty = (int)blockIdx.x / tiles_x;
     const int tid = threadIdx.x;
     {
@@ -399,10 +417,57 @@ __global__ __launch_bounds__(kMMX * kMMY) void k_model_maps(ModelLevels a, int t
     }
 }
 
+// Blocks [0, nb1): a 16x16 tile of level 1 each and the 8x8 level-2 outputs it
+// covers; then 256 level-0 pixels per block.
+__global__ __launch_bounds__(256) void k_model_maps(ModelLevels a, int nb1, int tiles_x)
+{
+    __shared__ float s1[6][256];
+    float R[9], t[3];
+    model_pose(a, R, t);
+    const int tid = threadIdx.x;
+    float z;
+    if ((int)blockIdx.x >= nb1) {
+        const int i = ((int)blockIdx.x - nb1) * 256 + tid, w = a.w[0];
+        if (i >= w * a.h[0]) return;
+        const int y = i / w, x = i - y * w;
+        const Cam6 c = model_l0(a, x, y, z);
+        if (a.vz) gp(a.vz)[i] = z;
+        model_store(a, 0, (size_t)i, c, R, t);
+        return;
+    }
+    const int ty = (int)blockIdx.x / tiles_x, tx = (int)blockIdx.x - ty * tiles_x;
+    {
+        const int x = 16 * tx + tid % 16, y = 16 * ty + tid / 16;
+        if (x < a.w[1] && y < a.h[1]) {
+            Cam6 q[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[k] = model_l0(a, 2 * x + (k & 1), 2 * y + (k >> 1), z);
+            const Cam6 c = mean_cam(q);
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                s1[m][tid] = c.v[m];
+                s1[3 + m][tid] = c.n[m];
+            }
+            model_store(a, 1, (size_t)y * a.w[1] + x, c, R, t);
+        }
+    }
+    __syncthreads();
+    if (tid < 64) {
+        const int lx = tid % 8, ly = tid / 8, x = 8 * tx + lx, y = 8 * ty + ly;
+        if (x < a.w[2] && y < a.h[2])
+            model_store(a, 2, (size_t)y * a.w[2] + x, mean_lds<256>(s1, 2 * ly * 16 + 2 * lx, 16), R, t);
+    }
+}
+
 void launch_model_maps(const ModelLevels& a, hipStream_t s)
 {
-    const int tiles_x = cdiv(a.w[0], kMMX);
-    hipLaunchKernelGGL(k_model_maps, dim3(tiles_x * cdiv(a.h[0], kMMY)), dim3(kMMX * kMMY), 0, s, a, tiles_x);
+    if (a.w[0] * a.h[0] >= kTileMapsFrom) {
+        const int tiles_x = cdiv(a.w[0], kMMX);
+        hipLaunchKernelGGL(k_model_maps_tile, dim3(tiles_x * cdiv(a.h[0], kMMY)), dim3(kMMX * kMMY), 0, s, a, tiles_x);
+    } else {
+        const int tiles_x = cdiv(a.w[1], 16), nb1 = tiles_x * cdiv(a.h[1], 16);
+        hipLaunchKernelGGL(k_model_maps, dim3(nb1 + cdiv(a.w[0] * a.h[0], 256)), dim3(256), 0, s, a, nb1, tiles_x);
+    }
 }
 
 // ============================================== a9 + a11 Gaussian pyrDown

@@ -65,6 +65,27 @@ def test_pyramids_at_tile_edges(orc, w, h, ch, pad):
             assert np.array_equal(a, b), (mine, l, np.argwhere(a != b)[:4])
 
 
+@pytest.mark.parametrize("w,h", [(704, 496), (705, 497), (1025, 343), (577, 607)])
+def test_model_maps_of_both_forms(orc, w, h):
+    """From 350 000 pixels on a workgroup forms all levels of a 64x16 tile,
+    below it level 1 has workgroups of its own: sizes on both sides of the
+    line, the tiles' remainders, with a transform and without."""
+    _, v4, _ = inputs(w, h, 3)
+    n4 = np.random.default_rng(w).normal(size=v4.shape).astype(np.float32)
+    T = synth.perturb(np.eye(4), np.random.default_rng(h), 0.5, 30.0).astype(np.float32)
+    cam = (w, h, (w - 1) / 2, (h - 1) / 2, 0.8 * w, 0.8 * w)
+    gpu, ref = RGBDOdometry(*cam), orc.Odometry(*cam)
+    for o in (gpu, ref):
+        o.initICPModel(v4, n4, 20.0, T)
+        o.initICPMaps(n4, v4, 20.0)
+    for l in range(3):
+        for name in ("vmap_curr", "nmap_curr", "vmap_g_prev", "nmap_g_prev"):
+            a = gpu.read_buffer(name, l)
+            b = np.asarray(ref.buf(name, l)).reshape(a.shape)
+            assert np.array_equal(np.isnan(a), np.isnan(b)), (name, l)
+            assert np.array_equal(np.nan_to_num(a), np.nan_to_num(b)), (name, l)
+
+
 @pytest.mark.parametrize("w", [16, 65])
 def test_last_texel_of_a_device_image(w):
     """Three-byte colour that ends with its allocation's last byte."""
