@@ -968,10 +968,9 @@ static_assert(kInferIn <= kInferBufB, "the input fits its buffer");
 struct InferParams {
     const bf16* W[kConvs];                   // k_fwd's fragment order
     const float* b[kConvs];
-    int Kp[kConvs];
     const bf16* fc1W;                        // [128][3840]
     const float* fc1b;
-    const bf16* fc2W;                        // [256][8]
+    const bf16* fc2W;                        // [3840][8]
     const float* fc2b;
 };
 
@@ -1158,7 +1157,8 @@ __global__ __launch_bounds__(kInferThreads) void k_cnn_infer(const bf16* __restr
     __syncthreads();
     infer_conv<128, 128, 2, 3, 1, 2, P128, P128, 1>(S, A, B, P.W[5], P.b[5]);
     __syncthreads();
-    // global average pooling over the 1 x 2 output (k_gap_fwd's arithmetic)
+    // global average pooling over the 1 x 2 output (the arithmetic of
+    // k_fwd's kReluGap)
     if (t < kFc1In) {
         const float sgap = bf2f(bufB[t]) + bf2f(bufB[P128 + t]);
         s_gap[t] = bf2f(f2bf(sgap / 2.0f));
@@ -1520,7 +1520,6 @@ int cnn_infer(cnn_net c, const void* x, int N, float* out)
     for (int l = 0; l < kConvs; ++l) {
         P.W[l] = c->forms.fwd[l];
         P.b[l] = c->p + c->convB[l].off;
-        P.Kp[l] = c->Kp[l];
     }
     P.fc1W = c->pb + c->fc1W.off;
     P.fc1b = c->p + c->fc1B.off;

@@ -54,9 +54,9 @@ static inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 // image) into LDS with all of a thread's loads in flight together: the
 // coordinates are clamped into the image, so every address is valid, and the
 // stores follow the last load.  An entry whose texel lies outside the image
-// holds `fill` (FILL_OUT) or its clamped neighbour.
-template <int N, int NT, bool FILL_OUT, class T, class Load>
-__device__ __forceinline__ void stage_tile(T* tile, int ld, int ox, int oy, int w, int h, Load load, T fill = T(0))
+// holds `fill`.
+template <int N, int NT, class T, class Load>
+__device__ __forceinline__ void stage_tile(T* tile, int ld, int ox, int oy, int w, int h, Load load, T fill)
 {
     constexpr int R = (N + NT - 1) / NT;
     T v[R];
@@ -65,7 +65,7 @@ __device__ __forceinline__ void stage_tile(T* tile, int ld, int ox, int oy, int 
         const int i = min((int)threadIdx.x + r * NT, N - 1);
         const int gx = ox + i % ld, gy = oy + i / ld;
         v[r] = load(min(max(gx, 0), w - 1), min(max(gy, 0), h - 1));
-        if (FILL_OUT && (gx < 0 || gx >= w || gy < 0 || gy >= h)) v[r] = fill;
+        if (gx < 0 || gx >= w || gy < 0 || gy >= h) v[r] = fill;
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -124,9 +124,8 @@ __global__ __launch_bounds__(256) void k_bilateral(const uint16_t* __restrict__ 
     const int x0 = blockIdx.x * kBT, y0 = blockIdx.y * kBTY;
     const bool unclipped = maxv < 65535u - kBilatRange ||
                            (x0 >= 6 && y0 >= 6 && x0 + kBT + 6 <= w && y0 + kBTY + 6 <= h);
-    stage_tile<kBLY * kBL, 256, true>(tile, kBL, x0 - 6, y0 - 6, w, h,
-                                      [&](int gx, int gy) { return (float)gp(src)[(size_t)gy * pitch + gx]; },
-                                      65535.0f);
+    stage_tile<kBLY * kBL, 256>(tile, kBL, x0 - 6, y0 - 6, w, h,
+                                [&](int gx, int gy) { return (float)gp(src)[(size_t)gy * pitch + gx]; }, 65535.0f);
     for (int i = tid; i <= kBilatRange; i += 256)
         sEC[i] = (i < kBilatRange) ? bexpf(-((float)(i * i) * 0.000555556f)) : 0.0f;
     __syncthreads();
