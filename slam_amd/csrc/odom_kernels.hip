@@ -19,6 +19,7 @@
 #include <atomic>
 #include <type_traits>
 
+#include "image_reads.h"
 #include "odom_internal.h"
 #include "odom_math.h"
 
@@ -597,8 +598,7 @@ struct PyrGrid {
 
 // Level 0 of the depth pyramid (a8 verticesToDepth): NaN outside (0, cutoff].
 // Level 0 of the intensity pyramid (populateRGBDData, RGBDOdometryef.cpp:212,
-// 225) from the texel's first three bytes, read as one 4-byte word; the
-// image's last texel is read one byte early, so that no byte past it is read.
+// 225) from the texel's first three bytes, read as one 4-byte word.
 typedef uint32_t __attribute__((aligned(1))) word_at_any_byte;
 
 template <bool DEPTH>
@@ -620,9 +620,8 @@ __device__ void pyr_tile(const PyrSrc& P, int w0, int h0, int tx, int ty, unsign
         if constexpr (DEPTH) {
             raw[r] = gp((const uint32_t*)P.vz)[(size_t)y * w0 + x];
         } else {
-            const int early = (x == w0 - 1 && y == h0 - 1 && P.ch == 3) ? 1 : 0;
-            const GLOBAL_AS uint8_t* px = gp(P.rgb) + ((size_t)y * P.pitch + (size_t)x * P.ch - early);
-            raw[r] = *(const GLOBAL_AS word_at_any_byte*)px >> (8 * early);
+            const TexelRead t = texel_read(x, y, w0, h0, P.pitch, P.ch);
+            raw[r] = *(const GLOBAL_AS word_at_any_byte*)(gp(P.rgb) + t.offset) >> (8 * t.early);
         }
     }
 #pragma unroll
@@ -806,18 +805,6 @@ void launch_depth_pyramid_maps(const VNLevels& a, hipStream_t s)
 // nine of its derivatives, and G pixels' windows lie in 4 (G = 1) or 8 (G = 4)
 // bytes of each of four rows: one load a row instead of 25 a pixel, and a
 // pixel next to the border takes its taps from the same bytes.
-// The bytes of T from column x of row y of an image of n bytes (row length w):
-// any x; bytes outside the image are 0.
-template <class T>
-__device__ __forceinline__ T row_bytes(const uint8_t* __restrict__ img, int n, int w, int y, int x)
-{
-    constexpr int B = sizeof(T);
-    const int want = y * w + x, at = min(max(want, 0), n - B);
-    T v;
-    __builtin_memcpy(&v, img + at, B);
-    return want < at ? v << (8 * (at - want)) : v >> (8 * min(want - at, B - 1));
-}
-
 // Group k of one level.
 template <int G>
 __device__ __forceinline__ void rgb_prep_group(const uint8_t* __restrict__ img, const float* __restrict__ depth,
