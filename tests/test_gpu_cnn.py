@@ -312,3 +312,47 @@ def test_replayed_training_steps_move_the_weights_of_later_calls(setup):
         out, inf = net.forward(x), net.infer(x)
         torch.cuda.synchronize()
         assert np.array_equal(out.cpu().numpy(), ref[0]) and np.array_equal(inf.cpu().numpy(), ref[1])
+
+
+def test_backward_uses_the_weights_of_its_own_time(setup):
+    """Weights doubled between forward and backward: the gradients are those of
+    the forward's activations through the new weights, so each layer of weights
+    between the output and a gradient doubles it, exactly."""
+    import torch
+    from slam_amd.warmstart import WarmStartNet, he_init
+    co, x, target = setup["co"], setup["xt"], torch.from_numpy(setup["target"]).cuda()
+    net = WarmStartNet(max_batch=4)
+    flat = he_init(net.layout, net.nparam, 31)
+    got = []
+    for scale in (1.0, 2.0):
+        net.set_params(flat)
+        net.forward(x)
+        net.set_params(flat * np.float32(scale))
+        net.backward(4, target)
+        got.append(co.unpack(net.get_grads()))
+    passed = {"fc2": 0, "fc1": 1, **{f"conv{i}": 7 - i for i in range(6)}}
+    for name in got[0]:
+        assert np.any(got[0][name])
+        assert np.array_equal(got[1][name], got[0][name] * 2.0 ** passed[name.split(".")[0]]), name
+
+
+def test_gradients_of_a_batch_beyond_a_thousand(setup):
+    """1 200 samples in one pass against four passes of 300: the mean of their
+    gradients but for bf16 roundings (a quarter of a batch scales every output
+    gradient by 4, which rounds the same; the sums of FC2 and of the parts
+    have other orders)."""
+    from slam_amd.warmstart import WarmStartNet
+    co = setup["co"]
+    rng = np.random.default_rng(41)
+    x = bf16_round(rng.uniform(0, 1, size=(1200, 60, 80, 4)))
+    target = rng.normal(size=(1200, 6)).astype(np.float32)
+    net = WarmStartNet(max_batch=1200)
+    net.init_params(seed=5)
+    out, loss, flat = gradients(net, x, target)
+    parts = [gradients(net, x[i:i + 300], target[i:i + 300]) for i in range(0, 1200, 300)]
+    net.close()
+    assert rel(out, np.concatenate([p[0] for p in parts])) < 1e-2
+    assert rel(loss, np.concatenate([p[1] for p in parts])) < 1e-2
+    G, ref = co.unpack(flat), co.unpack(np.mean([p[2] for p in parts], axis=0))
+    for name in ref:
+        assert rel(G[name], ref[name]) < 1e-2 and cos(G[name], ref[name]) > 0.9999, (name, rel(G[name], ref[name]))
