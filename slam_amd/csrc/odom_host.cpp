@@ -369,6 +369,7 @@ StepLaunch step_launch(odom_ctx* c, int kernel, int level)
     L.blk_pair = nullptr;
     L.shape = kernel == 0 ? c->shape_a[level] : c->shape_b[level];
     L.total_blocks = kernel == 0 ? c->h_pair[0].nblk_a[level] : c->h_pair[0].nblk_b[level];
+    L.pixels = c->n[level];
     return L;
 }
 
@@ -1317,7 +1318,7 @@ struct CallSpec {
     float t_scale = 1.0f, r_scale = 1.0f;
 };
 
-// A batch's pass A reads z planes alone if every pair's maps are a depth
+// A batch's pass A may read z planes alone if every pair's maps are a depth
 // image's (TrackParams::zcur).
 int batch_from_depth(const odom_batch_s* b)
 {
@@ -1456,6 +1457,8 @@ StepLaunch plan_launch(odom_batch_s* b, int hyp, PairDesc* dp, int kernel, int l
     L.npairs = (int)b->h.size() * hyp;
     L.blk_pair = pl.d_blk[kernel][level];
     L.total_blocks = pl.total[kernel][level];
+    L.pixels = 0;
+    for (const auto* c : b->h) L.pixels += (long long)c->n[level] * hyp;
     L.shape = b->shape[kernel][level];
     return L;
 }

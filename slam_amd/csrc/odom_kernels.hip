@@ -2228,10 +2228,16 @@ int step_shape_supported(StepShape sh)
 void launch_step_a(const StepLaunch& L, int level, int iter, int k, int prev_level, const TrackParams& P, int mode,
                    uint8_t* dbg_mask, hipStream_t s)
 {
-    // the fused pass of a single pair waits for latency, not for bytes: with z
-    // planes alone 29.6 against 30.2 us at 1920x1080, nothing below
+    // The fused pass of a single pair waits for latency, not for bytes: with z
+    // planes alone 29.6 against 30.2 us at 1920x1080, nothing below.
+    // The unfused pass of a batch gains where its bytes are the time.  With
+    // the photometric loads from 300 000 pixels a launch (us without, with: 0.08M
+    // 14.1, 14.3; 0.31M 17.4, 17.2; 0.61M 24.2, 22.9; 4.9M 63.6, 60.6; 19.7M
+    // 213, 196), without them, where forming x and y shows more, from 8 million
+    // (1.2M 27.4, 28.0; 4.9M 51.6, 52.0; 9.8M 97.8, 94.5; 19.7M 178, 171).
+    const bool z = P.zcur && L.pixels >= (P.rgb ? 300000 : 8000000);
     if (mode == 0) STEP_DISPATCH_A(true, false, L.pairs, L.blk_pair, level, iter, k, prev_level, P, dbg_mask);
-    else if (P.zcur) STEP_DISPATCH_A(false, true, L.pairs, L.blk_pair, level, iter, k, prev_level, P, dbg_mask);
+    else if (z) STEP_DISPATCH_A(false, true, L.pairs, L.blk_pair, level, iter, k, prev_level, P, dbg_mask);
     else STEP_DISPATCH_A(false, false, L.pairs, L.blk_pair, level, iter, k, prev_level, P, dbg_mask);
 }
 
