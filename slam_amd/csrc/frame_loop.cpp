@@ -273,7 +273,7 @@ int efloop_create(int width, int height, float cx, float cy, float fx, float fy,
     const size_t npix = (size_t)width * height;
     if (!rc && (hipMalloc((void**)&c->filtered, npix * 2) != hipSuccess ||
                 hipMalloc((void**)&c->dev_rgb, npix * 3) != hipSuccess ||
-                hipMalloc((void**)&c->dev_depth, npix * 2) != hipSuccess || c->uploads.create() != hipSuccess))
+                hipMalloc((void**)&c->dev_depth, npix * 2) != hipSuccess || c->uploads.create(npix * 3) != hipSuccess))
         rc = ODOM_ERR_HIP;
     for (hipEvent_t* e : {&c->order, &c->fused})
         if (!rc && hipEventCreateWithFlags(e, hipEventDisableTiming) != hipSuccess) rc = ODOM_ERR_HIP;

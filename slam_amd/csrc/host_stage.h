@@ -5,9 +5,9 @@
 // five such copies per frame (23 ms of a 23 ms frame).  Here the host copies
 // the rows into one of two pinned slots and enqueues the slot's copy, so the
 // caller's memory is free on return and one slot fills while the other is in
-// flight.  The host waits only for a slot: an image of up to two slots does not
+// flight.  The host waits only for a slot: an image of up to 2 MiB does not
 // wait for the device unless the images before it are still on their way, but
-// the third slot of a larger one waits until the first has been copied, and so
+// the third MiB of a larger one waits until the first has been copied, and so
 // for the work queued ahead of it.
 #pragma once
 
@@ -34,16 +34,17 @@ public:
         if (pin_) (void)hipHostFree(pin_);
     }
 
-    // The slots (2 MiB of pinned memory, about 50 us), with the owner's other
-    // memory, so that no upload allocates.
-    hipError_t create()
+    // The slots, with the owner's other memory, so that no upload allocates
+    // (about 50 us): two of its largest image, at most 1 MiB each.
+    hipError_t create(size_t largest)
     {
-        if (hipError_t e = hipHostMalloc((void**)&pin_, 2 * kSlot, hipHostMallocDefault)) {
+        slot_ = std::min(kSlot, (largest + 4095) / 4096 * 4096);
+        if (hipError_t e = hipHostMalloc((void**)&pin_, 2 * slot_, hipHostMallocDefault)) {
             pin_ = nullptr;
             return e;
         }
         for (int k = 0; k < 2; ++k) {
-            slots_[k].pin = pin_ + k * kSlot;
+            slots_[k].pin = pin_ + k * slot_;
             if (hipError_t e = hipEventCreateWithFlags(&slots_[k].ev, hipEventDisableTiming)) {
                 slots_[k].ev = nullptr;
                 return e;
@@ -65,7 +66,7 @@ public:
             Slot& q = slots_[next_];
             next_ ^= 1;
             if (hipError_t e = ready(q)) return e;
-            const size_t n = std::min(kSlot, total - at);
+            const size_t n = std::min(slot_, total - at);
             for (size_t done = 0; done < n;) {
                 const size_t y = (at + done) / row, x = (at + done) % row;
                 const size_t m = pitch == row ? n - done : std::min(n - done, row - x);
@@ -100,6 +101,7 @@ private:
     }
 
     uint8_t* pin_ = nullptr;
+    size_t slot_ = 0;
     Slot slots_[2];
     int next_ = 0;
 };

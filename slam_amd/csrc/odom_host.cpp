@@ -582,7 +582,7 @@ int odom_create(const odom_params* p, odom_handle* out)
     for (auto& r : reqs) total += align_up(r.bytes, 256);
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc((void**)&c->arena, total) != hipSuccess ||
-        hipHostMalloc((void**)&c->h_pin, sizeof(TrackState), 0) != hipSuccess || c->uploads.create() != hipSuccess) {
+        hipHostMalloc((void**)&c->h_pin, sizeof(TrackState), 0) != hipSuccess || c->uploads.create(N0 * 16) != hipSuccess) {
         odom_destroy(c);
         return ODOM_ERR_HIP;
     }

@@ -118,7 +118,7 @@ struct StepLaunch {
     int npairs;
     const int* blk_pair;            // device table, per level (null when npairs == 1)
     int total_blocks;               // blocks of this level over all pairs
-    long long pixels;               // of this level over all pairs
+    long long pixels = 0;           // of this level over all pairs
     StepShape shape;
 };
 // SO3 pre-alignment; max_px_l2: largest level-2 pixel count over the pairs

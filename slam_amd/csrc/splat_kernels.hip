@@ -607,7 +607,7 @@ int splat_create(int width, int height, float cx, float cy, float fx, float fy, 
     c->cam.h = height;
     const size_t npix = (size_t)width * height;
     bool ok = hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking) == hipSuccess;
-    ok = ok && c->uploads.create() == hipSuccess;
+    ok = ok && c->uploads.create(npix * 4) == hipSuccess;
     c->stream = c->own;
     ok = ok && hipMalloc((void**)&c->keys, npix * 8) == hipSuccess;
     ok = ok && hipMalloc((void**)&c->rays, npix * 16) == hipSuccess;

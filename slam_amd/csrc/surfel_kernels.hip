@@ -1162,7 +1162,7 @@ int surfel_create(int width, int height, float cx, float cy, float fx, float fy,
     c->max_surfels = max_surfels;
     const size_t ms = (size_t)max_surfels, np = (size_t)npix, ni = ms + np;
     bool ok = hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking) == hipSuccess;
-    ok = ok && c->uploads.create() == hipSuccess;
+    ok = ok && c->uploads.create(np * 3) == hipSuccess;
     c->stream = c->own;
     auto A = [&](void** p, size_t bytes) { ok = ok && hipMalloc(p, bytes) == hipSuccess; };
     A((void**)&c->model[0], ms * 48);
