@@ -214,3 +214,25 @@ def test_batch_of_64_pairs_against_the_fp64_oracle(orc):
         dt, dr = synth.pose_error(got[j], alone)
         assert dt <= 2e-5 and dr <= 2e-3, (j, dt, dr)
     b.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5])
+def test_the_solve_in_the_prologue_or_on_its_own(pairs, n):
+    """With the single call's shapes and blocks the solve runs in the prologue
+    up to two rounds of workgroups and in a launch of its own past them (from 3
+    pairs of 640x480 on the finest level is past them, from 5 the next one):
+    the bits of the call alone either way, and of the split form."""
+    chosen = [pairs[1 + 3 * (i % 2)] for i in range(n)]
+    alone = [track_alone(p, "joint")[0] for p in chosen]
+    for split in (False, True):
+        odos = batch_handles(chosen)
+        b = Batch(odos)
+        b.set_blocks(0)
+        for kernel in range(2):
+            for level in range(3):
+                b.set_step_shape(kernel, level, *odos[0].get_step_shape(kernel, level))
+        b.set_split_solve(split)
+        b.track(**MODES["joint"])
+        for got, exp in zip(poses_of(odos), alone):
+            assert np.array_equal(got, exp), split
+        b.close()
