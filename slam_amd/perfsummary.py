@@ -16,7 +16,8 @@
         device copies of ``bench.py --calibrate-copy``.
     python -m slam_amd.perfsummary batch-traffic FETCH_DIR WRITE_DIR [--out JSON]
         the same for the 64-pair batch's passes A (unfused) and B per level,
-        with the joint (A + B) traffic against the 62 B/px contract
+        with the joint (A + B) traffic against the bytes per pixel that the
+        passes need: A 58, or 50 where it reads z planes alone, and B 4
     python -m slam_amd.perfsummary kernel-traffic FETCH_DIR WRITE_DIR --kernel NAME --algorithmic BYTES
         the same for every dispatch of the kernels whose name contains NAME:
         mean FETCH_SIZE and WRITE_SIZE, copy-scaled bytes, and their ratio to
@@ -174,6 +175,12 @@ def _level(name: str, grid: int, wg: int) -> int | None:
     return None
 
 
+def _pass_a(name: str) -> tuple[bool, bool] | None:
+    """(fused, z planes alone) of a pass A kernel's name, else None."""
+    m = re.search(r"k_step_a<\d+, \d+, (true|false)(?:, (true|false))?>", name)
+    return (m.group(1) == "true", m.group(2) == "true") if m else None
+
+
 def _calibration_copies(rows) -> list:
     """Counter values of the four 256 MiB calibration copies of
     ``bench.py --calibrate-copy``: the first four device copies of the run in
@@ -190,7 +197,8 @@ def _per_level(path: str):
     copy = _calibration_copies(rows)
     lv = defaultdict(list)
     for r in rows:
-        if "k_step_a" not in r["Kernel_Name"] or "true>" not in r["Kernel_Name"]:
+        form = _pass_a(r["Kernel_Name"])
+        if form is None or not form[0]:
             continue  # the fused pass of tracking calls only
         level = _level(r["Kernel_Name"], int(r["Grid_Size"]), int(r["Workgroup_Size"]))
         if level is not None:
@@ -251,40 +259,46 @@ CALL_LEVELS = [2] * 4 + [1] * 5 + [0] * 10
 
 def _batch_levels(path: str, kernel: str):
     """Counter values of the batched calls' dispatches of `kernel` (the
-    unfused pass A or pass B), by level: every batched call launches each
-    pass 19 times in the schedule's order (4 at level 2, 5 at 1, 10 at 0)."""
+    unfused pass A or pass B), by level, their number, and the bytes per pixel
+    that the pass needs there: every batched call launches each pass 19 times
+    in the schedule's order (4 at level 2, 5 at 1, 10 at 0)."""
     rows = list(csv.DictReader(open(path)))
     copy = _calibration_copies(rows)
     if "Dispatch_Id" in rows[0]:
         rows.sort(key=lambda r: int(r["Dispatch_Id"]))
     if kernel == "a":
-        sel = [r for r in rows if "k_step_a" in r["Kernel_Name"] and "false>" in r["Kernel_Name"]]
+        sel = [r for r in rows if (_pass_a(r["Kernel_Name"]) or (True,))[0] is False]
     else:
         sel = [r for r in rows if "k_step_b" in r["Kernel_Name"]]
     if not copy or not sel or len(sel) % len(CALL_LEVELS):
         raise ValueError(f"{path}: {len(copy)} calibration copies, {len(sel)} dispatches of pass {kernel}")
-    lv = defaultdict(list)
+    lv, bpp = defaultdict(list), {}
     for i, r in enumerate(sel):
-        lv[CALL_LEVELS[i % len(CALL_LEVELS)]].append(float(r["Counter_Value"]))
-    return sum(copy) / len(copy), {k: sum(v) / len(v) for k, v in lv.items()}, {k: len(v) for k, v in lv.items()}
+        level = CALL_LEVELS[i % len(CALL_LEVELS)]
+        lv[level].append(float(r["Counter_Value"]))
+        need = 4 if kernel == "b" else (50 if _pass_a(r["Kernel_Name"])[1] else 58)
+        if bpp.setdefault(level, need) != need:
+            raise ValueError(f"{path}: pass {kernel} has two forms at level {level}")
+    return sum(copy) / len(copy), {k: sum(v) / len(v) for k, v in lv.items()}, {k: len(v) for k, v in lv.items()}, bpp
 
 
 def cmd_batch_traffic(fetch_dir: str, write_dir: str) -> dict:
     """HBM bytes per dispatch of the batched passes A and B per level, copy-scaled,
     against the algorithmic bytes (A 58 B/px: the ICP maps and the photometric
-    association reads; B 4 B/px: the gradients; joint 62 B/px)."""
+    association reads, or 50 with the current vertices' z planes alone; B 4
+    B/px: the gradients; joint their sum)."""
     out = {"workload": "64 pairs (16 x 320x240, 32 x 640x480, 16 x 848x480), batched ICP+RGB+SO3 calls",
            "counter_unit": "KiB per dispatch", "levels": {}}
-    per = {}
-    for k, bpp in (("a", 58), ("b", 4)):
-        fc, fl, fn = _batch_levels(os.path.join(fetch_dir, "run_counter_collection.csv"), k)
-        wc, wl, wn = _batch_levels(os.path.join(write_dir, "run_counter_collection.csv"), k)
+    per, need = {}, {}
+    for k in ("a", "b"):
+        fc, fl, fn, bpp = _batch_levels(os.path.join(fetch_dir, "run_counter_collection.csv"), k)
+        wc, wl, wn, _ = _batch_levels(os.path.join(write_dir, "run_counter_collection.csv"), k)
         fs, ws = COPY_BYTES / (1024.0 * fc), COPY_BYTES / (1024.0 * wc)
         out[f"calibration_{k}"] = {"fetch_kib": round(fc, 1), "write_kib": round(wc, 1),
                                    "fetch_scale": round(fs, 4), "write_scale": round(ws, 4)}
         for l in sorted(fl):
             fb, wb = fl[l] * 1024.0 * fs, wl[l] * 1024.0 * ws
-            alg = bpp * BATCH_LEVEL_PX[l]
+            alg = need[(k, l)] = bpp[l] * BATCH_LEVEL_PX[l]
             per[(k, l)] = fb + wb
             out["levels"].setdefault(str(l), {})[k] = {
                 "dispatches": fn[l], "fetch_kib": round(fl[l], 1), "write_kib": round(wl[l], 1),
@@ -292,14 +306,14 @@ def cmd_batch_traffic(fetch_dir: str, write_dir: str) -> dict:
                 "algorithmic_bytes": alg, "ratio": round((fb + wb) / alg, 3)}
     for l in range(3):
         if ("a", l) in per and ("b", l) in per:
-            alg = 62 * BATCH_LEVEL_PX[l]
+            alg = need[("a", l)] + need[("b", l)]
             out["levels"][str(l)]["joint"] = {"traffic_bytes": int(per[("a", l)] + per[("b", l)]),
                                               "algorithmic_bytes": alg,
                                               "ratio": round((per[("a", l)] + per[("b", l)]) / alg, 3)}
     iters = (10, 5, 4)
     out["a_traffic_bytes_per_launch_10_5_4"] = int(sum(iters[l] * per[("a", l)] for l in range(3)) / sum(iters))
     out["joint_ratio_10_5_4"] = round(sum(iters[l] * (per[("a", l)] + per[("b", l)]) for l in range(3)) /
-                                      sum(iters[l] * 62 * BATCH_LEVEL_PX[l] for l in range(3)), 3)
+                                      sum(iters[l] * (need[("a", l)] + need[("b", l)]) for l in range(3)), 3)
     return out
 
 

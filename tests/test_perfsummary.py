@@ -108,6 +108,29 @@ def test_batch_traffic_assigns_levels_in_schedule_order(tmp_path):
     assert r["a_traffic_bytes_per_launch_10_5_4"] == int((10 * per_a[0] + 5 * per_a[1] + 4 * per_a[2]) / 19)
 
 
+def test_pass_a_forms_are_told_apart(tmp_path):
+    """Pass A's names carry whether the solve is in its prologue and whether it
+    reads z planes alone: a batch's launches are the unfused ones of either
+    kind, whose bytes per pixel differ, and single calls' fused launches are
+    left out; the single-call summary takes just those."""
+    fused, z, whole, b = ("k_step_a<512, 3, true, false>(x)", "k_step_a<512, 2, false, true>(x)",
+                          "k_step_a<256, 1, false, false>(x)", "k_step_b<512, 3>(x)")
+    rows = [(fused, 200 * 256, 7.0)]
+    for lv in ps.CALL_LEVELS:
+        rows += [(whole if lv == 2 else z, 4096, 10.0), (b, 4096, 1.0), (fused, 200 * 256, 7.0)]
+    fetch = tmp_path / "f"
+    counters(fetch, "FETCH_SIZE", [(COPY, 131072, 262144.0)] * 4 + rows)
+    r = ps.cmd_batch_traffic(str(fetch), str(fetch))
+    for lv in range(3):
+        level = r["levels"][str(lv)]
+        assert level["a"]["dispatches"] == (10, 5, 4)[lv]
+        assert level["a"]["algorithmic_bytes"] == (50, 50, 58)[lv] * ps.BATCH_LEVEL_PX[lv]
+        assert level["joint"]["algorithmic_bytes"] == (54, 54, 62)[lv] * ps.BATCH_LEVEL_PX[lv]
+    path = fetch / "run_counter_collection.csv"
+    _, mean, count = ps._per_level(str(path))
+    assert mean == {0: 7.0} and count == {0: 20}
+
+
 def test_batch_traffic_rejects_a_partial_call(tmp_path):
     fetch = tmp_path / "f"
     counters(fetch, "FETCH_SIZE", [(COPY, 131072, 1.0)] * 4 + [("k_step_a<512, 2, false>", 4096, 1.0)] * 18)
