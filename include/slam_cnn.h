@@ -11,7 +11,10 @@
  *
  * All tensor pointers are device pointers.  Work is enqueued on the stream
  * set with cnn_set_stream (default: the null stream).  A net is not
- * re-entrant.
+ * re-entrant.  cnn_forward, cnn_infer, cnn_backward and cnn_adam_step only
+ * enqueue kernels, so they may be captured into a hipGraph: a replay works
+ * with the weights that it finds (the loss weights, the learning rate and
+ * Adam's step number are those of the capture).
  */
 #ifndef SLAM_CNN_H
 #define SLAM_CNN_H
